@@ -55,7 +55,7 @@ struct KArgs {
     long long m;
     long long e_lo, e_hi;        // root edges of this count: [e_lo, e_hi)
     const GatPlanDev *plan;
-    unsigned long long *counts;  // [n_patterns]
+    unsigned long long *counts;  // kCountCopies copies of [GATP_MAX_TERMS]
     unsigned long long *queue;   // [0] main queue head, [1] overflow head
     long long *ovf;              // overflow task starts
     unsigned long long *ovf_n;   // overflow task count
@@ -263,6 +263,15 @@ __device__ __forceinline__ bool has(P a, int len, int x, int lin_thr) {
         n -= half;
     }
     return a[base] == x;
+}
+
+// Counters are kept in kCountCopies copies of GATP_MAX_TERMS, one per group of
+// workgroups, which the host adds up: atomics on one address are performed one
+// after the other, 17 ns each, and every wave of a launch ends with one per
+// pattern (4,096 waves and 21 patterns: 1.5 ms on one copy).
+constexpr int kCountCopies = 32;
+__device__ __forceinline__ unsigned long long *count_copy(unsigned long long *counts) {
+    return counts + (blockIdx.x % kCountCopies) * GATP_MAX_TERMS;
 }
 
 struct Ctx {
@@ -1211,7 +1220,7 @@ __global__ void __launch_bounds__(256) engine_kernel(const KArgs *__restrict__ a
         wsync();
     }
     for (int i = ln; i < np; i += W)
-        if (S->wave_acc[i]) atomicAdd(&a.counts[i], S->wave_acc[i]);
+        if (S->wave_acc[i]) atomicAdd(&count_copy(a.counts)[i], S->wave_acc[i]);
     if (a.account && ln == 0 && S->bytes) atomicAdd(a.bytes, S->bytes);
     if (a.tl && ln == 0)
         tl_write(a.tl, a.tl_base + blockIdx.x * wpb + wid, GS ? kLevelsHbm : 0, blockIdx.x * wpb + wid, tl_t0,
@@ -1290,7 +1299,7 @@ __global__ void __launch_bounds__(256) engine_sub_kernel(const KArgs *__restrict
         wsync();
     }
     for (int i = ln; i < np; i += W)
-        if (S->wave_acc[i]) atomicAdd(&a.counts[i], S->wave_acc[i]);
+        if (S->wave_acc[i]) atomicAdd(&count_copy(a.counts)[i], S->wave_acc[i]);
     if (a.account && ln == 0 && S->bytes) atomicAdd(a.bytes, S->bytes);
     if (a.tl && ln == 0)
         tl_write(a.tl, a.tl_base + blockIdx.x * wpb + wid, a.sub_mode + (GS ? 1 : 0), blockIdx.x * wpb + wid, tl_t0,
@@ -1301,51 +1310,80 @@ __global__ void __launch_bounds__(256) engine_sub_kernel(const KArgs *__restrict
 // Bitmap vertex store for clique plans (the reference declares
 // VertexStoreType::Bitmap in include/configs/vertex_set_config.hpp:3-6 but
 // never implements it). On the degree-oriented graph every k-clique is a
-// chain v0 > v1 > ... with v_{i+1} in N+(v_i). Per vertex v0 the wave stages
-// L = N+(v0) (sorted, d entries) and builds the oriented adjacency of the
-// subgraph induced on L as bit rows over positions in L:
+// chain v0 > v1 > ... with v_{i+1} in N+(v_i). Per vertex v0 with list
+// L = N+(v0) (sorted, d entries) the oriented adjacency of the subgraph
+// induced on L is built as bit rows over positions in L:
 //   M_p = { q < p : L[q] in N+(L[p]) }.
 // Every clique with top vertex v0 is then a clique of these rows:
 //   #K3 += sum_p popc(M_p)
 //   #K4 += sum_p sum_{q in M_p} popc(M_p & M_q)
 //   #K5 += sum over q in M_p, r in M_p & M_q of popc(M_p & M_q & M_r)
 //   #K6 one level deeper.
-// Each neighbour pair inside N+(v0) is tested once per v0 (one flattened
-// sweep over the lists N+(L[p]), binary search in L or the reverse for
-// skewed pairs), so the deeper levels are pure bit operations. Tiers by d:
-// the main launch gives each vertex with d <= 256 one wave and 8-word rows in
-// LDS; larger vertices are shared by the 8 waves of a workgroup, with
-// 16-word rows in LDS (d <= 512) or rows in the workgroup's HBM scratch.
-constexpr int CMAXW = 8;   // main tier: d <= 256
-constexpr int CMIDW = 16;  // workgroup tier 0: d <= 512, rows in LDS
-constexpr int CBIGW = 32;  // workgroup tier 1: d <= 1024, rows in LDS when it fits, else HBM
-// Workgroup-tier items are (vertex, part) pairs, vertex * CSPLIT_ENC + part:
-// the parts of a vertex share out its pairs (each builds the rows).
-constexpr int CSPLIT_ENC = 16;
-constexpr int CSPLIT12 = 2;   // parts per vertex in tiers 1 and 2
-constexpr int CSPLIT0 = 1;    // parts per tier-0 vertex with d > CSPLIT0_D
-constexpr int CSPLIT0_D = 256;
-__device__ __forceinline__ int clique_parts(int tier, int d) {
-    return tier ? CSPLIT12 : (d > CSPLIT0_D ? CSPLIT0 : 1);
+//
+// Rows. One ballot of the wave gives 64 bits of a row: lane q tests whether
+// L[q] lies in N+(L[p]) with one word of the core bitmap (dense rows of the
+// first core_n vertices, see core_row), or by a search of the list when L[p]
+// is not a core vertex. That is d^2/128 wave steps for a vertex, with no
+// shared writes; the sweep of the lists N+(L[p]) it replaces took
+// sum_p |N+(L[p])| / 64 steps with a hash probe and an LDS atomic each (on
+// R-MAT s20: 2 to 13 times more steps for d >= 16).
+//
+// Tiers by d: the main launch gives a vertex with d <= CMAIN (64) one wave,
+// whose rows are single 64-bit words; larger vertices are shared by the
+// waves of a workgroup with rows in LDS (d <= 256, 512, 1024) or in HBM.
+constexpr int CMAXD = 256;  // largest slot_capacity the clique store honours
+constexpr int CMAIN = 64;   // main launch: d <= min(CMAIN, slot_capacity)
+constexpr int CT0W = 8;     // workgroup tier 0: rows of 8 words, d <= 256
+constexpr int CT1W = 16;    // workgroup tier 1: d <= 512
+constexpr int CT2W = 32;    // workgroup tier 2: d <= 1024
+constexpr int CTIERS = 4;   // tier 3: any d, rows in HBM
+// Items of a tier's queue: clique_parts() per vertex, which share out its
+// counting (each builds the rows). One part when the vertices fill the
+// launch's workgroups four times over, else more, up to what the depth of the
+// counting pays for: with whole vertices the last ones of R-MAT s20's tier 2
+// (665 vertices, 256 workgroups) end unevenly, and a single vertex of 259
+// neighbours took 3.7 ms for #K6 on one workgroup.
+__host__ __device__ constexpr int clique_max_parts(int kmax) {
+    return kmax >= 6 ? 16 : kmax == 5 ? 8 : kmax == 4 ? 4 : 1;
 }
-constexpr int CBLOCKW0 = 8;   // waves per workgroup, tier 0
-constexpr int CBLOCKW1 = 16;  // waves per workgroup, tiers 1 and 2 (few, heavy vertices)
+__device__ __forceinline__ int clique_parts(int kmax, unsigned long long vertices, int groups) {
+    const unsigned long long want = 4ull * groups, mx = clique_max_parts(kmax);
+    const unsigned long long p = vertices ? (want + vertices - 1) / vertices : 1;
+    return (int)(p < mx ? p : mx);
+}
+// Waves per workgroup: enough to share one vertex's work, few enough that
+// the workgroups of a CU (bounded by LDS, 11, 39 and 160 KB each, and by registers) overlap
+// one's row build with another's counting.
+constexpr int CNW0 = 4, CNW1 = 4, CNW2 = 12, CNW3 = 16;
+// Waves per SIMD the tiers' registers leave room for.
+constexpr int clique_occupancy(int tier) { return tier == 0 ? 4 : 3; }
 // Words per bit row of a list of d vertices: enough for d bits, rounded up
 // to an odd number so that lanes reading the same word of different rows
 // hit different LDS banks (an even stride folds them onto a few banks).
 __host__ __device__ constexpr int row_words(int d) { return ((d + 31) >> 5) | 1; }
-// LDS index of a workgroup tier's list L (lists of up to lcap vertices):
-// open addressing with linear probing over 2 lcap 16-bit slots (a power of
-// two), each 0 or 1 + the position in L of the vertex stored there.
-__host__ __device__ constexpr int index_slots(int lcap) { return 2 * lcap; }
-__device__ __forceinline__ unsigned index_hash(int y, unsigned mask) {
-    return ((unsigned)y * 0x9E3779B1u >> 16) & mask;
+// LDS of a workgroup tier with rows of up to mw words: the rows of lcap = 32
+// mw vertices, slack for the chunks of four words the matrix operands are
+// read in, and the waves' column lists (the list L shares their space: it is
+// not needed once the rows are built).
+__host__ __device__ constexpr int tier_row_words(int mw) { return 32 * mw * row_words(32 * mw) + 8; }
+constexpr size_t tier_lds(int mw, int nw) {
+    return (size_t)4 * tier_row_words(mw) + (size_t)4 * (32 * mw > 128 * nw ? 32 * mw : 128 * nw);
+}
+
+// Core bitmap: for x < core_n, row x holds bit y set iff y in N+(x), y < x,
+// in ceil(x / 32) words; the rows follow one another from x = 1 on.
+__host__ __device__ __forceinline__ unsigned core_row(int x) {
+    if (x < 1) return 0;
+    const unsigned k = (unsigned)(x - 1) >> 5;
+    return (k + 1) * ((unsigned)(x - 1) - 16 * k);
 }
 
 struct CArgs {
     const long long *off;
     const int *adj;
     const int *split;
+    const unsigned *core;        // core bitmap
+    int core_n;                  // its vertices: [0, core_n)
     int n;
     long long m;
     int root_lo, root_hi;        // top vertices of this count: [root_lo, root_hi)
@@ -1353,79 +1391,307 @@ struct CArgs {
     int pat_of_k[8];
     int kmax;
     unsigned long long *queue;   // [0] main vertex queue, [1 + t] workgroup tier t
-    long long *tier[3];          // vertices of the workgroup tiers (counts ovf_n[t])
+    int *tier[CTIERS];           // vertices of the workgroup tiers
+    long long tier_cap[CTIERS];
+    // [t] vertices of tier t, [4] vertices with d > cap, [5] of those the
+    // ones with d <= 512
     unsigned long long *ovf_n;
-    long long ovf_cap;
     unsigned long long *bytes;   // W_alg accumulator of this launch
     unsigned int *err;
-    unsigned *grows;             // HBM tier: per-workgroup rows, hcap * ceil(hcap/32) words
+    unsigned *grows;             // HBM tier: per-workgroup rows, hcap * row_words(hcap) words
     int *goff;                   // HBM tier: per-workgroup pair offsets, hcap + 1 entries
     int hcap;                    // HBM tier capacity (>= maximum out-degree)
+    int lds_dmax;                // largest d of the LDS tiers
     int account;
-    int cap;                     // main-tier limit on d (<= 32 * CMAXW)
+    int cap;                     // slot_capacity as the clique store takes it
+    int main_max;                // largest d of the main launch: min(CMAIN, cap)
     int chunk;                   // vertices per main-queue grab
     int lin_thr;
-    int gallop_ratio;
     long long *tl;               // timeline records (GAT_FLAG_TIMELINE), or null
     int tl_base;                 // first record of this launch
 };
 
-// Rows M_p of the list L (d entries) into rows (w words per row, already
-// zeroed), for the rows p = first, first + stride, first + 2 stride, ...
-// (a workgroup's waves interleave their rows, so light and heavy rows mix):
-// lanes sweep the (row, element) pairs of 64 of these rows at a time; each
-// element of N+(L[p]) is searched in L[0,p) (by the LDS index ix of L when
-// given, else by binary search), or each L[q], q < p, in N+(L[p]) when that
-// list is gallop_ratio times longer than p.
-template <bool ACC, class LP, class RP>
-__device__ void vtx_rows(const CArgs &a, LP L, int d, RP rows, int w, int first, int stride, int ln,
-                         unsigned long long &bytes, const unsigned short *ix = nullptr, unsigned ix_mask = 0) {
-    for (int cb = 0; first + cb * stride < d; cb += W) {
-        const int ci = first + (cb + ln) * stride;
-        const bool valid = ci < d;
-        const int x = valid ? L[ci] : 0;
-        const long long xb = valid ? a.off[x] : 0;
-        const int xl = valid ? a.split[x] : 0;  // N+(x): all below x
-        const bool sx = (long long)xl <= (long long)a.gallop_ratio * (long long)ci;
-        const int mylen = valid ? (sx ? xl : ci) : 0;
-        if (ACC && valid) bytes += 4ull * (xl + ci) + 16ull;
-        int T = 0;
-        const int myoff = excl_scan(mylen, &T);
-        for (int k0 = 0; k0 < T; k0 += W) {
-            const int j = k0 + ln;
-            // every lane takes part in the cross-lane reads: a segment's
-            // owner lane may itself have no element here
-            by_owner(myoff, k0, T, [&](const auto &pull) {
-                const int s_off = pull(myoff);
-                const int s_sx = pull((int)sx);
-                const long long s_xb = pull(xb);
-                const int s_xl = pull(xl);
-                const int s_ci = pull(ci);
-                if (j < T) {
-                    const int idx = j - s_off;
-                    int pos = -1;
-                    if (s_sx) {
-                        const int y = a.adj[s_xb + idx];
-                        if (ix) {  // probe the index of L: a slot of 0 ends the probe
-                            for (unsigned h = index_hash(y, ix_mask);; h = (h + 1) & ix_mask) {
-                                const int e = ix[h];
-                                if (e == 0) break;
-                                if (L[e - 1] == y) {
-                                    if (e - 1 < s_ci) pos = e - 1;
-                                    break;
-                                }
-                            }
-                        } else {
-                            const int p = lbound(L, s_ci, y);
-                            if (p < s_ci && L[p] == y) pos = p;
-                        }
-                    } else {
-                        if (has(a.adj + s_xb, s_xl, L[idx], a.lin_thr)) pos = idx;
-                    }
-                    if (pos >= 0) atomicOr(&rows[(long long)s_ci * w + (pos >> 5)], 1u << (pos & 31));
-                }
-            });
+// hit[u] |= y[u] in N+(x[u]) for the lanes with act[u]: U searches of lists
+// side by side, so that a round of them waits for one memory latency.
+template <int U>
+__device__ __forceinline__ void search_below(const CArgs &a, const int (&x)[U], const int (&y)[U], const bool (&act)[U],
+                                             bool (&hit)[U]) {
+    long long base[U];
+    int n[U], longest = 0;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        base[u] = 0;
+        n[u] = 0;
+        if (act[u]) {
+            base[u] = a.off[x[u]];
+            n[u] = a.split[x[u]];
         }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) longest = max(longest, n[u]);
+    // halve every list until one entry is left (the last entry <= y, if any)
+    while (ballot(longest > 1)) {
+        int v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = n[u] > 1 ? a.adj[base[u] + (n[u] >> 1)] : INT_MAX;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int half = n[u] >> 1;
+            if (v[u] <= y[u]) base[u] += half;
+            if (n[u] > 1) n[u] -= half;
+        }
+        longest -= longest >> 1;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) hit[u] |= n[u] > 0 && a.adj[base[u]] == y[u];
+}
+
+// Rows of the list L (d entries) for p = first, first + stride, ... (a
+// workgroup's waves interleave their rows, so light and heavy rows mix), w
+// words each, all of them written. Returns the bits set (the pairs of these
+// rows). R rows and two ballots of each are taken at a time, so that 2 R reads
+// are in flight (one row at a time: 2.0 instead of 1.8 ms for the rows of
+// R-MAT s20's tier 0; 8 rows are no faster than 4).
+template <bool ACC, class LP, class RP>
+__device__ __forceinline__ unsigned long long vtx_rows(const CArgs &a, LP L, int d, RP rows, int w, int first,
+                                                       int stride, int ln, unsigned long long &bytes) {
+    constexpr int R = 4;
+    unsigned long long pairs = 0;
+    auto put = [&](int p, int b, unsigned long long m) {  // the 64 bits of ballot b of row p
+        pairs += __popcll(m);
+        const int k = 2 * b + ln;
+        if (ln < 2 && k < w) rows[(long long)p * w + k] = ln ? (unsigned)(m >> 32) : (unsigned)m;
+    };
+    for (int p0 = first; p0 < d; p0 += R * stride) {
+        const int last = min(R - 1, (d - 1 - p0) / stride);  // rows p0 + j stride, j = 0 .. last
+        const int nb = (p0 + last * stride + W - 1) / W;      // ballots of the longest of them
+        int x[R];
+#pragma unroll
+        for (int j = 0; j < R; j++) x[j] = uni(L[p0 + min(j, last) * stride]);
+        if (ACC && ln == 0)
+            for (int j = 0; j <= last; j++) {
+                const int p = p0 + j * stride;
+                bytes += 4ull * (a.split[x[j]] + p) + 16ull + 4ull * ((p >> 5) + 1);
+            }
+        if (x[R - 1] < a.core_n) {  // the largest of the x
+            const unsigned *cr[R];
+#pragma unroll
+            for (int j = 0; j < R; j++) cr[j] = a.core + core_row(x[j]);
+            for (int b = 0; b < nb; b += 2) {
+                unsigned v[2][R];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int q = (b + u) * W + ln;
+                    const int y = q < d ? L[q] : 0;
+#pragma unroll
+                    for (int j = 0; j < R; j++) {
+                        v[u][j] = 0;
+                        if (q < p0 + j * stride && j <= last) v[u][j] = cr[j][y >> 5] >> (y & 31);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int j = 0; j < R; j++)
+                        if (j <= last) put(p0 + j * stride, b + u, ballot(v[u][j] & 1u));
+            }
+        } else {
+            for (int j = 0; j <= last; j++) {
+                const int p = p0 + j * stride, xj = uni(L[p]);
+                const int *xa = a.adj + a.off[xj];
+                const int xl = a.split[xj];
+                const bool core = xj < a.core_n;
+                const unsigned *cr = a.core + core_row(core ? xj : 0);
+                for (int b = 0; b < nb; b++) {
+                    const int q = b * W + ln;
+                    bool hit = false;
+                    if (q < p) {
+                        const int y = L[q];
+                        hit = core ? (cr[y >> 5] >> (y & 31)) & 1u : has(xa, xl, y, a.lin_thr);
+                    }
+                    put(p, b, ballot(hit));
+                }
+            }
+        }
+        const int done = x[R - 1] < a.core_n ? 2 * ((nb + 1) / 2 * 2) : 2 * nb;  // words written
+        for (int j = 0; j <= last; j++)
+            for (int k = done + ln; k < w; k += W) rows[(long long)(p0 + j * stride) * w + k] = 0u;
+    }
+    return pairs;
+}
+
+// ---- counting on the matrix cores ------------------------------------------
+// The deepest two levels of a clique count are, for a set T of positions (the
+// AND of 1, 2 or 3 rows for #K4, #K5, #K6: one "column"),
+//   sum_{r in T} |T & M_r| = sum_r [r in T] |T & M_r|,   and one level up |T|.
+// Both factors are products over positions of 0/1 vectors: for 16 columns and
+// the 16 rows of a tile of consecutive positions r, the counts |T & M_r| are
+// one 16x16x128 matrix instruction per 128 positions with operands M_r and T,
+// and the bits [r in T] are one more with unit vectors e_r in the place of
+// M_r. The operands are 4-bit floats (2.0, 1.0 or 0.5, their products always
+// 1), made from a word of a row by shifts and masks: lane i + 16 g of an
+// operand holds word g of the row's 128-bit chunk, so one LDS word is one
+// lane's operand, and the order of the 32 positions within it is the same on
+// both sides. The sums of a batch of columns are taken in FP32, below 2^24.
+//
+// A wave keeps RT row tiles (a group of 16 RT positions) in registers and
+// streams its columns past them, 16 at a time from a list in LDS, whatever
+// set they come from: the tiles are full even where the sets are small. Only
+// columns with an element above the group's first position are listed. The
+// pair walk this replaces spent about 100 lane-instructions per triple (find
+// the next bit, read two words of its row, AND, popcount) with half of the
+// lanes idle; here a column tile costs RT (chunks + 1) matrix instructions of
+// 16 cycles and about half as many cycles of vector instructions. R-MAT s20,
+// K4 + K5, tiers 0 to 2: 28.0 ms with the pair walk and swept rows, 10.6 ms
+// with this (rows 2.6 ms of it); K6 on R-MAT s16: 840 ms against 5.4 ms. The
+// tiles in registers are what counts: two row tiles instead of four in tier 1
+// cost 2 ms, because every column tile is read and unpacked once per group.
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int kFp4 = 4;  // operand format of the instruction: 4-bit float
+__device__ __forceinline__ v4i operand_rows(unsigned x) {  // bits 0..3 of each nibble as 2.0, 1.0, 0.5, 0.5
+    return v4i{(int)((x << 2) & 0x44444444u), (int)(x & 0x22222222u), (int)((x >> 2) & 0x11111111u),
+               (int)((x >> 3) & 0x11111111u)};
+}
+__device__ __forceinline__ v4i operand_cols(unsigned x) {  // ... as 0.5, 1.0, 2.0, 2.0
+    return v4i{(int)(x & 0x11111111u), (int)(x & 0x22222222u), (int)(x & 0x44444444u), (int)((x >> 1) & 0x44444444u)};
+}
+__device__ __forceinline__ v4f mfma_bits(v4i rows, v4i cols, v4f c) {  // 4-bit operands take four registers; scale arguments 0 select the unscaled form
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+        __builtin_shufflevector(rows, rows, 0, 1, 2, 3, -1, -1, -1, -1),
+        __builtin_shufflevector(cols, cols, 0, 1, 2, 3, -1, -1, -1, -1), c, kFp4, kFp4, 0, 0, 0, 0);
+}
+
+constexpr int CCOLS = 64;  // columns a wave lists before it counts them
+
+// Counts of the columns of the rows p = first, first + stride, ... < d by one
+// wave: DEPTH 1: M_p; 2: M_p & M_q, q in M_p; 3: M_p & M_q & M_x, x in M_p &
+// M_q. deep += sum |T & M_r| over r in T, mid += |T|; for DEPTH 3 cols +=
+// number of columns. KC: chunks of 128 positions a row can have; buf: 2 CCOLS
+// entries of this wave in LDS. Row 0 has no bits: entry 0 pads a tile.
+template <int KC, int RT, int DEPTH, bool ACC>
+__device__ __forceinline__ void count_columns(const unsigned *rows, int w, int d, unsigned *buf, int first, int stride,
+                                              int ln, unsigned long long &deep, unsigned long long &mid,
+                                              unsigned long long &cols, unsigned long long &bytes) {
+    constexpr int GP = 16 * RT;  // positions of a row group
+    const int i = ln & 15, g = ln >> 4;
+    for (int r0 = 0; r0 < d; r0 += GP) {
+        const int khi = (min(d, r0 + GP) - 1) >> 7;  // the chunk of the group; rows have bits up to there
+        v4i A[RT][KC], E[RT];
+#pragma unroll
+        for (int t = 0; t < RT; t++) {
+            const int r = r0 + 16 * t + i;
+            const unsigned *rr = rows + __umul24(min(r, d - 1), w) + g;
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                if (k > khi) break;
+                A[t][k] = operand_rows(4 * k + g < w ? rr[4 * k] : 0u);
+            }
+            E[t] = operand_rows(r < d && (r >> 5) == 4 * khi + g ? 1u << (r & 31) : 0u);
+        }
+        // the group's own words of a column: this lane's word of chunk khi
+        const int own = 4 * khi + g;
+        const unsigned own_mask = own >= r0 >> 5 && own <= (r0 + GP - 1) >> 5 && own < w ? ~0u : 0u;
+        unsigned size = 0;
+        float tri = 0.f;
+        auto tile = [&](int at) {  // the 16 columns buf[at ..]
+            const unsigned e = buf[at + i];
+            const unsigned *r1 = rows + __umul24((int)(e & 1023u), w) + g;
+            const unsigned *r2 = rows + __umul24((int)(e >> 10 & 1023u), w) + g;
+            const unsigned *r3 = rows + __umul24((int)(e >> 20), w) + g;
+            v4f D[RT] = {}, M[RT] = {};
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                if (k > khi) break;
+                unsigned c = r1[4 * k];
+                if (DEPTH >= 2) c &= r2[4 * k];
+                if (DEPTH >= 3) c &= r3[4 * k];
+                const v4i B = operand_cols(c);
+#pragma unroll
+                for (int t = 0; t < RT; t++) D[t] = mfma_bits(A[t][k], B, D[t]);
+                if (k == khi) {
+#pragma unroll
+                    for (int t = 0; t < RT; t++) M[t] = mfma_bits(E[t], B, M[t]);
+                    const unsigned n = __popc(c & own_mask);
+                    size += n;
+                    if (ACC) bytes += 8ull * n * (own + 1);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int x = 0; x < 4; x++) tri += D[t][x] * M[t][x];
+        };
+        int n = 0;
+        // the last CCOLS columns listed; their sums are below 2^24, so exact
+        auto batch = [&]() {
+            n -= CCOLS;
+#pragma unroll 1
+            for (int c = 0; c < CCOLS; c += 16) tile(n + c);
+            deep += (unsigned)tri;
+            tri = 0.f;
+            wsync();
+        };
+        auto list = [&](unsigned long long m, int b, unsigned entry, int shift) {  // a column per bit of m
+            if (m >> ln & 1ull) {
+                buf[n + mbcnt(m)] = entry | (unsigned)(b * W + ln) << shift;
+                if (ACC && r0 == 0) bytes += 8ull * (((b * W + ln) >> 5) + 1);
+            }
+            n += __popcll(m);
+            wsync();
+            if (n >= CCOLS) batch();
+        };
+        // bits of the 64-position block b at or above the group's first position
+        auto above = [&](int b) { return b * W >= r0 ? ~0ull : ~0ull << (r0 & (W - 1)); };
+        auto block = [&](unsigned word, int b) {  // block b of the words the lanes hold
+            return ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)word, 2 * b + 1) << 32 |
+                    (unsigned)__builtin_amdgcn_readlane((int)word, 2 * b)) & above(b);
+        };
+        if (DEPTH == 1) {
+            for (int p = r0 + 1 + first; p < d; p += stride * W) {  // lanes list their rows
+                const int q = p + ln * stride;
+                const unsigned long long m = ballot(q < d);
+                if (q < d) buf[n + mbcnt(m)] = (unsigned)q;
+                n += __popcll(m);
+                wsync();
+                if (n >= CCOLS) batch();
+            }
+        } else {
+            // rows p of this wave above the group, the next row's words read ahead
+            int p = first;
+            if (p <= r0) p += (r0 + stride - first) / stride * stride;
+            unsigned next = p < d && ln < w ? rows[p * w + ln] : 0u;
+            for (; p < d; p += stride) {
+                const unsigned word = next;
+                next = p + stride < d && ln < w ? rows[(p + stride) * w + ln] : 0u;
+                for (int b = r0 / W; b * W < p; b++) {
+                    unsigned long long m = block(word, b);
+                    if (DEPTH == 2) {
+                        if (m) list(m, b, (unsigned)p, 10);
+                    } else {
+                        for (; m; m &= m - 1) {
+                            const int q = b * W + __ffsll((long long)m) - 1;
+                            if (ACC && r0 == 0 && ln == 0) bytes += 8ull * ((q >> 5) + 1);
+                            const unsigned both = word & (ln < w ? rows[q * w + ln] : 0u);
+                            for (int c = r0 / W; c * W < q; c++) {
+                                const unsigned long long mm = block(both, c);
+                                if (r0 == 0 && ln == 0) cols += (unsigned long long)__popcll(mm);
+                                if (mm) list(mm, c, (unsigned)p | (unsigned)q << 10, 20);
+                            }
+                        }
+                    }
+                }
+            }
+        }
+        if (n) {
+            if (ln < (-n & 15)) buf[n + ln] = 0u;
+            wsync();
+#pragma unroll 1
+            for (int c = 0; c < n; c += 16) tile(c);
+            deep += (unsigned)tri;
+            wsync();
+        }
+        mid += size;
     }
 }
 
@@ -1444,80 +1710,24 @@ __device__ __forceinline__ int select_bit(unsigned x, int j) {
     return pos;
 }
 
-// popc(M_p): row p has bits below p only.
-template <class RP>
-__device__ __forceinline__ int row_popc(RP rows, int p, int w) {
-    int c = 0;
-    for (int u = 0; u <= (p >> 5); u++) c += __popc(rows[(long long)p * w + u]);
-    return c;
-}
-
-// t[i] for a run-time i < N, by selects (constant indexes keep t in registers).
-template <int N>
-__device__ __forceinline__ unsigned pick(const unsigned (&t)[N], int i) {
-    unsigned v = t[0];
-#pragma unroll
-    for (int k = 1; k < N; k++) v = i == k ? t[k] : v;
-    return v;
-}
-
-// sum over TC <= u < n of popc(a[u] & b[u]) (and of a[u] & b[u] & c[u]):
-// with MAXW > 0 (n <= MAXW) the loop is unrolled, so every word is read at
-// an immediate offset from its row's base and costs its reads, one bit op
-// and one popcount; MAXW = 0 loops (rows of any width).
-template <int MAXW, int TC, class RP>
-__device__ __forceinline__ unsigned and2_popc(RP a, RP b, int n) {
-    unsigned c = 0;
-    if constexpr (MAXW > 0) {
-#pragma unroll
-        for (int u = TC; u < MAXW; u++) {
-            if (u >= n) break;
-            c += __popc(a[u] & b[u]);
-        }
-    } else {
-        for (int u = TC; u < n; u++) c += __popc(a[u] & b[u]);
-    }
-    return c;
-}
-template <int MAXW, int TC, class RP>
-__device__ __forceinline__ unsigned and3_popc(RP a, RP b, RP c3, int n) {
-    unsigned c = 0;
-    if constexpr (MAXW > 0) {
-#pragma unroll
-        for (int u = TC; u < MAXW; u++) {
-            if (u >= n) break;
-            c += __popc(a[u] & b[u] & c3[u]);
-        }
-    } else {
-        for (int u = TC; u < n; u++) c += __popc(a[u] & b[u] & c3[u]);
-    }
-    return c;
-}
-
-// Counts at and below the pair level. The pairs (p, q), q in M_p, are
-// numbered through off[p] = sum of popc(M_p') over p' < p (off[d] = P), and
-// worker k takes pairs first, first + step, ..., so lanes share the work
-// evenly however uneven the rows are. For a pair: t = M_p & M_q gives #K4
-// += popc(t); each r in t adds popc(t & M_r) to #K5; each s in t & M_r adds
-// popc(t & M_r & M_s) to #K6. Words are read from the rows as needed (no
-// per-lane row copies: that keeps register use, and so occupancy, low),
-// each loop stopping at the last word that can hold bits. Rows are w words
-// apart (w <= MAXW when MAXW > 0); row offsets fit 32 bits and their
-// factors 24 bits, so they take full-rate 24-bit multiplies.
-template <int MAXW, bool ACC, class RP>
-__device__ void vtx_pairs(const CArgs &a, RP rows, int d, int w, const int *off, int P, int first, int step,
-                          unsigned long long *acc, unsigned long long &bytes) {
+// HBM tier: counts at and below the pair level, one pair per lane. The pairs
+// (p, q), q in M_p, are numbered through off[p] = sum of popc(M_p') over p' <
+// p (off[d] = P); worker k takes pairs first, first + step, ... For a pair:
+// t = M_p & M_q gives #K4 += popc(t); each r in t adds popc(t & M_r) to #K5;
+// each s in t & M_r adds popc(t & M_r & M_s) to #K6.
+template <bool ACC>
+__device__ void vtx_pairs(const CArgs &a, const unsigned *rows, int d, int w, const int *off, int P, int first,
+                          int step, unsigned long long *acc, unsigned long long &bytes) {
     for (int k = first; k < P; k += step) {
         int lo = 0, hi = d;  // off[lo] <= k < off[hi]
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
             if (off[mid] <= k) lo = mid; else hi = mid;
         }
-        const int p = lo;
-        const RP rp = rows + __umul24(p, w);
-        int j = k - off[p];
+        const unsigned *rp = rows + (long long)lo * w;
+        int j = k - off[lo];
         int q = 0;
-        for (int u = 0; u <= (p >> 5); u++) {
+        for (int u = 0; u <= (lo >> 5); u++) {
             const unsigned x = rp[u];
             const int c = __popc(x);
             if (j < c) {
@@ -1528,73 +1738,28 @@ __device__ void vtx_pairs(const CArgs &a, RP rows, int d, int w, const int *off,
         }
         const int wq = (q >> 5) + 1;
         if (ACC) bytes += 8ull * wq;
-        const RP rq = rows + __umul24(q, w);
-        // the first TC words of t = M_p & M_q stay in registers; the rest
-        // are re-read from the rows when needed
-        constexpr int TC = 2;
-        unsigned tc[TC];
+        const unsigned *rq = rows + (long long)q * w;
         unsigned c4 = 0;
-#pragma unroll
-        for (int u = 0; u < TC; u++) {
-            tc[u] = u < wq ? (rp[u] & rq[u]) : 0u;
-            c4 += __popc(tc[u]);
-        }
-        c4 += and2_popc<MAXW, TC>(rp, rq, wq);
+        for (int u = 0; u < wq; u++) c4 += __popc(rp[u] & rq[u]);
         acc[4] += c4;
         if (a.kmax < 5) continue;
-        unsigned c5 = 0;  // at most |t| * d bits: fits 32 bits
-        if (a.kmax == 5) {
-            // the next r's row words are read before the current r's are
-            // used, so the LDS latency overlaps the bit operations
-            for (int rw = 0; rw < wq; rw++) {
-                unsigned br = rw < TC ? pick(tc, rw) : (rp[rw] & rq[rw]);
-                if (!br) continue;
-                int r = rw * 32 + __ffs(br) - 1;
-                br &= br - 1;
-                RP rr = rows + __umul24(r, w);
-                unsigned x0 = rr[0], x1 = rr[1];
-                for (;;) {
-                    const bool more = br != 0;
-                    const int rn = more ? rw * 32 + __ffs(br) - 1 : r;
-                    br &= br - 1;
-                    const RP rnp = rows + __umul24(rn, w);
-                    const unsigned y0 = rnp[0], y1 = rnp[1];
-                    if (ACC) bytes += 8ull * (rw + 1);
-                    c5 += __popc(tc[0] & x0) + __popc(tc[1] & x1);
-                    if (rw >= TC) c5 += and3_popc<MAXW, TC>(rp, rq, rr, rw + 1);
-                    if (!more) break;
-                    rr = rnp;
-                    x0 = y0;
-                    x1 = y1;
-                }
-            }
-            acc[5] += c5;
-            continue;
-        }
+        unsigned long long c5 = 0;
         for (int rw = 0; rw < wq; rw++) {
-            // every r in word rw of t needs words 0 .. rw (the same count
-            // for all lanes still in the loop)
-            unsigned br = rw < TC ? pick(tc, rw) : (rp[rw] & rq[rw]);
+            unsigned br = rp[rw] & rq[rw];
             while (br) {
                 const int r = rw * 32 + __ffs(br) - 1;
                 br &= br - 1;
-                const RP rr = rows + __umul24(r, w);
+                const unsigned *rr = rows + (long long)r * w;
                 if (ACC) bytes += 8ull * (rw + 1);
-                // words 0 and 1 of t sit in registers. Word 1 of M_r is read
-                // whatever rw is: it is 0 when r < 32, and it lies within the
-                // rows (lists of more than 32 vertices have rows of 3 or more
-                // words; a shorter list has t's word 1 = 0, and its slice of
-                // at least 32 words runs past row r + 1)
-                c5 += __popc(tc[0] & rr[0]) + __popc(tc[1] & rr[1]);
-                if (rw >= TC) c5 += and3_popc<MAXW, TC>(rp, rq, rr, rw + 1);
+                for (int u = 0; u <= rw; u++) c5 += __popc(rp[u] & rq[u] & rr[u]);
                 if (a.kmax < 6) continue;
-                unsigned c6 = 0;
+                unsigned long long c6 = 0;
                 for (int sw = 0; sw <= rw; sw++) {
                     unsigned bs = rp[sw] & rq[sw] & rr[sw];
                     while (bs) {
                         const int sx = sw * 32 + __ffs(bs) - 1;
                         bs &= bs - 1;
-                        const RP rs = rows + __umul24(sx, w);
+                        const unsigned *rs = rows + (long long)sx * w;
                         if (ACC) bytes += 8ull * ((sx >> 5) + 1);
                         for (int u = 0; u <= (sx >> 5); u++) c6 += __popc(rp[u] & rq[u] & rr[u] & rs[u]);
                     }
@@ -1613,92 +1778,312 @@ __device__ __forceinline__ void clique_flush(const CArgs &a, unsigned long long 
     if (ACC) bytes = wave_sum64(bytes);
     if (ln == 0) {
         for (int k = 3; k <= 6; k++)
-            if (a.pat_of_k[k] >= 0 && acc[k]) atomicAdd(&a.counts[a.pat_of_k[k]], acc[k]);
+            if (a.pat_of_k[k] >= 0 && acc[k]) atomicAdd(&count_copy(a.counts)[a.pat_of_k[k]], acc[k]);
         if (ACC && bytes) atomicAdd(a.bytes, bytes);
     }
 }
 
-// Main tier: one wave per vertex, vertices from the main queue, d <= a.cap
-// (rows in LDS, 8 words wide); larger vertices go to the block tiers.
+// Largest d whose pairs all fit one 64-bit word: d (d - 1) / 2 <= 64.
+constexpr int CTINY = 11;
+// LDS of one wave of the main launch: L, the rows (or the tiny vertices'
+// words) and the pair list.
+struct alignas(16) CWave {
+    int L[CMAIN];
+    unsigned long long rows[CMAIN];
+    unsigned short pairs[W * (CTINY * (CTINY - 1) / 2)];
+};
+static_assert(W * (CTINY * (CTINY - 1) / 2) >= CMAIN * (CMAIN - 1) / 2, "pairs of one vertex fit");
+// p and q of the k-th pair (q < p) in the order of the triangle, k < 2^22.
+__device__ __forceinline__ void tri_pair(int k, int *p, int *q) {
+    int x = (int)((1.f + __builtin_amdgcn_sqrtf(1.f + 8.f * (float)k)) * 0.5f);
+    if (x * (x - 1) / 2 > k) x--;
+    if ((x + 1) * x / 2 <= k) x++;
+    *p = x;
+    *q = k - x * (x - 1) / 2;
+}
+
+// Pairs (p, q), q in M_p, of a main-launch vertex, one per lane: rows are
+// single words, row(r) gives M_r.
+template <bool ACC, class F>
+__device__ __forceinline__ void word_pair(const CArgs &a, F row, unsigned long long mp, unsigned long long mq, int q,
+                                          unsigned long long *acc, unsigned long long &bytes) {
+    const unsigned long long t = mp & mq;
+    if (ACC) bytes += 8ull * ((q >> 5) + 1);
+    acc[4] += __popcll(t);
+    if (a.kmax < 5) return;
+    unsigned c5 = 0;
+    unsigned long long c6 = 0;
+    for (unsigned long long br = t; br; br &= br - 1) {
+        const int r = __ffsll((long long)br) - 1;
+        const unsigned long long mr = t & row(r);
+        if (ACC) bytes += 8ull * ((r >> 5) + 1);
+        c5 += __popcll(mr);
+        if (a.kmax < 6) continue;
+        for (unsigned long long bs = mr; bs; bs &= bs - 1) {
+            const int x = __ffsll((long long)bs) - 1;
+            if (ACC) bytes += 8ull * ((x >> 5) + 1);
+            c6 += __popcll(mr & row(x));
+        }
+    }
+    acc[5] += c5;
+    acc[6] += c6;
+}
+
+// The workgroup tiers' lists: every vertex of the count with d > main_max. A
+// workgroup counts its slab's vertices per tier, reserves their places with
+// one atomic per tier and writes them in a second pass (the main launch's
+// waves did this themselves, at several atomics per chunk on one cache line:
+// 1.2 of the 1.5 ms of R-MAT s20's main launch). Few, large workgroups for the
+// same reason.
+constexpr int kClassifyThreads = 1024;
+__global__ void __launch_bounds__(kClassifyThreads) clique_classify(CArgs a) {
+    __shared__ unsigned long long cnt[CTIERS + 2];
+    const int per = (int)(((long long)(a.root_hi - a.root_lo) + gridDim.x - 1) / gridDim.x);
+    const long long lo = a.root_lo + (long long)blockIdx.x * per;
+    const long long hi = lo + per < a.root_hi ? lo + per : a.root_hi;
+    auto tier_of = [&](int d) {
+        return d <= a.main_max ? -1 : d <= 32 * CT0W ? 0 : d <= 32 * CT1W ? 1 : d <= a.lds_dmax ? 2 : 3;
+    };
+    if (threadIdx.x < CTIERS + 2) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    for (long long v = lo + threadIdx.x; v < hi; v += kClassifyThreads) {
+        const int d = a.split[v], t = tier_of(d);
+        if (t >= 0) atomicAdd(&cnt[t], 1ull);
+        if (d > a.cap) atomicAdd(&cnt[CTIERS], 1ull);
+        if (d > a.cap && d <= 512) atomicAdd(&cnt[CTIERS + 1], 1ull);
+    }
+    __syncthreads();
+    if (threadIdx.x < CTIERS + 2) {
+        const unsigned long long c = cnt[threadIdx.x];
+        if (c) cnt[threadIdx.x] = atomicAdd(&a.ovf_n[threadIdx.x], c);
+        if (threadIdx.x == 3 && c && !a.grows) atomicOr(a.err, 16u);  // no HBM tier in this count
+    }
+    __syncthreads();
+    for (long long v = lo + threadIdx.x; v < hi; v += kClassifyThreads) {
+        const int t = tier_of(a.split[v]);
+        if (t < 0) continue;
+        const long long idx = (long long)atomicAdd(&cnt[t], 1ull);
+        if (idx < a.tier_cap[t]) a.tier[t][idx] = (int)v;
+        else if (a.tier_cap[t] > 0) atomicOr(a.err, 4u);
+    }
+}
+static_assert(CTIERS == 4, "ovf_n[4] and [5] count vertices with d > cap");
+
+// Main launch: vertices with d <= main_max; the tiers take the larger ones. The
+// vertices are dealt out in chunks; chunk c of the N chunks holds the vertices
+// root_lo + c + i N, so that the heavy vertices, which are neighbours in the
+// degree order, spread over the chunks. A wave starts with the chunk of its
+// own number and takes further ones from the queue: a grab is an atomic on
+// one address, 17 ns each however many waves there are (chunks of 4 vertices
+// from a counter alone held R-MAT s20's launch at 4.6 ms).
+// Of a block of up to 64 vertices of a chunk, the tiny ones (d <= CTINY) are
+// taken together, one position pair per lane, and keep all their rows in one
+// word (row p at bit p (p - 1) / 2); the others follow one by one, with the
+// next one's list read ahead.
 // MODE bit 0: accumulate W_alg; bit 1: timeline records (separate
 // instantiations, so that a timed count carries none of their work or
 // registers).
 template <int MODE>
-__global__ void __launch_bounds__(256) clique_kernel(CArgs a, int wave_bytes) {
+__global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
-    unsigned char *base = smem + (size_t)wid * wave_bytes;
-    int *L = reinterpret_cast<int *>(base);
-    unsigned *rows = reinterpret_cast<unsigned *>(L + a.cap + 4);  // L: d entries, then d + 1 offsets
+    CWave &C = reinterpret_cast<CWave *>(smem)[wid];
     unsigned long long acc[7] = {0, 0, 0, 0, 0, 0, 0}, bytes = 0;  // per lane
     constexpr bool ACC = MODE & 1, tl = (MODE & 2) != 0;
     const long long tl_t0 = tl ? wall_clock64() : 0;
     long long tl_build = 0, tl_count = 0, tl_items = 0, tl_pairs = 0;
-    for (;;) {
-        unsigned long long r = 0;
-        if (ln == 0) r = atomicAdd(&a.queue[0], (unsigned long long)a.chunk);
-        const long long v_lo = a.root_lo + uni64((long long)__shfl(r, 0));
-        if (v_lo >= a.root_hi) break;
-        const long long v_hi = v_lo + a.chunk < a.root_hi ? v_lo + a.chunk : a.root_hi;
-        for (long long vv = v_lo; vv < v_hi; vv++) {
-            const int v0 = (int)vv;
-            const int d = uni(a.split[v0]);
-            if (d < 2) continue;
-            if (d > a.cap) {
-                if (ln == 0) {
-                    const int t = d <= 32 * CMIDW ? 0 : (d <= 32 * CBIGW ? 1 : 2);
-                    const int parts = clique_parts(t, d);
-                    atomicAdd(&a.ovf_n[3], 1ull);  // vertices handed on (statistics)
-                    if (t == 2 && !a.grows) {
-                        atomicOr(a.err, 16u);  // no HBM tier in this count (allocation-free entry point)
-                    } else {
-                        const unsigned long long idx = atomicAdd(&a.ovf_n[t], (unsigned long long)parts);
-                        if ((long long)(idx + parts) <= a.ovf_cap) {
-                            for (int k = 0; k < parts; k++) a.tier[t][idx + k] = (long long)v0 * CSPLIT_ENC + k;
-                        } else {
-                            atomicOr(a.err, 4u);
+    const int lim = a.main_max;
+    const long long chunks = ((long long)(a.root_hi - a.root_lo) + a.chunk - 1) / a.chunk;
+    const int wpb = blockDim.x / W;
+    const long long waves = (long long)gridDim.x * wpb;
+    long long chunk = uni64((long long)blockIdx.x * wpb + wid);
+    while (chunk < chunks) {
+        for (int cb = 0; cb < a.chunk; cb += W) {
+            const long long v = a.root_lo + chunk + (cb + ln) * chunks;
+            const bool mine = cb + ln < a.chunk && v < a.root_hi;
+            const int d_l = mine ? a.split[v] : 0;
+            const long long b_l = mine ? a.off[v] : 0;
+            const unsigned long long tiny = ballot(d_l >= 2 && d_l <= min(lim, CTINY));
+            if (tiny) {
+                const long long c0 = tl ? clock64() : 0;
+                const bool is = tiny >> ln & 1ull;
+                C.rows[ln] = 0;
+                if (ACC && is) {
+                    bytes += 4ull * d_l + 16ull;
+                    for (int p = 0; p < d_l; p++) bytes += 4ull * (a.split[a.adj[b_l + p]] + p) + 16ull + 4ull;
+                }
+                int T = 0, run = 0;
+                const int myoff = excl_scan(is ? d_l * (d_l - 1) / 2 : 0, &T);
+                wsync();
+                constexpr int U = 4;  // steps in flight
+                for (int k0 = 0; k0 < T; k0 += U * W) {
+                    int x[U], y[U], s[U], pos[U];
+                    unsigned word[U];
+                    bool in[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const int k = k0 + u * W + ln;
+                        s[u] = 0;
+#pragma unroll
+                        for (int step = 32; step >= 1; step >>= 1)
+                            if (bperm(myoff, s[u] + step) <= k && s[u] + step < W) s[u] += step;
+                        in[u] = k < T;
+                        pos[u] = k - bperm(myoff, s[u]);
+                        const long long rb = bperm64(b_l, s[u]);
+                        x[u] = y[u] = 0;
+                        if (in[u]) {
+                            int p, q;
+                            tri_pair(pos[u], &p, &q);
+                            x[u] = a.adj[rb + p];
+                            y[u] = a.adj[rb + q];
                         }
                     }
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        word[u] = 0;
+                        if (in[u] && x[u] < a.core_n) word[u] = a.core[core_row(x[u]) + (y[u] >> 5)] >> (y[u] & 31);
+                    }
+                    bool hit[U], far[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        hit[u] = word[u] & 1u;
+                        far[u] = in[u] && x[u] >= a.core_n;
+                    }
+                    search_below<U>(a, x, y, far, hit);
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const unsigned long long m = ballot(hit[u]);
+                        if (hit[u] && a.kmax >= 4) {
+                            atomicOr(reinterpret_cast<unsigned *>(&C.rows[s[u]]) + (pos[u] >> 5), 1u << (pos[u] & 31));
+                            C.pairs[run + mbcnt(m)] = (unsigned short)(s[u] << 6 | pos[u]);
+                        }
+                        run += __popcll(m);
+                    }
                 }
-                continue;
+                if (ln == 0) acc[3] += (unsigned long long)run;
+                wsync();
+                const long long c1 = tl ? clock64() : 0;
+                if (a.kmax >= 4) {
+                    for (int k = ln; k < run; k += W) {
+                        const int e = C.pairs[k];
+                        const unsigned long long m = C.rows[e >> 6];
+                        int p, q;
+                        tri_pair(e & 63, &p, &q);
+                        auto row = [&](int r) { return (m >> (r * (r - 1) / 2)) & ((1ull << r) - 1); };
+                        word_pair<ACC>(a, row, row(p), row(q), q, acc, bytes);
+                    }
+                    wsync();
+                }
+                if (tl) {
+                    tl_build += c1 - c0;
+                    tl_count += clock64() - c1;
+                    tl_items += __popcll(tiny);
+                    tl_pairs += run;
+                }
             }
-            const long long c0 = tl ? clock64() : 0;
-            const long long rb = a.off[v0];
-            const int w = row_words(d);
-            for (int k = ln; k < d; k += W) L[k] = a.adj[rb + k];
-            for (int k = ln; k < d * w; k += W) rows[k] = 0u;
-            if (ACC && ln == 0) bytes += 4ull * d + 16ull;
-            wsync();
-            vtx_rows<ACC>(a, L, d, rows, w, 0, 1, ln, bytes);
-            wsync();
-            // L is no longer needed: it holds the pair offsets from here on
-            int *off = L;
-            int run = 0;
-            for (int pb = 0; pb < d; pb += W) {
-                const int p = pb + ln;
-                const int c = p < d ? row_popc(rows, p, w) : 0;
-                if (ACC && p < d) bytes += 4ull * ((p >> 5) + 1);
-                int tot = 0;
-                const int x = excl_scan(c, &tot);
-                if (p < d) off[p] = run + x;
-                run += tot;
+            unsigned long long todo = ballot(d_l > CTINY && d_l <= lim);
+            int d = 0, y = 0;
+            if (todo) {
+                const int l = __ffsll((long long)todo) - 1;
+                d = LanePull{l}(d_l);
+                const long long rb = LanePull{l}(b_l);
+                if (ln < d) y = a.adj[rb + ln];
             }
-            if (ln == 0) {
-                off[d] = run;
-                acc[3] += (unsigned long long)run;
-            }
-            wsync();
-            const long long c1 = tl ? clock64() : 0;
-            if (a.kmax >= 4)
-                vtx_pairs<row_words(32 * CMAXW), ACC>(a, (const unsigned *)rows, d, w, off, run, ln, W, acc, bytes);
-            wsync();
-            if (tl) {
-                tl_build += c1 - c0;
-                tl_count += clock64() - c1;
-                tl_items++;
-                tl_pairs += run;
+            while (todo) {
+                const long long c0 = tl ? clock64() : 0;
+                todo &= todo - 1;
+                int dn = 0, yn = 0;  // the next vertex's list
+                if (todo) {
+                    const int l = __ffsll((long long)todo) - 1;
+                    dn = LanePull{l}(d_l);
+                    const long long rb = LanePull{l}(b_l);
+                    if (ln < dn) yn = a.adj[rb + ln];
+                }
+                if (ACC) {
+                    if (ln == 0) bytes += 4ull * d + 16ull;
+                    if (ln < d) bytes += 4ull * (a.split[y] + ln) + 16ull + 4ull * ((ln >> 5) + 1);
+                }
+                int run = 0;
+                C.L[ln] = y;
+                // core vertices come first in the sorted list
+                const int pc = __popcll(ballot(ln < d && y < a.core_n));
+                unsigned long long row_l = 0;  // row ln
+                constexpr int U = 8;           // row reads in flight
+                for (int p = 1; p < pc; p += U) {
+                    unsigned v[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        v[u] = 0;
+                        const int x = LanePull{min(p + u, W - 1)}(y);
+                        if (ln < p + u && p + u < pc) v[u] = a.core[core_row(x) + (y >> 5)] >> (y & 31);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const unsigned long long m = ballot(v[u] & 1u);
+                        if (ln == p + u) row_l = m;
+                        if (v[u] & 1u) C.pairs[run + mbcnt(m)] = (unsigned short)((p + u) << 8 | ln);
+                        run += __popcll(m);
+                    }
+                }
+                C.rows[ln] = row_l;
+                wsync();
+                // the other vertices' rows: one pair (p, q) per lane
+                const int p0 = max(pc, 1), k0 = p0 * (p0 - 1) / 2, k1 = d * (d - 1) / 2;
+                constexpr int F = 4;  // searches in flight
+                for (int kb = k0; kb < k1; kb += F * W) {
+                    int p[F], q[F], x[F], z[F];
+                    bool in[F], hit[F];
+#pragma unroll
+                    for (int u = 0; u < F; u++) {
+                        const int k = kb + u * W + ln;
+                        in[u] = k < k1;
+                        hit[u] = false;
+                        p[u] = q[u] = 0;
+                        if (in[u]) tri_pair(k, &p[u], &q[u]);
+                        x[u] = C.L[p[u]];
+                        z[u] = C.L[q[u]];
+                    }
+                    search_below<F>(a, x, z, in, hit);
+#pragma unroll
+                    for (int u = 0; u < F; u++) {
+                        const unsigned long long m = ballot(hit[u]);
+                        if (hit[u]) {
+                            atomicOr(reinterpret_cast<unsigned *>(&C.rows[p[u]]) + (q[u] >> 5), 1u << (q[u] & 31));
+                            C.pairs[run + mbcnt(m)] = (unsigned short)(p[u] << 8 | q[u]);
+                        }
+                        run += __popcll(m);
+                    }
+                }
+                if (ln == 0) acc[3] += (unsigned long long)run;
+                wsync();
+                const long long c1 = tl ? clock64() : 0;
+                if (a.kmax >= 4) {
+                    auto row = [&](int p) { return C.rows[p]; };
+                    for (int k = ln; k < run; k += W) {
+                        const int pq = C.pairs[k];
+                        word_pair<ACC>(a, row, C.rows[pq >> 8], C.rows[pq & 255], pq & 255, acc, bytes);
+                    }
+                }
+                wsync();
+                if (tl) {
+                    tl_build += c1 - c0;
+                    tl_count += clock64() - c1;
+                    tl_items++;
+                    tl_pairs += run;
+                }
+                d = dn;
+                y = yn;
             }
         }
+        // the queue counts the chunks after the waves' own; it is read before
+        // it is grabbed, so that a drained queue costs no atomic
+        if (waves >= chunks) break;
+        unsigned long long r = 0;
+        if (ln == 0) {
+            r = __atomic_load_n(&a.queue[0], __ATOMIC_RELAXED);
+            if ((long long)r + waves < chunks) r = atomicAdd(&a.queue[0], 1ull);
+        }
+        chunk = waves + uni64((long long)__shfl(r, 0));
     }
     clique_flush<ACC>(a, acc, bytes, ln);
     if (tl && ln == 0) {
@@ -1707,134 +2092,179 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a, int wave_bytes) {
     }
 }
 
-// Workgroup tiers: the NW waves of a workgroup share one vertex of tier
-// list TIER. Rows MW words wide (d <= 32 * MW) sit in LDS or, without LDS,
-// in the workgroup's HBM scratch; MW == 0 (any d up to hcap) reads every
-// word from HBM as needed. The waves split the rows between them for the
-// build and take pairs round-robin for the count.
-template <int MW, bool LDS, int TIER, int NW, int MODE>
-__global__ void __launch_bounds__(64 * NW, NW == CBLOCKW0 ? 8 : 1) clique_block_kernel(CArgs a) {
+// Next item of a tier's queue: the vertex, or -1 when the queue is drained.
+__device__ __forceinline__ int tier_item(const CArgs &a, int tier, int *part, int *parts) {
+    const unsigned long long made = a.ovf_n[tier], cap = (unsigned long long)a.tier_cap[tier];
+    const unsigned long long vertices = made < cap ? made : cap;
+    const int np = clique_parts(a.kmax, vertices, (int)gridDim.x);
+    const unsigned long long r = atomicAdd(&a.queue[1 + tier], 1ull);
+    *part = (int)(r % np);
+    *parts = np;
+    return r / np < vertices ? a.tier[tier][r / np] : -1;
+}
+
+// Workgroup tiers with rows in LDS: the NW waves of a workgroup share one
+// vertex of tier list TIER, d <= 32 MW. They split the rows for the build, and
+// the columns of the count by their first row.
+template <int MW, int TIER, int NW, int MODE>
+__global__ void __launch_bounds__(64 * NW, clique_occupancy(TIER)) clique_block_kernel(CArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
     constexpr int lcap = 32 * MW;
-    // LDS: the list (then the pair offsets), then the rows
-    int *Ls = reinterpret_cast<int *>(smem);
-    unsigned *rows_l = reinterpret_cast<unsigned *>(Ls + (LDS ? lcap + 4 : 0));
-    // the index of L after the rows (LDS tiers): one entry per thread
-    static_assert(!LDS || lcap <= 64 * NW, "one index entry per thread");
-    unsigned short *ix = LDS ? reinterpret_cast<unsigned short *>(rows_l + lcap * row_words(lcap)) : nullptr;
-    constexpr unsigned ix_mask = (unsigned)index_slots(lcap) - 1;
-    static_assert((index_slots(lcap) & (index_slots(lcap) - 1)) == 0, "index slots are a power of two");
-    __shared__ long long vsh;
-    __shared__ int wtot[NW];
-    const int hws = row_words(a.hcap);
-    unsigned *rows_g = LDS ? nullptr : a.grows + (long long)blockIdx.x * a.hcap * hws;
-    int *off_g = LDS ? nullptr : a.goff + (long long)blockIdx.x * (a.hcap + 1);
+    constexpr int KC = MW / 4;            // chunks of 128 positions
+    constexpr int RT = MW <= 16 ? 4 : 2;  // row tiles held at once (registers)
+    unsigned *rows = reinterpret_cast<unsigned *>(smem);
+    int *L = reinterpret_cast<int *>(rows + tier_row_words(MW));
+    unsigned *buf = reinterpret_cast<unsigned *>(L) + wid * 2 * CCOLS;
+    __shared__ int vsh, psh, nsh;
     unsigned long long acc[7] = {0, 0, 0, 0, 0, 0, 0}, bytes = 0;
     constexpr bool ACC = MODE & 1, tl = (MODE & 2) != 0;
     const long long tl_t0 = tl ? wall_clock64() : 0;
     long long tl_build = 0, tl_count = 0, tl_items = 0, tl_pairs = 0, c0 = 0, c1 = 0;
     for (;;) {
         if (tl) c0 = clock64();
-        if (threadIdx.x == 0) {
-            const unsigned long long r = atomicAdd(&a.queue[1 + TIER], 1ull);
-            const unsigned long long cnt = a.ovf_n[TIER];
-            vsh = (r < cnt && (long long)r < a.ovf_cap) ? a.tier[TIER][r] : -1;
-        }
+        if (threadIdx.x == 0) vsh = tier_item(a, TIER, &psh, &nsh);
         __syncthreads();
-        if (vsh < 0) break;
-        const int v0 = (int)(vsh / CSPLIT_ENC);
-        const int part = (int)(vsh % CSPLIT_ENC);
+        const int v0 = vsh, part = psh, parts = nsh;
+        if (v0 < 0) break;
         const int d = a.split[v0];
-        const int parts = clique_parts(TIER, d);
         const long long rb = a.off[v0];
         const int w = row_words(d);
-        if (d > (MW > 0 ? lcap : a.hcap) || d > a.hcap) {  // cannot happen: lists are split by d
-            if (threadIdx.x == 0) atomicOr(a.err, 8u);
-        } else {
-            if (LDS)
-                for (int k = threadIdx.x; k < d; k += 64 * NW) Ls[k] = a.adj[rb + k];
-            unsigned *rows = LDS ? rows_l : rows_g;
-            for (long long k = threadIdx.x; k < (long long)d * w; k += 64 * NW) rows[k] = 0u;
-            if (LDS)
-                for (int k = threadIdx.x; k < index_slots(lcap); k += 64 * NW) ix[k] = 0;
-            // every part builds the rows; W_alg charges one build
-            unsigned long long build_bytes = 0;
-            if (ACC && threadIdx.x == 0) build_bytes += 4ull * d + 16ull;
-            if (!LDS) __threadfence();
-            __syncthreads();
-            if (LDS) {
-                // thread i enters L[i]: each round it writes 1 + i to its slot
-                // if the slot is empty, and after a barrier moves on if
-                // another thread's entry holds the slot. Entries are never
-                // overwritten, and one moves past a slot only when that slot
-                // is taken, so every slot between an entry's hash and its
-                // place stays full, as linear probing needs.
-                const int i = threadIdx.x;
-                bool pending = i < d;
-                unsigned h = pending ? index_hash(Ls[i], ix_mask) : 0u;
-                while (__syncthreads_or(pending)) {
-                    if (pending && ix[h] == 0) ix[h] = (unsigned short)(i + 1);
-                    __syncthreads();
-                    if (pending) {
-                        if (ix[h] == i + 1) pending = false;
-                        else h = (h + 1) & ix_mask;
-                    }
-                }
-            }
-            const int *L = LDS ? Ls : a.adj + rb;
-            vtx_rows<ACC>(a, L, d, rows, w, wid, NW, ln, build_bytes, ix, ix_mask);
-            if (!LDS) __threadfence();
-            __syncthreads();
-            // pair offsets: block-wide exclusive prefix of popc(M_p)
-            int *off = LDS ? Ls : off_g;
-            int run = 0;
-            for (int pb = 0; pb < d; pb += 64 * NW) {
-                const int p = pb + (int)threadIdx.x;
-                const int c = p < d ? row_popc((const unsigned *)rows, p, w) : 0;
-                if (ACC && p < d) build_bytes += 4ull * ((p >> 5) + 1);
-                int tot = 0;
-                const int x = excl_scan(c, &tot);
-                if (ln == 0) wtot[wid] = tot;
-                __syncthreads();
-                int pre = 0, all = 0;
-                for (int k = 0; k < NW; k++) {
-                    const int t = wtot[k];
-                    if (k < wid) pre += t;
-                    all += t;
-                }
-                if (p < d) off[p] = run + pre + x;
-                run += all;
-                __syncthreads();
-            }
-            if (threadIdx.x == 0) {
-                off[d] = run;
-                if (part == 0) acc[3] += (unsigned long long)run;
-            }
-            if (part == 0) bytes += build_bytes;
-            if (!LDS) __threadfence();
-            __syncthreads();
-            if (tl) c1 = clock64();
-            if (a.kmax >= 4)
-                vtx_pairs<(MW > 0 ? row_words(32 * MW) : 0), ACC>(a, (const unsigned *)rows, d, w, off, run,
-                                                           part * 64 * NW + (int)threadIdx.x,
-                          64 * NW * parts, acc, bytes);
-            if (tl) {
-                tl_pairs += run;
-                tl_items++;
+        const bool fits = d <= lcap;  // always: lists are split by d
+        if (!fits && threadIdx.x == 0) atomicOr(a.err, 8u);
+        if (fits)
+            for (int k = threadIdx.x; k < d; k += 64 * NW) L[k] = a.adj[rb + k];
+        __syncthreads();
+        if (fits) {
+            unsigned long long bb = 0;  // every part builds the rows; W_alg and #K3 charge one build
+            const unsigned long long pr = vtx_rows<ACC>(a, (const int *)L, d, rows, w, wid, NW, ln, bb);
+            if (part == 0) {
+                if (ln == 0) acc[3] += pr;
+                if (ACC) bytes += bb + (threadIdx.x == 0 ? 4ull * d + 16ull : 0ull);
+                tl_pairs += (long long)pr;
             }
         }
+        __syncthreads();  // the rows are complete, and L is free for the column lists
+        if (tl) c1 = clock64();
+        if (fits && a.kmax >= 4) {
+            const int first = part * NW + wid, stride = NW * parts;
+            unsigned long long none = 0;
+            if (a.kmax == 4)
+                count_columns<KC, RT, 1, ACC>(rows, w, d, buf, first, stride, ln, acc[4], none, none, bytes);
+            else if (a.kmax == 5)
+                count_columns<KC, RT, 2, ACC>(rows, w, d, buf, first, stride, ln, acc[5], acc[4], none, bytes);
+            else
+                count_columns<KC, RT, 3, ACC>(rows, w, d, buf, first, stride, ln, acc[6], acc[5], acc[4], bytes);
+        }
         __syncthreads();
-        if (tl && c1) {
+        if (tl) {
             tl_build += c1 - c0;
             tl_count += clock64() - c1;
-            c1 = 0;
+            tl_items++;
         }
     }
     clique_flush<ACC>(a, acc, bytes, ln);
     if (tl && threadIdx.x == 0)
         tl_write(a.tl, a.tl_base + blockIdx.x, 1 + TIER, blockIdx.x, tl_t0, wall_clock64(), tl_build, tl_count,
                  tl_items, tl_pairs);
+}
+
+// Workgroup tier 3: vertices whose rows do not fit LDS. Rows and pair
+// offsets sit in the workgroup's HBM scratch; the waves split the rows for
+// the build and take pairs round-robin for the count.
+template <int MODE>
+__global__ void __launch_bounds__(64 * CNW3) clique_hbm_kernel(CArgs a) {
+    constexpr int TIER = 3, NW = CNW3;
+    const int wid = threadIdx.x / W, ln = threadIdx.x % W;
+    __shared__ int vsh, psh, nsh;
+    __shared__ int wtot[NW];
+    unsigned *rows = a.grows + (long long)blockIdx.x * a.hcap * row_words(a.hcap);
+    int *off = a.goff + (long long)blockIdx.x * (a.hcap + 1);
+    unsigned long long acc[7] = {0, 0, 0, 0, 0, 0, 0}, bytes = 0;
+    constexpr bool ACC = MODE & 1, tl = (MODE & 2) != 0;
+    const long long tl_t0 = tl ? wall_clock64() : 0;
+    long long tl_build = 0, tl_count = 0, tl_items = 0, tl_pairs = 0, c0 = 0, c1 = 0;
+    for (;;) {
+        if (tl) c0 = clock64();
+        if (threadIdx.x == 0) vsh = tier_item(a, TIER, &psh, &nsh);
+        __syncthreads();
+        const int v0 = vsh, part = psh, parts = nsh;
+        if (v0 < 0) break;
+        const int d = a.split[v0];
+        const int w = row_words(d);
+        const bool fits = d <= a.hcap;  // always: hcap is the maximum out-degree
+        if (!fits && threadIdx.x == 0) atomicOr(a.err, 8u);
+        unsigned long long bb = 0;
+        if (fits) (void)vtx_rows<ACC>(a, a.adj + a.off[v0], d, rows, w, wid, NW, ln, bb);
+        if (ACC && fits && part == 0) bytes += bb + (threadIdx.x == 0 ? 4ull * d + 16ull : 0ull);
+        __threadfence();
+        __syncthreads();
+        // pair offsets: block-wide exclusive prefix of popc(M_p)
+        int run = 0;
+        for (int pb = 0; fits && pb < d; pb += 64 * NW) {
+            const int p = pb + (int)threadIdx.x;
+            int c = 0;
+            if (p < d)
+                for (int u = 0; u <= (p >> 5); u++) c += __popc(rows[(long long)p * w + u]);
+            int tot = 0;
+            const int x = excl_scan(c, &tot);
+            if (ln == 0) wtot[wid] = tot;
+            __syncthreads();
+            int pre = 0, all = 0;
+            for (int k = 0; k < NW; k++) {
+                const int t = wtot[k];
+                if (k < wid) pre += t;
+                all += t;
+            }
+            if (p < d) off[p] = run + pre + x;
+            run += all;
+            __syncthreads();
+        }
+        if (fits && threadIdx.x == 0) {
+            off[d] = run;
+            if (part == 0) acc[3] += (unsigned long long)run;
+        }
+        __threadfence();
+        __syncthreads();
+        if (tl) c1 = clock64();
+        if (fits && a.kmax >= 4)
+            vtx_pairs<ACC>(a, rows, d, w, off, run, part * 64 * NW + (int)threadIdx.x, 64 * NW * parts, acc, bytes);
+        __syncthreads();
+        if (tl) {
+            tl_build += c1 - c0;
+            tl_count += clock64() - c1;
+            tl_items++;
+            tl_pairs += run;
+        }
+    }
+    clique_flush<ACC>(a, acc, bytes, ln);
+    if (tl && threadIdx.x == 0)
+        tl_write(a.tl, a.tl_base + blockIdx.x, 1 + TIER, blockIdx.x, tl_t0, wall_clock64(), tl_build, tl_count,
+                 tl_items, tl_pairs);
+}
+
+// Core bitmap rows of the vertices [0, core_n): a wave builds a row in its
+// LDS slice (core_n <= CCORE bits) and writes it out whole.
+constexpr int CCORE = 1 << 16;
+__global__ void __launch_bounds__(256) core_rows_kernel(const long long *off, const int *adj, const int *split,
+                                                        int core_n, unsigned *core) {
+    __shared__ unsigned buf[4][CCORE / 32];
+    const int wid = threadIdx.x / W, ln = threadIdx.x % W;
+    unsigned *b = buf[wid];
+    for (int x = blockIdx.x * 4 + wid; x < core_n; x += gridDim.x * 4) {
+        const int words = (x + 31) >> 5, len = split[x];
+        const long long xb = off[x];
+        for (int k = ln; k < words; k += W) b[k] = 0u;
+        wsync();
+        for (int k = ln; k < len; k += W) {
+            const int y = adj[xb + k];
+            atomicOr(&b[y >> 5], 1u << (y & 31));
+        }
+        wsync();
+        unsigned *row = core + core_row(x);
+        for (int k = ln; k < words; k += W) row[k] = b[k];
+        wsync();
+    }
 }
 
 __global__ void fill_u64(unsigned long long *p, long long n, unsigned long long v) {
@@ -1931,6 +2361,9 @@ struct DeviceGraph {
     long long *off = nullptr;
     int *adj = nullptr;
     int *split = nullptr;
+    // core bitmap of the clique store (core_n < 0: not built)
+    unsigned *core = nullptr;
+    int core_n = -1;
     // hub bitmaps, built for the threshold hub_degree (0 = not built)
     int hub_degree = 0;
     int n_hubs = 0;
@@ -1951,6 +2384,7 @@ struct DeviceGraph {
         if (off) (void)hipFree(off);
         if (adj) (void)hipFree(adj);
         if (split) (void)hipFree(split);
+        if (core) (void)hipFree(core);
     }
 };
 
@@ -1964,7 +2398,7 @@ struct PlanDevice {
     gatk::KArgs *dargs = nullptr;     // arguments of the array-store launches of a count
     long long *tl = nullptr;          // timeline records of the last GAT_FLAG_TIMELINE count
     int tl_n = 0;                     // records that count reserved (0: none)
-    long long *tier[3] = {};  // clique vertices of the workgroup tiers
+    int *tier[gatk::CTIERS] = {};  // clique vertices of the workgroup tiers
     long long ovf_cap = 0;
     int *gstore = nullptr;
     size_t gstore_bytes = 0;
@@ -1973,7 +2407,7 @@ struct PlanDevice {
     // clique HBM-tier rows and pair offsets
     unsigned *grows = nullptr;
     int *goff = nullptr;
-    int big_waves = 0, big_cap = 0;
+    int big_groups = 0, big_cap = 0;
     std::shared_ptr<DeviceGraph> dg;
     // captured graph
     hipGraphExec_t gexec = nullptr;
@@ -1987,7 +2421,7 @@ void destroy_plan_device(PlanDevice *d) {
     for (auto &e : d->ev)
         if (e) (void)hipEventDestroy(e);
     for (void *p : {(void *)d->plan, (void *)d->dargs, (void *)d->tl, (void *)d->counts, (void *)d->queue, (void *)d->ovf_n, (void *)d->bytes,
-                    (void *)d->err, (void *)d->ovf, (void *)d->subs, (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2],
+                    (void *)d->err, (void *)d->ovf, (void *)d->subs, (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2], (void *)d->tier[3],
                     (void *)d->gstore, (void *)d->grows,
                     (void *)d->goff})
         if (p) (void)hipFree(p);
@@ -2063,6 +2497,34 @@ static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr) {
     return GAT_OK;
 }
 
+// Core bitmap of the clique store: the rows of the first core vertices, at
+// most gatk::CCORE of them and within `words` words (about four times the
+// CSR: on R-MAT s20 the 65,536 core vertices hold 86-100 % of the positions,
+// 268 MB against 126 MB of lists).
+static int core_vertices(int64_t n, long long words) {
+    int lo = 0, hi = (int)std::min<int64_t>(n, gatk::CCORE);  // the largest x with core_row(x) <= words
+    while (lo < hi) {
+        const int mid = lo + (hi - lo + 1) / 2;
+        if ((long long)gatk::core_row(mid) <= words) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+static int ensure_core(const Graph &g, DeviceGraph *dg) {
+    if (dg->core_n >= 0) return GAT_OK;
+    const int h = core_vertices(g.n, std::max<long long>(1 << 21, 4ll * g.m));
+    const size_t words = gatk::core_row(h);
+    HIPCHECK(hipMalloc(&dg->core, sizeof(unsigned) * std::max<size_t>(words, 16)));
+    if (h > 0) {
+        hipLaunchKernelGGL(gatk::core_rows_kernel, dim3(std::min((h + 3) / 4, 4096)), dim3(256), 0, nullptr, dg->off,
+                           dg->adj, dg->split, h, dg->core);
+        HIPCHECK(hipGetLastError());
+        HIPCHECK(hipDeviceSynchronize());
+    }
+    dg->core_n = h;
+    return GAT_OK;
+}
+
 // Split subtasks: capacity of each level's list, and the default time a
 // task runs in the tail of a launch before it hands on its unfinished loops.
 // Subtask counters live at ovf_n[8 + k] (k = 1 .. levels: LDS levels, then
@@ -2088,14 +2550,21 @@ struct Launch {
     bool clique = false;  // bitmap clique path
     gatk::CArgs ca;
     size_t clique_lds = 0;
-    int clique_wave_bytes = 0;
-    dim3 mid_grid;      // workgroup tier 0 (rows in LDS)
-    size_t mid_lds = 0;
-    dim3 t1_grid;       // workgroup tier 1 (LDS when t1_lds > 0, else HBM)
-    size_t t1_lds = 0;
-    dim3 big_grid;      // workgroup tier 2 (HBM)
+    dim3 tier_grid[gatk::CTIERS];  // workgroup tiers; x = 0: no vertex can reach the tier
+    size_t tier_lds[gatk::CTIERS] = {};
     long long tasks = 0;  // root edges of the count
+    int chunk = 1;        // queue_chunk
+    bool heavy = false;   // clique: some vertex may have more than main_max neighbours below it
 };
+
+// Vertices per chunk of the clique main launch: as configured, but no more
+// than one and no fewer than a quarter of a wave's share. (Chunks mix heavy
+// and light vertices, so that few of them balance; a chunk per grab costs an
+// atomic, and a wave without a chunk is idle.)
+static int clique_chunk(int configured, long long vertices, long long waves) {
+    const long long share = std::max(1ll, (vertices + waves - 1) / waves);
+    return (int)std::min(share, std::max<long long>(configured, (share + 3) / 4));
+}
 
 // Restrict a prepared count to the root vertices [lo, hi): the array store
 // takes the directed edges of those vertices, the bitmap store those top
@@ -2103,9 +2572,11 @@ struct Launch {
 static void set_roots(Launch *L, const Graph &g, int32_t lo, int32_t hi) {
     L->a.e_lo = L->ao.e_lo = g.off[lo];
     L->a.e_hi = L->ao.e_hi = g.off[hi];
+    L->tasks = g.off[hi] - g.off[lo];
     L->ca.root_lo = lo;
     L->ca.root_hi = hi;
-    L->tasks = g.off[hi] - g.off[lo];
+    if (!L->clique) return;
+    L->ca.chunk = clique_chunk(L->chunk, hi - lo, (long long)L->grid.x * (L->block.x / 64));
 }
 
 static void fill_defaults(gat_kernel_config *c) {
@@ -2121,28 +2592,34 @@ static void fill_defaults(gat_kernel_config *c) {
 }
 
 // Knobs and launch shapes of the clique store: the main launch (one wave
-// per vertex, rows in the wave's LDS slice) and workgroup tiers 0 and 1
-// (rows in LDS; t1_lds = 0 when the device cannot give tier 1 its LDS).
-static int clique_shape(const DeviceInfo &di, const gat_kernel_config &cfg, Launch *L) {
+// per vertex) and the workgroup tiers with rows in LDS. max_out: an upper
+// bound of the out-degrees; tiers beyond it are not launched.
+static int clique_shape(const DeviceInfo &di, const gat_kernel_config &cfg, int max_out, Launch *L) {
     gatk::CArgs &c = L->ca;
-    c.cap = std::max(32, std::min(32 * gatk::CMAXW, cfg.slot_capacity / 32 * 32));
-    c.chunk = cfg.queue_chunk;
+    c.cap = std::max(32, std::min(gatk::CMAXD, cfg.slot_capacity / 32 * 32));
+    L->chunk = cfg.queue_chunk;
     c.lin_thr = cfg.search_linear_threshold;
-    c.gallop_ratio = cfg.gallop_ratio;
     L->block = dim3(64 * cfg.block_waves);
     L->grid = dim3(std::max(1, std::max(1, cfg.waves_per_cu * di.cus) / cfg.block_waves));
-    L->clique_wave_bytes = (4 * (c.cap + 4) + 4 * c.cap * gatk::row_words(c.cap) + 15) / 16 * 16;
-    L->clique_lds = size_t(L->clique_wave_bytes) * cfg.block_waves;
-    if (L->clique_lds > di.lds_per_block)
-        GAT_FAIL(GAT_EINFEASIBLE, "bitmap config needs %zu B of LDS per workgroup", L->clique_lds);
-    L->mid_lds = (size_t)4 * (32 * gatk::CMIDW + 4) + (size_t)4 * 32 * gatk::CMIDW * gatk::row_words(32 * gatk::CMIDW) +
-                 (size_t)2 * gatk::index_slots(32 * gatk::CMIDW);
-    if (L->mid_lds > di.lds_per_block) GAT_FAIL(GAT_EINFEASIBLE, "device LDS too small for the clique block tier");
-    L->mid_grid = dim3(std::max(1, (int)(di.lds_per_cu / L->mid_lds)) * di.cus);
-    const size_t t1 = (size_t)4 * (32 * gatk::CBIGW + 4) + (size_t)4 * 32 * gatk::CBIGW * gatk::row_words(32 * gatk::CBIGW) +
-                      (size_t)2 * gatk::index_slots(32 * gatk::CBIGW);
-    L->t1_lds = t1 <= di.lds_per_block ? t1 : 0;
-    if (L->t1_lds) L->t1_grid = dim3(std::max(1, (int)(di.lds_per_cu / t1)) * di.cus);
+    L->clique_lds = sizeof(gatk::CWave) * cfg.block_waves;
+    const size_t lds[3] = {gatk::tier_lds(gatk::CT0W, gatk::CNW0), gatk::tier_lds(gatk::CT1W, gatk::CNW1),
+                           gatk::tier_lds(gatk::CT2W, gatk::CNW2)};
+    if (lds[1] + 64 > di.lds_per_block) GAT_FAIL(GAT_EINFEASIBLE, "device LDS too small for the clique block tiers");
+    // 64 B: the kernels' own static LDS
+    c.lds_dmax = lds[2] + 64 <= di.lds_per_block ? 32 * gatk::CT2W : 32 * gatk::CT1W;
+    const int waves[3] = {gatk::CNW0, gatk::CNW1, gatk::CNW2};
+    // #K6 leaves the main launch earlier: its walk on one wave grows with d^3
+    // (R-MAT s14: 1.75 ms with vertices up to 64 there, 0.60 ms up to 32; s16
+    // the same either way; #K3 to #K5 lose up to 10 % below 64)
+    c.main_max = std::min(c.kmax >= 6 ? gatk::CMAIN / 2 : gatk::CMAIN, c.cap);
+    const int above[4] = {c.main_max, 32 * gatk::CT0W, 32 * gatk::CT1W, c.lds_dmax};
+    for (int t = 0; t < 3; t++) {
+        L->tier_lds[t] = lds[t];
+        const int per_cu = std::max(1, std::min((int)(di.lds_per_cu / (lds[t] + 64)), 4 * gatk::clique_occupancy(t) / waves[t]));
+        L->tier_grid[t] = dim3(max_out > above[t] && above[t] < c.lds_dmax ? per_cu * di.cus : 0);
+    }
+    L->tier_grid[3] = dim3(max_out > above[3] ? 2 * di.cus : 0);
+    L->heavy = max_out > c.main_max;
     return GAT_OK;
 }
 
@@ -2167,7 +2644,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         HIPCHECK(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
         HIPCHECK(hipMalloc(&d->plan, sizeof(GatPlanDev)));
         HIPCHECK(hipMemcpy(d->plan, &pd, sizeof(GatPlanDev), hipMemcpyHostToDevice));
-        HIPCHECK(hipMalloc(&d->counts, sizeof(unsigned long long) * GATP_MAX_TERMS));
+        HIPCHECK(hipMalloc(&d->counts, sizeof(unsigned long long) * GATP_MAX_TERMS * gatk::kCountCopies));
         HIPCHECK(hipMalloc(&d->queue, sizeof(unsigned long long) * 16));
         HIPCHECK(hipMalloc(&d->ovf_n, sizeof(unsigned long long) * 16));
         HIPCHECK(hipMalloc(&d->bytes, sizeof(unsigned long long) * 4));
@@ -2201,15 +2678,10 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     if (split && !d->subs) HIPCHECK(hipMalloc(&d->subs, sizeof(gatk::SplitTask) * (kLevels + 3) * kSubCap));
     if (ovf_cap > d->ovf_cap) {
         if (d->ovf) HIPCHECK(hipFree(d->ovf));
-        for (auto &t : d->tier)
-            if (t) HIPCHECK(hipFree(t));
         d->ovf = nullptr;
-        for (auto &t : d->tier) t = nullptr;
         HIPCHECK(hipMalloc(&d->ovf, sizeof(long long) * ovf_cap));
         d->ovf_cap = ovf_cap;
     }
-    if (clique && !d->tier[0])
-        for (auto &t : d->tier) HIPCHECK(hipMalloc(&t, sizeof(long long) * (size_t)(g.n + 1) * gatk::CSPLIT_ENC));
     const int wave_bytes = int((sizeof(gatk::WaveState) + size_t(pd.n_store) * cfg.slot_capacity * 4 + 15) / 16 * 16);
     const size_t lds = size_t(wave_bytes) * cfg.block_waves;
     if (lds > di.lds_per_block)
@@ -2270,24 +2742,6 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     L->ovf_lds = L->ovf_wave_bytes;
     L->clique = clique;
     if (clique) {
-        gatk::CArgs c{};
-        c.off = a.off;
-        c.adj = a.adj;
-        c.split = a.split;
-        c.n = a.n;
-        c.m = a.m;
-        c.root_lo = 0;
-        c.root_hi = a.n;
-        c.counts = a.counts;
-        for (int k = 0; k < 8; k++) c.pat_of_k[k] = p->cp.clique_pattern[k];
-        c.kmax = 31 - __builtin_clz(p->cp.clique_ks);
-        c.queue = a.queue;
-        for (int t = 0; t < 3; t++) c.tier[t] = d->tier[t];
-        c.ovf_n = a.ovf_n;
-        c.ovf_cap = (long long)(g.n + 1) * gatk::CSPLIT_ENC;
-        c.bytes = a.bytes;
-        c.err = a.err;
-        // HBM tier: rows sized by the maximum out-degree
         if (g.max_out < 0) {
             int32_t mo = 0;
             for (int32_t v = 0; v < g.n; v++) {
@@ -2296,31 +2750,70 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
             }
             g.max_out = mo;
         }
-        const int hcap = std::max(32, g.max_out);
-        const int ws = gatk::row_words(hcap);
-        int waves = std::max(64, 8 * di.cus);
-        while (waves > 64 && (double)waves * hcap * ws * 4 > 16e9) waves /= 2;
-        if (d->big_cap < hcap || d->big_waves < waves) {
-            if (d->grows) HIPCHECK(hipFree(d->grows));
-            if (d->goff) HIPCHECK(hipFree(d->goff));
-            d->grows = nullptr;
-            d->goff = nullptr;
-            HIPCHECK(hipMalloc(&d->grows, (size_t)waves * hcap * ws * 4));
-            HIPCHECK(hipMalloc(&d->goff, (size_t)waves * (hcap + 1) * 4));
-            d->big_cap = hcap;
-            d->big_waves = waves;
-        }
-        c.grows = d->grows;
-        c.goff = d->goff;
-        c.hcap = d->big_cap;
-        L->ca = c;
-        rc = clique_shape(di, cfg, L);
+        rc = ensure_core(g, d->dg.get());
         if (rc) return rc;
-        L->big_grid = dim3(std::min(d->big_waves, 2 * di.cus));  // one scratch area per workgroup
-        if (!L->t1_lds) L->t1_grid = L->big_grid;
+        gatk::CArgs c{};
+        c.off = a.off;
+        c.adj = a.adj;
+        c.split = a.split;
+        c.core = d->dg->core;
+        c.core_n = d->dg->core_n;
+        c.n = a.n;
+        c.m = a.m;
+        c.root_lo = 0;
+        c.root_hi = a.n;
+        c.counts = a.counts;
+        for (int k = 0; k < 8; k++) c.pat_of_k[k] = p->cp.clique_pattern[k];
+        c.kmax = 31 - __builtin_clz(p->cp.clique_ks);
+        c.queue = a.queue;
+        c.ovf_n = a.ovf_n;
+        c.bytes = a.bytes;
+        c.err = a.err;
+        L->ca = c;
+        rc = clique_shape(di, cfg, g.max_out, L);
+        if (rc) return rc;
+        for (int t = 0; t < gatk::CTIERS; t++) {
+            if (L->tier_grid[t].x && !d->tier[t]) HIPCHECK(hipMalloc(&d->tier[t], sizeof(int) * ((size_t)g.n + 1)));
+            L->ca.tier[t] = d->tier[t];
+            L->ca.tier_cap[t] = d->tier[t] ? g.n + 1ll : 0;
+        }
+        if (L->tier_grid[3].x) {
+            // HBM tier: one scratch area per workgroup, sized by the maximum out-degree
+            const int hcap = std::max(32, g.max_out), ws = gatk::row_words(hcap);
+            int groups = (int)L->tier_grid[3].x;
+            while (groups > 64 && (double)groups * hcap * ws * 4 > 16e9) groups /= 2;
+            if (d->big_cap < hcap || d->big_groups < groups) {
+                if (d->grows) HIPCHECK(hipFree(d->grows));
+                if (d->goff) HIPCHECK(hipFree(d->goff));
+                d->grows = nullptr;
+                d->goff = nullptr;
+                HIPCHECK(hipMalloc(&d->grows, (size_t)groups * hcap * ws * 4));
+                HIPCHECK(hipMalloc(&d->goff, (size_t)groups * (hcap + 1) * 4));
+                d->big_cap = hcap;
+                d->big_groups = groups;
+            }
+            L->tier_grid[3] = dim3(std::min(groups, d->big_groups));
+            L->ca.grows = d->grows;
+            L->ca.goff = d->goff;
+            L->ca.hcap = d->big_cap;
+        }
     }
     set_roots(L, g, 0, g.n);
     return GAT_OK;
+}
+
+static unsigned classify_grid(const gatk::CArgs &c) {
+    const long long n = (long long)c.root_hi - c.root_lo;
+    return (unsigned)std::max(1ll, std::min(64ll, n / (4 * gatk::kClassifyThreads)));
+}
+
+// Launch of a workgroup tier with rows in LDS.
+template <int MODE, int MW, int TIER, int NW, class F>
+static void launch_tier(const Launch &L, gatk::CArgs &c, hipStream_t s, F &&tl_take) {
+    if (!L.tier_grid[TIER].x) return;
+    c.tl_base = tl_take((int)L.tier_grid[TIER].x);
+    hipLaunchKernelGGL((gatk::clique_block_kernel<MW, TIER, NW, MODE>), L.tier_grid[TIER], dim3(64 * NW),
+                       L.tier_lds[TIER], s, c);
 }
 
 // Enqueue the whole count on the plan's stream (capturable: no memsets).
@@ -2337,7 +2830,8 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
     };
     if (timeline) {
         const int waves = (int)(L.grid.x * (L.block.x / 64));
-        const long long need = L.clique ? (long long)waves + L.mid_grid.x + L.t1_grid.x + L.big_grid.x
+        const long long need = L.clique ? (long long)waves + L.tier_grid[0].x + L.tier_grid[1].x + L.tier_grid[2].x +
+                                              L.tier_grid[3].x
                                         : (long long)waves * (1 + (L.a.split_ticks > 0 ? kLevels : 0)) +
                                               (long long)L.ovf_grid.x * (L.a.split_ticks > 0 ? 2 : 1);
         if (need > kTlCap) GAT_FAIL(GAT_ELIMIT, "timeline needs %lld records (> %d)", need, kTlCap);
@@ -2346,7 +2840,8 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
                            (long long)gatk::kTlFields * kTlCap, ~0ull);
         tl = d->tl;
     }
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->counts, (long long)GATP_MAX_TERMS, 0ull);
+    hipLaunchKernelGGL(gatk::fill_u64, dim3(4), dim3(256), 0, s, d->counts,
+                       (long long)GATP_MAX_TERMS * gatk::kCountCopies, 0ull);
     hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->queue, 16ll, 0ull);
     hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->ovf_n, 16ll, 0ull);
     hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->bytes, 4ll, 0ull);
@@ -2365,25 +2860,21 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
         // instantiations (MODE bits 0 and 1)
         auto run = [&](auto mode_tag) -> int {
             constexpr int T = decltype(mode_tag)::value;
+            if (L.heavy)
+                hipLaunchKernelGGL(gatk::clique_classify, dim3(classify_grid(c)), dim3(gatk::kClassifyThreads), 0, s, c);
             c.tl_base = tl_take(waves);
-            hipLaunchKernelGGL(gatk::clique_kernel<T>, L.grid, L.block, L.clique_lds, s, c, L.clique_wave_bytes);
+            hipLaunchKernelGGL(gatk::clique_kernel<T>, L.grid, L.block, L.clique_lds, s, c);
             if (events) HIPCHECK(hipEventRecord(d->ev[1], s));
-            c.bytes = d->bytes + 1;  // workgroup tier 0: its own W_alg counter
-            c.tl_base = tl_take((int)L.mid_grid.x);
-            hipLaunchKernelGGL((gatk::clique_block_kernel<gatk::CMIDW, true, 0, gatk::CBLOCKW0, T>), L.mid_grid,
-                               dim3(64 * gatk::CBLOCKW0), L.mid_lds, s, c);
+            c.bytes = d->bytes + 1;  // tiers 0 and 1: their own W_alg counter
+            launch_tier<T, gatk::CT0W, 0, gatk::CNW0>(L, c, s, tl_take);
+            launch_tier<T, gatk::CT1W, 1, gatk::CNW1>(L, c, s, tl_take);
             if (events) HIPCHECK(hipEventRecord(d->ev[3], s));
-            c.bytes = d->bytes + 2;  // tiers 1 and 2
-            c.tl_base = tl_take((int)L.t1_grid.x);
-            if (L.t1_lds)
-                hipLaunchKernelGGL((gatk::clique_block_kernel<gatk::CBIGW, true, 1, gatk::CBLOCKW1, T>), L.t1_grid,
-                                   dim3(64 * gatk::CBLOCKW1), L.t1_lds, s, c);
-            else
-                hipLaunchKernelGGL((gatk::clique_block_kernel<gatk::CBIGW, false, 1, gatk::CBLOCKW1, T>), L.t1_grid,
-                                   dim3(64 * gatk::CBLOCKW1), 0, s, c);
-            c.tl_base = tl_take((int)L.big_grid.x);
-            hipLaunchKernelGGL((gatk::clique_block_kernel<0, false, 2, gatk::CBLOCKW1, T>), L.big_grid,
-                               dim3(64 * gatk::CBLOCKW1), 0, s, c);
+            c.bytes = d->bytes + 2;  // tiers 2 and 3
+            launch_tier<T, gatk::CT2W, 2, gatk::CNW2>(L, c, s, tl_take);
+            if (L.tier_grid[3].x) {
+                c.tl_base = tl_take((int)L.tier_grid[3].x);
+                hipLaunchKernelGGL(gatk::clique_hbm_kernel<T>, L.tier_grid[3], dim3(64 * gatk::CNW3), 0, s, c);
+            }
             return GAT_OK;
         };
         const int mode = (account ? 1 : 0) | (timeline ? 2 : 0);
@@ -2444,13 +2935,16 @@ static int finish(gat_plan *p, const Launch &L, uint64_t *counts_out, gat_count_
                   bool raw_sums = false) {
     PlanDevice *d = p->dev;
     const int np = p->cp.dev.n_patterns;
-    unsigned long long raw[GATP_MAX_TERMS], ovf[16] = {}, bytes[3] = {0, 0, 0};
+    unsigned long long raw[GATP_MAX_TERMS] = {}, ovf[16] = {}, bytes[3] = {0, 0, 0};
+    unsigned long long copies[gatk::kCountCopies * GATP_MAX_TERMS];
     unsigned int err = 0;
-    HIPCHECK(hipMemcpyAsync(raw, d->counts, sizeof(unsigned long long) * np, hipMemcpyDeviceToHost, d->stream));
+    HIPCHECK(hipMemcpyAsync(copies, d->counts, sizeof(copies), hipMemcpyDeviceToHost, d->stream));
     HIPCHECK(hipMemcpyAsync(ovf, d->ovf_n, sizeof(ovf), hipMemcpyDeviceToHost, d->stream));
     HIPCHECK(hipMemcpyAsync(bytes, d->bytes, sizeof(bytes), hipMemcpyDeviceToHost, d->stream));
     HIPCHECK(hipMemcpyAsync(&err, d->err, sizeof(err), hipMemcpyDeviceToHost, d->stream));
     HIPCHECK(hipStreamSynchronize(d->stream));
+    for (int c = 0; c < gatk::kCountCopies; c++)
+        for (int i = 0; i < np; i++) raw[i] += copies[c * GATP_MAX_TERMS + i];
     // flags 2 and 4: a device work list (overflow tasks, subtasks, clique
     // tiers) filled up; 1 and 8: states the host's sizing rules out
     if (err & 6u) GAT_FAIL(GAT_ELIMIT, "a device work list overflowed (engine flags 0x%x)", err);
@@ -2475,7 +2969,7 @@ static int finish(gat_plan *p, const Launch &L, uint64_t *counts_out, gat_count_
             st->main_kernel_ms = ms_main;
             st->second_kernel_ms = ms_second;
         }
-        st->overflow_tasks = L.clique ? ovf[3] : ovf[0];
+        st->overflow_tasks = L.clique ? ovf[4] : ovf[0];
         unsigned long long made = 0;
         for (int k = 1; k <= kLevels; k++) made += std::min<unsigned long long>(ovf[8 + k], (unsigned long long)kSubCap);
         made += std::min<unsigned long long>(ovf[8 + kLevels + 1], (unsigned long long)(3 * kSubCap));
@@ -2586,14 +3080,18 @@ extern "C" int gat_count_shard_edges(gat_plan *p, const gat_kernel_config *cfg, 
 
 // ---- allocation-free clique count ---------------------------------------
 // Scratch of gat_count_cliques_noalloc, one copy per device for the life of
-// the process: kNaHead words of counters (counts [0,8), queues [8,24),
-// work-list sizes [24,40), W_alg [40,44), error flags at word 44), then the
-// split[] array (int32, kNaMaxV entries), then the lists of workgroup tiers 0
-// and 1 (int64, kNaTierCap entries each): 32 MiB and 512 B in all.
+// the process: kNaHead words of counters (queues [8,24), work-list sizes
+// [24,40), W_alg [40,44), error flags at word 44, the copies of the counts
+// from word 64 on), then
+// kNaBody int32 entries laid out for the graph's size: the split[] array (n),
+// the lists of workgroup tiers 0 (n), 1 (kNaTierCap) and 2 (kNaTierCap / 2),
+// and the core bitmap in the rest (28 to 58 MiB, so 21,000 to 31,000 core
+// vertices). 64 MiB and 17 KiB in all.
 constexpr int kNaMaxV = 1 << 22;
 constexpr long long kNaTierCap = 1 << 20;
-constexpr long long kNaHead = 64;
-constexpr long long kNaWords = kNaHead + kNaMaxV / 2 + 2 * kNaTierCap;
+constexpr long long kNaHead = 64 + GATP_MAX_TERMS * gatk::kCountCopies;
+constexpr long long kNaBody = 1 << 24;
+constexpr long long kNaWords = kNaHead + kNaBody / 2;
 static __device__ __align__(256) unsigned long long scratch[kNaWords];
 
 // Device address of this device's scratch, looked up once per device (the
@@ -2631,11 +3129,13 @@ extern "C" int gat_count_cliques_noalloc(const int64_t *d_offsets, const int32_t
     fill_defaults(&cfg);
     if (cfg.block_waves > 4) GAT_FAIL(GAT_EINFEASIBLE, "block_waves %d > 4", cfg.block_waves);
     Launch L;
-    rc = clique_shape(di, cfg, &L);
+    L.ca = {};
+    L.ca.kmax = kmax;
+    rc = clique_shape(di, cfg, 32 * gatk::CT2W, &L);  // the out-degrees are not known here: every LDS tier runs
     if (rc) return rc;
-    if (!L.t1_lds)
+    if (L.ca.lds_dmax < 32 * gatk::CT2W)
         GAT_FAIL(GAT_EINFEASIBLE, "the allocation-free count needs %d KiB of LDS per workgroup",
-                 (int)((4 * (32 * gatk::CBIGW + 4) + 4 * 32 * gatk::CBIGW * gatk::row_words(32 * gatk::CBIGW)) / 1024));
+                 (int)((gatk::tier_lds(gatk::CT2W, gatk::CNW2) + 1023) / 1024));
     unsigned long long *h = nullptr;
     rc = noalloc_scratch(&h);
     if (rc) return rc;
@@ -2644,49 +3144,64 @@ extern "C" int gat_count_cliques_noalloc(const int64_t *d_offsets, const int32_t
     c.adj = d_adj;
     int *split = reinterpret_cast<int *>(h + kNaHead);
     c.split = split;
+    c.tier[0] = split + v_cnt;
+    c.tier[1] = c.tier[0] + v_cnt;
+    c.tier[2] = c.tier[1] + kNaTierCap;
+    c.tier[3] = nullptr;
+    c.tier_cap[0] = v_cnt;
+    c.tier_cap[1] = kNaTierCap;
+    c.tier_cap[2] = kNaTierCap / 2;
+    c.tier_cap[3] = 0;
+    unsigned *core = reinterpret_cast<unsigned *>(c.tier[2] + c.tier_cap[2]);
+    const long long used = reinterpret_cast<int *>(core) - split;
+    c.core = core;
+    c.core_n = core_vertices(v_cnt, kNaBody - used);
     c.n = v_cnt;
     c.m = 0;
     c.root_lo = 0;
     c.root_hi = v_cnt;
-    c.counts = h;
+    c.chunk = clique_chunk(L.chunk, v_cnt, (long long)L.grid.x * (L.block.x / 64));
+    c.counts = h + 64;
     for (int k = 0; k < 8; k++) c.pat_of_k[k] = (k >= 3 && k <= kmax) ? k - 3 : -1;
-    c.kmax = kmax;
     c.queue = h + 8;
-    c.tier[0] = reinterpret_cast<long long *>(h + kNaHead + kNaMaxV / 2);
-    c.tier[1] = c.tier[0] + kNaTierCap;
-    c.tier[2] = nullptr;
     c.ovf_n = h + 24;
-    c.ovf_cap = kNaTierCap;
     c.bytes = h + 40;
     c.err = reinterpret_cast<unsigned *>(h + 44);
-    c.grows = nullptr;  // no HBM tier: vertices with more than 32 * CBIGW neighbours below them are refused
+    c.grows = nullptr;  // no HBM tier: vertices with more than lds_dmax neighbours below them are refused
     c.goff = nullptr;
-    c.hcap = 32 * gatk::CBIGW;
+    c.hcap = c.lds_dmax;
     c.account = 0;
     c.tl = nullptr;
     c.tl_base = 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, h, kNaHead, 0ull);
+    hipLaunchKernelGGL(gatk::fill_u64, dim3(4), dim3(256), 0, s, h, kNaHead, 0ull);
     if (v_cnt > 0) {
         hipLaunchKernelGGL(gatk::split_kernel, dim3(1024), dim3(256), 0, s, reinterpret_cast<const long long *>(d_offsets),
                            d_adj, v_cnt, split);
-        hipLaunchKernelGGL(gatk::clique_kernel<0>, L.grid, L.block, L.clique_lds, s, c, L.clique_wave_bytes);
-        hipLaunchKernelGGL((gatk::clique_block_kernel<gatk::CMIDW, true, 0, gatk::CBLOCKW0, 0>), L.mid_grid,
-                           dim3(64 * gatk::CBLOCKW0), L.mid_lds, s, c);
-        hipLaunchKernelGGL((gatk::clique_block_kernel<gatk::CBIGW, true, 1, gatk::CBLOCKW1, 0>), L.t1_grid,
-                           dim3(64 * gatk::CBLOCKW1), L.t1_lds, s, c);
+        if (c.core_n > 0)
+            hipLaunchKernelGGL(gatk::core_rows_kernel, dim3(std::min((c.core_n + 3) / 4, 4096)), dim3(256), 0, s,
+                               reinterpret_cast<const long long *>(d_offsets), d_adj, split, c.core_n, core);
+        hipLaunchKernelGGL(gatk::clique_classify, dim3(classify_grid(c)), dim3(gatk::kClassifyThreads), 0, s, c);
+        hipLaunchKernelGGL(gatk::clique_kernel<0>, L.grid, L.block, L.clique_lds, s, c);
+        auto no_tl = [](int) { return 0; };
+        launch_tier<0, gatk::CT0W, 0, gatk::CNW0>(L, c, s, no_tl);
+        launch_tier<0, gatk::CT1W, 1, gatk::CNW1>(L, c, s, no_tl);
+        launch_tier<0, gatk::CT2W, 2, gatk::CNW2>(L, c, s, no_tl);
     }
     HIPCHECK(hipGetLastError());
-    unsigned long long raw[8] = {};
+    unsigned long long copies[gatk::kCountCopies * GATP_MAX_TERMS], raw[8] = {}, heavy = 0;
     unsigned int err = 0;
-    HIPCHECK(hipMemcpyAsync(raw, h, sizeof(raw), hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipMemcpyAsync(copies, c.counts, sizeof(copies), hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipMemcpyAsync(&heavy, h + 24 + 5, sizeof(heavy), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipMemcpyAsync(&err, h + 44, sizeof(err), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     if (err & 16u)
         GAT_FAIL(GAT_ELIMIT, "a vertex has more than %d neighbours below it; the allocation-free count has no HBM tier",
-                 32 * gatk::CBIGW);
-    if (err & 4u) GAT_FAIL(GAT_ELIMIT, "more than %lld heavy vertices for one workgroup tier", kNaTierCap);
+                 c.lds_dmax);
+    if ((err & 4u) || heavy > (unsigned long long)kNaTierCap) GAT_FAIL(GAT_ELIMIT, "more than %lld heavy vertices for one workgroup tier", kNaTierCap);
     if (err) GAT_FAIL(GAT_EINTERNAL, "engine reported an internal inconsistency (flags 0x%x)", err);
+    for (int i = 0; i < gatk::kCountCopies; i++)
+        for (int k = 0; k < 8; k++) raw[k] += copies[i * GATP_MAX_TERMS + k];
     for (int k = 3; k <= kmax; k++) counts_out[k - 3] = raw[k - 3];
     return GAT_OK;
 }

@@ -121,7 +121,10 @@ typedef struct gat_kernel_config {
     int32_t waves_per_cu;     /* persistent grid = waves_per_cu * CUs (0: 16
                                  for the array store, 8 for the clique store) */
     int32_t queue_chunk;      /* directed edges taken per work-queue grab      */
-    int32_t slot_capacity;    /* int32 entries per LDS prefix-set slot         */
+    int32_t slot_capacity;    /* int32 entries per LDS prefix-set slot; clique
+                                 store: vertices with more neighbours below
+                                 them (at most 256 counts) always leave the
+                                 main launch                                   */
     int32_t leaf_mode;        /* 0 flattened, else lanes per candidate 1..64
                                  (threads_per_warp, engine_config.hpp:6)      */
     int32_t intersect_strategy; /* how one wave intersects two sorted lists:
@@ -168,10 +171,11 @@ typedef struct gat_count_stats {
     double main_kernel_ms;    /* duration of the main engine launch          */
     double second_kernel_ms;  /* array store: the split and HBM overflow
                                  launches after the main one; bitmap store:
-                                 workgroup tier 0                             */
+                                 workgroup tiers 0 and 1                      */
     uint64_t overflow_tasks;  /* array store: tasks re-run with HBM-resident
-                                 prefix sets; bitmap store: vertices passed to
-                                 the workgroup tiers                          */
+                                 prefix sets; bitmap store: vertices with more
+                                 than slot_capacity (at most 256) neighbours
+                                 below them                                   */
     uint64_t alg_bytes;       /* W_alg of the whole count (GAT_FLAG_ACCOUNT)  */
     uint64_t alg_bytes_main;  /* W_alg of the main launch alone              */
     uint64_t alg_bytes_second;/* W_alg of the launches second_kernel_ms times  */
@@ -341,8 +345,8 @@ void gat_plan_free(gat_plan *p);
  * runs the kernels of gat_count's bitmap clique store (the vertex of each
  * clique with the highest id is its root; ids in degree-descending order
  * keep the per-vertex lists short) and calls no allocating routine: its
- * counters, per-vertex split array and workgroup-tier lists sit in a static
- * 32 MiB device array, one per GPU, held until the process ends.
+ * counters, per-vertex split array, workgroup-tier lists and core bitmap sit
+ * in a static 64 MiB device array, one per GPU, held until the process ends.
  *   d_offsets[v_cnt+1], d_adj: device CSR, rows sorted, symmetric, no
  *   self-loops or duplicates, ids in [0, v_cnt).
  *   stream: a hipStream_t (NULL = the null stream); the call enqueues on it
@@ -358,7 +362,7 @@ int gat_count_cliques_noalloc(const int64_t *d_offsets, const int32_t *d_adj, in
                               uint64_t *counts_out);
 
 /* Records of the last gat_count run with GAT_FLAG_TIMELINE on this plan, 8
- * int64 each: launch (clique store: 0 main, 1-3 workgroup tiers; array
+ * int64 each: launch (clique store: 0 main, 1-4 workgroup tiers; array
  * store: 0 main, 1-3 subtask levels, 4 HBM launch, 5 its subtasks), unit
  * (wave of the launch, or workgroup of a clique tier), start and end in
  * wall-clock ticks from the count's first start, shader cycles spent
