@@ -92,6 +92,22 @@ struct KArgs {
     long long in_base, out_base, sovf_base;
     long long in_cap, out_cap, sovf_cap;
     long long split_ticks;  // <= 0: no splitting
+    // Kept COUNT values (GATP_KEEP_*), null without. A leaf's |N(c) ∩ father|
+    // is the same for every path that ends in c while the father stays, and
+    // there are many (R-MAT s13's C5: 1.3e9 paths over 6.7e7 pairs of vertices).
+    // edge_tab[k][e] is the value of directed edge e with truncation k, or -1.
+    // Pool i holds tables of tab_size entries from pool + i pool_tables
+    // tab_size on; key x uses table x % pool_tables, whose entry c is {x + 1,
+    // value | epoch << 24} for the key that wrote it last. Every count has its
+    // own epoch, so nothing of an earlier one is taken. One pool for all waves:
+    // with a table per wave the subtasks of one root each filled their own
+    // (C5 108 ms, now 56; house on Chung-Lu 65,536 46 ms, now 36).
+    int *edge_tab[4];
+    uint2 *pool;
+    unsigned pool_tables;
+    int tab_size;
+    unsigned epoch;
+    int keep;  // this count uses the tables
     // Timeline (GAT_FLAG_TIMELINE): one record of kTlFields int64 per wave
     // at tl + kTlFields * (tl_base + wave), or none when tl is null.
     long long *tl;
@@ -142,6 +158,7 @@ struct WaveState {
     int base_depth;             // frames exist from this depth on (2, or a subtask's depth)
     int path_pos[GATP_MAX_DEPTH + 1];  // a subtask's positions at depths 2 .. base_depth-1
     int abort;
+    int ex_in[GATP_MAX_LEAF_OPS];                  // leaf: excluded levels whose vertex lies in the op's father
 };
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
@@ -796,16 +813,144 @@ __device__ __forceinline__ bool visit(const Ctx &C, const GatNode &N, int d, int
     return true;
 }
 
+// |N(c) ∩ father ∩ [0,t)| without the nex values ex, for the lanes in `need`
+// (0 in the others): the (candidate, element) pairs of the wave's lanes form one
+// flattened index space. alen: the length of N(c) below t; *blen_out: that of
+// the father.
+template <bool GS>
+__device__ __forceinline__ int sweep_count(const Ctx &C, const GatOp &o, bool need, int c, long long ab, int alen, int t,
+                                           const int *ex, int nex, int *blen_out) {
+    const KArgs &a = C.a;
+    WaveState *S = C.S;
+    const int ln = C.ln;
+    int cnt = 0;
+    const int f = o.father;
+    int blen = 0;
+    // Bg: father in HBM (a neighbour list, or any set in the overflow
+    // launch); Bl: father in this wave's LDS buffers. hub_b: the
+    // father is a hub's neighbour list in HBM, probed by bitmap.
+    const int *Bg = a.adj;
+    const int *Bl = C.store;
+    int hub_b = -1, lim_b = 0;
+    const GatSlot &fs = C.P.slots[f];
+    const bool b_lds = in_lds<GS>(C, f);
+    if (b_lds) Bl = C.store + (long long)fs.store * a.cap;
+    else if (fs.kind == GATP_ALIAS) Bg = a.adj + S->sbeg[f];
+    else if constexpr (GS) Bg = C.store + (long long)fs.store * a.cap;
+    const int flen = S->slen[f];
+    if (need) blen = t == INT_MAX ? flen : (b_lds ? lbound(Bl, flen, t) : lbound(Bg, flen, t));
+    if (!b_lds && fs.kind == GATP_ALIAS) hub_b = uni(hub_of(a, S->val[fs.depth]));
+    // candidate lists with a hub bitmap are probed through it
+    const int hub_a = need ? hub_of(a, c) : -1;
+    const int lim_a = hub_a >= 0 ? list_lim(a, ab, alen) : 0;
+    if (hub_b >= 0 && need) lim_b = blen > 0 ? Bg[blen - 1] : -1;
+    const bool sa = stream_a(a, alen, blen, b_lds || hub_b >= 0, hub_a >= 0);
+    const int mylen = sa ? alen : blen;
+    int T = 0;
+    const int myoff = excl_scan(mylen, &T);
+    for (int k0 = 0; k0 < T; k0 += W) {
+        const int j = k0 + ln;
+        bool hit = false;
+        by_owner(myoff, k0, T, [&](const auto &pull) {
+            const int s_off = pull(myoff);
+            const int s_sa = pull((int)sa);
+            const long long s_ab = pull(ab);
+            const int s_alen = pull(alen);
+            const int s_blen = pull(blen);
+            const int s_hub = pull(hub_a);
+            const int s_lim = pull(lim_a);
+            const int s_limb = pull(lim_b);
+            if (j < T) {
+                const int idx = j - s_off;
+                int x;
+                if (s_sa) {
+                    x = a.adj[s_ab + idx];
+                    if (b_lds) hit = has(Bl, s_blen, x, a.lin_thr);
+                    else if (hub_b >= 0) hit = hub_has(a, hub_b, x, s_limb);
+                    else hit = has(Bg, s_blen, x, a.lin_thr);
+                } else {
+                    x = b_lds ? Bl[idx] : Bg[idx];
+                    hit = s_hub >= 0 ? hub_has(a, s_hub, x, s_lim) : has(a.adj + s_ab, s_alen, x, a.lin_thr);
+                }
+                for (int q = 0; q < nex; q++) hit &= (x != ex[q]);
+            }
+        });
+        const unsigned long long m = ballot(hit);
+        const int lo = max(myoff - k0, 0), hi2 = min(myoff + mylen - k0, W);
+        if (lo < hi2) cnt += __popcll(m & range_mask(lo, hi2));
+    }
+    *blen_out = blen;
+    return cnt;
+}
+// The same from the candidate alone, out of line (rare calls).
+template <bool GS>
+__device__ __noinline__ int sweep_kept(const Ctx C, int op, bool need, int c, int t) {
+    const long long ab = need ? C.a.off[c] : 0;
+    const int alen = need ? trunc_len(C.a, c, ab, (int)(C.a.off[c + 1] - ab), t) : 0;
+    int blen;
+    return sweep_count<GS>(C, C.P.ops[op], need, c, ab, alen, t, nullptr, 0, &blen);
+}
+
+// The table of a KEEP_POOL op for the chosen v_0, v_1 or root edge, and the tag
+// of its entries.
+__device__ __forceinline__ uint2 *pool_table(const Ctx &C, const GatOp &o, unsigned *tag) {
+    const KArgs &a = C.a;
+    const WaveState *S = C.S;
+    unsigned key;
+    if (o.key == 3) key = (unsigned)uni((int)(S->sub_edge >= 0 ? S->sub_edge : S->rb + (S->f_cur[1] - 1)));
+    else key = (unsigned)uni(S->val[o.key == 2 ? 1 : 0]);
+    *tag = key + 1;
+    return a.pool + ((long long)o.table * a.pool_tables + key % a.pool_tables) * a.tab_size;
+}
+
+// Is x adjacent to y? x is the same in every lane.
+__device__ __forceinline__ bool adjacent(const KArgs &a, int x, int y) {
+    const int hx = uni(hub_of(a, x));
+    if (hx >= 0) return hub_has(a, hx, y, INT_MAX);
+    const int hy = hub_of(a, y);
+    if (hy >= 0) return hub_has(a, hy, x, INT_MAX);
+    const long long b = a.off[x];
+    return has(a.adj + b, (int)(a.off[x + 1] - b), y, a.lin_thr);
+}
+
+// Excluded levels below `upto` of a kept COUNT whose chosen vertex lies in the op's father
+// set before truncation (repeated vertices once): what plan compilation does
+// not know is looked up here, once per leaf frame.
+__device__ __forceinline__ void leaf_exclusions(const Ctx &C, const GatNode &N, int upto) {
+    const KArgs &a = C.a;
+    WaveState *S = C.S;
+    for (int k = 0; k < N.op_count; k++) {
+        const GatOp &o = C.P.ops[N.op_begin + k];
+        if (o.kind != GATP_COUNT || o.keep == GATP_KEEP_NONE) continue;
+        int in = 0;
+        for (int f = 0; f < upto; f++) {
+            if (!(o.excl >> f & 1u)) continue;
+            const int x = uni(S->val[f]);
+            bool yes = true;
+            for (int g = 0; g < f; g++) yes &= !((o.excl >> g & 1u) && S->val[g] == x);
+            if (yes && !(o.ex_father >> f & 1u)) {
+                // the father's set is the intersection of N(v_l) over its levels
+                for (int l = 0; l < GATP_MAX_DEPTH && yes; l++)
+                    if (o.levels >> l & 1u) yes = adjacent(a, x, uni(S->val[l]));
+            }
+            if (uni((int)yes)) in |= 1 << f;
+        }
+        if (C.ln == 0) S->ex_in[o.leaf_idx] = in;
+    }
+    wsync();
+}
+
 // All candidates of a leaf frame, flattened across lanes.
 // With can_split, a wave that is due to split (want_split) hands the
 // batches after the current one to the next split launch.
-template <bool GS>
+template <bool GS, bool KEEP>
 __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int cur, int hi, bool can_split = false,
                                      int node = -1) {
     const KArgs &a = C.a;
     WaveState *S = C.S;
     const int ln = C.ln;
     unsigned long long bytes = 0;
+    if (KEEP) leaf_exclusions(C, N, d);
     for (int cb = cur; cb < hi; cb += W) {
         const int ci = cb + ln;
         int c = 0;
@@ -819,7 +964,7 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
         // after the first go, in about as many parts as the chunk holds
         // budgets of work (at most 64), so that whole waves sweep their lists
         // in parallel; the wave keeps the first candidate.
-        if (can_split && hi - cb > 1 && queue_drained<GS>(a)) {
+        if (can_split && !(KEEP && N.kept) && hi - cb > 1 && queue_drained<GS>(a)) {
             const long long lw = ci < hi ? a.off[c + 1] - a.off[c] : 0;
             const long long tot = uni64((long long)wave_sum64((unsigned long long)lw));
             if (3 * tot > a.split_ticks && !split_shallowest<GS>(C, d - 1)) {
@@ -832,12 +977,39 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
         const bool valid = ci < hi;
         bool pass = valid && !equals_any(S, N.excl, d, c);
         const bool dup = pass && N.ap_levels && equals_any(S, N.ap_levels, d, c);
-        const long long ab = valid ? a.off[c] : 0;
-        const int deg = valid ? (int)(a.off[c + 1] - ab) : 0;
+        long long ab = 0;
+        int deg = -1;  // read when an op needs it
         for (int k = 0; k < N.op_count; k++) {
             const GatOp &o = C.P.ops[N.op_begin + k];
             const int t = group_bound(S, o.groups, o.ngroups, d, c);
-            int alen = (pass && !dup) ? trunc_len(a, c, ab, deg, t) : 0;
+            // kept values first: the lanes in `need` compute theirs
+            const bool live = pass && !dup;
+            bool need = live;
+            int kept = 0;
+            int *edge = nullptr;
+            uint2 *slot = nullptr;
+            unsigned tag = 0;
+            if (KEEP && o.keep == GATP_KEEP_EDGE) edge = a.edge_tab[o.table];
+            if (KEEP && edge) {
+                edge += S->sbeg[N.loop_slot] + ci;
+                if (live) kept = *edge;
+                need = live && kept < 0;
+            } else if (KEEP && o.keep == GATP_KEEP_POOL) {
+                slot = pool_table(C, o, &tag) + c;
+                if (live && c < a.tab_size) {
+                    const uint2 e = *slot;
+                    kept = (int)(e.y & 0xffffffu);
+                    need = e.x != tag || e.y >> 24 != a.epoch;
+                }
+            }
+            const bool by_table = KEEP && (edge || slot);
+            int cnt = 0;
+            if (!by_table || ballot(need)) {
+            if (uni(deg) < 0) {
+                ab = valid ? a.off[c] : 0;
+                deg = valid ? (int)(a.off[c + 1] - ab) : 0;
+            }
+            int alen = need ? trunc_len(a, c, ab, deg, t) : 0;
             if (o.kind == GATP_ALIAS) {
                 S->leafcnt[o.leaf_idx][ln] = alen;
                 continue;
@@ -845,80 +1017,32 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
             // COUNT: |N(c) ∩ father ∩ [0,t)| minus excluded chosen vertices
             int ex[8];
             int nex = 0;
-            for (int f = 0; f < d; f++)
+            for (int f = 0; f < d && !by_table; f++)  // a kept value leaves them in
                 if (o.excl >> f & 1u) ex[nex++] = S->val[f];
             if (o.father < 0) {
                 // |N(c) ∩ [0,t)| minus the excluded chosen vertices it holds
-                const bool live = pass && !dup;
                 S->leafcnt[o.leaf_idx][ln] = live ? alen - excluded_in_list(a, c, ab, alen, ex, nex) : 0;
                 if (a.account && live) bytes += 4ull * alen + 16ull;
                 continue;
             }
-            const int f = o.father;
-            const bool has_r = f >= 0;
-            bool b_lds = false;
             int blen = 0;
-            // Bg: father in HBM (a neighbour list, or any set in the overflow
-            // launch); Bl: father in this wave's LDS buffers. hub_b: the
-            // father is a hub's neighbour list in HBM, probed by bitmap.
-            const int *Bg = a.adj;
-            const int *Bl = C.store;
-            int hub_b = -1, lim_b = 0;
-            if (has_r) {
-                const GatSlot &fs = C.P.slots[f];
-                b_lds = in_lds<GS>(C, f);
-                if (b_lds) Bl = C.store + (long long)fs.store * a.cap;
-                else if (fs.kind == GATP_ALIAS) Bg = a.adj + S->sbeg[f];
-                else if constexpr (GS) Bg = C.store + (long long)fs.store * a.cap;
-                const int flen = S->slen[f];
-                if (pass && !dup) blen = t == INT_MAX ? flen : (b_lds ? lbound(Bl, flen, t) : lbound(Bg, flen, t));
-                if (!b_lds && fs.kind == GATP_ALIAS) hub_b = uni(hub_of(a, S->val[fs.depth]));
+            cnt = sweep_count<GS>(C, o, need, c, ab, alen, t, ex, nex, &blen);
+            if (a.account && live)
+                bytes += 4ull * (alen + blen) + 16ull + (C.P.slots[o.father].kind == GATP_ALIAS ? 16ull : 0ull);
+            if (need && edge) *edge = cnt;
+            if (need && slot && c < a.tab_size) *slot = make_uint2(tag, (unsigned)cnt | a.epoch << 24);
             }
-            // candidate lists with a hub bitmap are probed through it
-            const int hub_a = (has_r && valid) ? hub_of(a, c) : -1;
-            const int lim_a = hub_a >= 0 ? list_lim(a, ab, alen) : 0;
-            if (hub_b >= 0 && pass && !dup) lim_b = blen > 0 ? Bg[blen - 1] : -1;
-            const bool sa = !has_r || stream_a(a, alen, blen, b_lds || hub_b >= 0, hub_a >= 0);
-            const int mylen = sa ? alen : blen;
-            int T = 0;
-            const int myoff = excl_scan(mylen, &T);
-            int cnt = 0;
-            for (int k0 = 0; k0 < T; k0 += W) {
-                const int j = k0 + ln;
-                bool hit = false;
-                by_owner(myoff, k0, T, [&](const auto &pull) {
-                    const int s_off = pull(myoff);
-                    const int s_sa = pull((int)sa);
-                    const long long s_ab = pull(ab);
-                    const int s_alen = pull(alen);
-                    const int s_blen = pull(blen);
-                    const int s_hub = pull(hub_a);
-                    const int s_lim = pull(lim_a);
-                    const int s_limb = pull(lim_b);
-                    if (j < T) {
-                        const int idx = j - s_off;
-                        int x;
-                        if (s_sa) {
-                            x = a.adj[s_ab + idx];
-                            if (!has_r) hit = true;
-                            else if (b_lds) hit = has(Bl, s_blen, x, a.lin_thr);
-                            else if (hub_b >= 0) hit = hub_has(a, hub_b, x, s_limb);
-                            else hit = has(Bg, s_blen, x, a.lin_thr);
-                        } else {
-                            x = b_lds ? Bl[idx] : Bg[idx];
-                            hit = s_hub >= 0 ? hub_has(a, s_hub, x, s_lim) : has(a.adj + s_ab, s_alen, x, a.lin_thr);
-                        }
-                        for (int q = 0; q < nex; q++) hit &= (x != ex[q]);
-                    }
-                });
-                const unsigned long long m = ballot(hit);
-                const int lo = max(myoff - k0, 0), hi2 = min(myoff + mylen - k0, W);
-                if (lo < hi2) cnt += __popcll(m & range_mask(lo, hi2));
+            if (by_table) {
+                if (!need) cnt = kept;
+                // the excluded vertices the set holds: in the father, below t, adjacent to c
+                const int in = uni(S->ex_in[o.leaf_idx]);
+                for (int f = 0; f < d; f++) {
+                    if (!(in >> f & 1)) continue;
+                    const int x = uni(S->val[f]);
+                    if (live && x < t && ((o.ex_cand >> f & 1u) || adjacent(a, x, c))) cnt--;
+                }
             }
-            S->leafcnt[o.leaf_idx][ln] = cnt;
-            if (a.account && pass && !dup)
-                bytes += 4ull * (alen + blen) + 16ull +
-                         ((has_r && C.P.slots[f].kind == GATP_ALIAS) ? 16ull : 0ull);
+            S->leafcnt[o.leaf_idx][ln] = live ? cnt : 0;
         }
         wsync();
         for (int k = 0; k < N.term_count; k++) {
@@ -935,6 +1059,115 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
         bytes = wave_sum64(bytes);
         if (ln == 0) S->ebytes += bytes;
     }
+}
+
+// The last two levels together (GatNode::pair): the frame's candidates v, 64 at
+// a time, and below them all their candidates c in N(v), flattened over the
+// lanes. A leaf frame of its own per v cost a visit, a frame and a chunk of 64
+// lanes for about 40 candidates: 35 us a chunk on R-MAT s13's C5, most of it
+// the chain of dependent reads from v to the table (285 ms with
+// tables and leaf frames, 108 ms with this, 820 ms without either).
+// Every c takes its value from the kept table; what is missing is computed by
+// sweep_kept. Chunks of v are cut where they would hold more than kPairMax
+// elements, so that the tail of a launch can still be split.
+constexpr int kPairMax = 1 << 14;
+template <bool GS>
+__device__ __noinline__ void pair_leaf(const Ctx C, int d, int node, int cur, int hi, bool can_split) {
+    const KArgs &a = C.a;
+    WaveState *S = C.S;
+    const int ln = C.ln;
+    const GatNode &N = C.P.nodes[node], &M = C.P.nodes[N.child_begin];
+    const GatOp &list = C.P.ops[N.op_begin], &o = C.P.ops[M.op_begin];
+    const GatTerm &Tm = C.P.terms[M.term_begin];
+    leaf_exclusions(C, M, d);
+    const int in = uni(S->ex_in[o.leaf_idx]);
+    unsigned tag;
+    uint2 *tab = pool_table(C, o, &tag);
+    const bool ex_v = o.excl >> d & 1u;
+    unsigned long long sum = 0;
+    int nl = W;
+    for (int cb = cur; cb < hi; cb += nl) {
+        const int vi = cb + ln;
+        int v = 0;
+        if (vi < hi) v = with_slot<GS>(C, N.loop_slot, [&](auto p) { return p[vi]; });
+        const bool use = vi < hi && !equals_any(S, N.excl, d, v);
+        long long vb = 0;
+        int len = 0;
+        bool in_v = false;  // v is excluded from the COUNT and lies in its father
+        if (use) {
+            vb = a.off[v];
+            const int t = min(group_bound(S, list.groups, list.ngroups, d, v), mask_bound(S, M.bound, d, v));
+            len = trunc_len(a, v, vb, (int)(a.off[v + 1] - vb), t);
+            in_v = ex_v;
+        }
+        if (ex_v && !(o.ex_father >> d & 1u))
+            for (int l = 0; l < d; l++)
+                if (o.levels >> l & 1u) in_v = in_v && adjacent(a, uni(S->val[l]), v);
+        int T = 0;
+        int myoff = excl_scan(len, &T);
+        nl = W;
+        if (T > kPairMax) {
+            nl = max(1, __popcll(ballot(myoff + len <= kPairMax)));  // a prefix of the lanes
+            T = __shfl(myoff + len, nl - 1);
+            if (ln >= nl) myoff = T;
+        }
+        constexpr int U = 2;  // steps in flight
+        for (int k0 = 0; k0 < T; k0 += U * W) {
+            int c[U], w[U], t[U];
+            uint2 e[U];
+            bool live[U], wex[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int j = k0 + u * W + ln;
+                c[u] = w[u] = 0;
+                wex[u] = false;
+                if (k0 + u * W < T)
+                    by_owner(myoff, k0 + u * W, T, [&](const auto &pull) {
+                        const long long s_vb = pull(vb);
+                        const int s_off = pull(myoff);
+                        w[u] = pull(v);
+                        wex[u] = pull((int)in_v);
+                        if (j < T) c[u] = a.adj[s_vb + (j - s_off)];
+                    });
+                live[u] = j < T;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                live[u] = live[u] && !equals_any(S, M.excl, d, c[u]) && !((M.excl >> d & 1u) && c[u] == w[u]);
+                e[u] = make_uint2(0, 0);
+                if (live[u] && c[u] < a.tab_size) e[u] = tab[c[u]];
+                t[u] = group_bound(S, o.groups, o.ngroups, d + 1, c[u]);
+            }
+            int cnt[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                cnt[u] = 0;
+                for (int f = 0; f < d; f++) {
+                    if (!(in >> f & 1)) continue;
+                    const int x = uni(S->val[f]);
+                    if (live[u] && x < t[u] && ((o.ex_cand >> f & 1u) || adjacent(a, x, c[u]))) cnt[u]--;
+                }
+                if (live[u] && wex[u] && w[u] < t[u]) cnt[u]--;  // c lies in N(w)
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool need = live[u] && (e[u].x != tag || e[u].y >> 24 != a.epoch);
+                int x = (int)(e[u].y & 0xffffffu);
+                if (ballot(need)) {
+                    const int fresh = sweep_kept<GS>(C, M.op_begin, need, c[u], t[u]);
+                    if (need) {
+                        x = fresh;
+                        if (c[u] < a.tab_size) tab[c[u]] = make_uint2(tag, (unsigned)fresh | a.epoch << 24);
+                    }
+                }
+                if (live[u]) sum += (unsigned long long)(long long)(x + cnt[u]);
+            }
+        }
+        if (can_split && hi - (cb + nl) >= 2 && want_split<GS>(a, S) && donate(C, d, node, cb + nl, hi, 1, !GS)) break;
+    }
+    sum = wave_sum64(sum);
+    if (ln == 0) S->task_acc[Tm.pattern] += sum * (unsigned long long)(long long)C.P.subs[Tm.sub_begin].coef;
+    wsync();
 }
 
 template <bool GS>
@@ -985,7 +1218,7 @@ __device__ __forceinline__ void drop_pending(WaveState *S, int np, int ln) {
 // an edge whose sets outgrow the LDS buffers is handed alone to the HBM
 // launch and the walk goes on with the next edge; otherwise the whole task
 // is abandoned and re-run there.
-template <bool GS>
+template <bool GS, bool KEEP>
 __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e1) {
     const KArgs &a = C.a;
     const GatPlanDev &P = C.P;
@@ -1022,7 +1255,12 @@ __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e
             // loops at depth >= 2 may be handed to a split launch
             const bool can_split = d >= 2;
             if (N.leaf) {
-                leaf<GS>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node);
+                leaf<GS, KEEP>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node);
+                exhausted = true;
+            } else if (KEEP && N.pair && d >= 2) {
+                const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
+                if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
+                pair_leaf<GS>(C, d, node, cur, fh, can_split);
                 exhausted = true;
             } else {
                 const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
@@ -1069,7 +1307,7 @@ __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e
 // path are rebuilt (neither counted nor accounted again), then the walk
 // covers candidates [lo, hi) of its node and their subtrees only. A set that
 // outgrows its LDS buffer leaves S->abort set (the HBM launch re-runs it).
-template <bool GS>
+template <bool GS, bool KEEP>
 __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
     const KArgs &a = C.a;
     const GatPlanDev &P = C.P;
@@ -1115,7 +1353,12 @@ __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
         const GatNode &N = P.nodes[node];
         bool exhausted = false;
         if (N.leaf) {
-            leaf<GS>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node);
+            leaf<GS, KEEP>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node);
+            exhausted = true;
+        } else if (KEEP && N.pair) {
+            const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
+            if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
+            pair_leaf<GS>(C, d, node, cur, fh, can_split);
             exhausted = true;
         } else {
             const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
@@ -1151,9 +1394,8 @@ __global__ void put_kargs(KArgs a, KArgs *dst) {
     if (threadIdx.x == 0) *dst = a;
 }
 
-template <bool GS>
-__global__ void __launch_bounds__(256) engine_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
-    extern __shared__ __align__(16) unsigned char smem[];
+template <bool GS, bool KEEP>
+__device__ __forceinline__ void engine_main(const KArgs *__restrict__ ap, int wave_bytes, unsigned char *smem) {
     const KArgs &a = *ap;
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
     const int wpb = blockDim.x / W;
@@ -1197,7 +1439,7 @@ __global__ void __launch_bounds__(256) engine_kernel(const KArgs *__restrict__ a
             S->t0 = wall_clock64();
         }
         wsync();
-        run_task<GS>(C, e0, e0 + a.chunk < a.e_hi ? e0 + a.chunk : a.e_hi);
+        run_task<GS, KEEP>(C, e0, e0 + a.chunk < a.e_hi ? e0 + a.chunk : a.e_hi);
         wsync();
         if (S->abort) {
             if (GS) {
@@ -1230,9 +1472,8 @@ __global__ void __launch_bounds__(256) engine_kernel(const KArgs *__restrict__ a
 // Subtask launches: list sub_mode (1 .. kSplitLevels: LDS buffers; then the
 // HBM list with HBM buffers). A subtask that outgrows LDS is copied to the
 // HBM list for the last launch.
-template <bool GS>
-__global__ void __launch_bounds__(256) engine_sub_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
-    extern __shared__ __align__(16) unsigned char smem[];
+template <bool GS, bool KEEP>
+__device__ __forceinline__ void engine_sub(const KArgs *__restrict__ ap, int wave_bytes, unsigned char *smem) {
     const KArgs &a = *ap;
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
     const int wpb = blockDim.x / W;
@@ -1269,7 +1510,7 @@ __global__ void __launch_bounds__(256) engine_sub_kernel(const KArgs *__restrict
             S->t0 = wall_clock64();
         }
         wsync();
-        if (uni(g->lo) < uni(g->hi)) run_sub<GS>(C, g);
+        if (uni(g->lo) < uni(g->hi)) run_sub<GS, KEEP>(C, g);
         wsync();
         if (S->abort) {
             if (GS) {
@@ -1304,6 +1545,31 @@ __global__ void __launch_bounds__(256) engine_sub_kernel(const KArgs *__restrict
     if (a.tl && ln == 0)
         tl_write(a.tl, a.tl_base + blockIdx.x * wpb + wid, a.sub_mode + (GS ? 1 : 0), blockIdx.x * wpb + wid, tl_t0,
                  wall_clock64(), 0, 0, tl_items, 0);
+}
+
+// Kernels of plans that keep COUNT values in tables, and of those that do not
+// (and of W_alg accounting, which charges every value): the code of the tables
+// costs the others 8 % (C4 + P4 on a sparse random graph). Four waves per SIMD
+// are worth the spills around the calls.
+template <bool GS>
+__global__ void __launch_bounds__(256, 4) engine_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    engine_main<GS, true>(ap, wave_bytes, smem);
+}
+template <bool GS>
+__global__ void __launch_bounds__(256, 4) engine_sub_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    engine_sub<GS, true>(ap, wave_bytes, smem);
+}
+template <bool GS>
+__global__ void __launch_bounds__(256) engine_plain_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    engine_main<GS, false>(ap, wave_bytes, smem);
+}
+template <bool GS>
+__global__ void __launch_bounds__(256) engine_plain_sub_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    engine_sub<GS, false>(ap, wave_bytes, smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -2402,6 +2668,13 @@ struct PlanDevice {
     long long ovf_cap = 0;
     int *gstore = nullptr;
     size_t gstore_bytes = 0;
+    // kept COUNT values (array store)
+    int *edge_tab[4] = {};
+    uint2 *pool = nullptr;
+    long long pool_entries = 0;
+    unsigned pool_tables = 0, epoch = 0;
+    int tab_size = 0;
+    bool keep = false;
     int ovf_grid = 0;
     hipEvent_t ev[4] = {};
     // clique HBM-tier rows and pair offsets
@@ -2422,7 +2695,8 @@ void destroy_plan_device(PlanDevice *d) {
         if (e) (void)hipEventDestroy(e);
     for (void *p : {(void *)d->plan, (void *)d->dargs, (void *)d->tl, (void *)d->counts, (void *)d->queue, (void *)d->ovf_n, (void *)d->bytes,
                     (void *)d->err, (void *)d->ovf, (void *)d->subs, (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2], (void *)d->tier[3],
-                    (void *)d->gstore, (void *)d->grows,
+                    (void *)d->gstore, (void *)d->edge_tab[0], (void *)d->edge_tab[1], (void *)d->edge_tab[2],
+                    (void *)d->edge_tab[3], (void *)d->pool, (void *)d->grows,
                     (void *)d->goff})
         if (p) (void)hipFree(p);
     if (d->stream) (void)hipStreamDestroy(d->stream);
@@ -2623,6 +2897,32 @@ static int clique_shape(const DeviceInfo &di, const gat_kernel_config &cfg, int 
     return GAT_OK;
 }
 
+// Tables of kept COUNT values (GATP_KEEP_*): an int per directed edge and
+// truncation, cleared by every count, and the pools. A pool's table covers the
+// first kTabVertices vertices (of a degree-ordered graph the most visited
+// ones); there are as many tables as kPoolBytes for all pools holds. Values
+// have 24 bits and keys 32: larger graphs go without.
+constexpr long long kPoolBytes = 1ll << 29;
+constexpr int kTabVertices = 1 << 14;
+static int ensure_tables(gat_plan *p) {
+    PlanDevice *d = p->dev;
+    const GatPlanDev &pd = p->cp.dev;
+    const Graph &g = *p->graph;
+    if (g.m == 0 || g.max_deg >= 1 << 24 || g.m >= (1ll << 32) - 1) return GAT_OK;
+    for (int k = 0; k < 4; k++)
+        if ((pd.edge_tables >> k & 1) && !d->edge_tab[k])
+            HIPCHECK(hipMalloc(&d->edge_tab[k], sizeof(int) * (((size_t)g.m + 1) / 2 * 2)));
+    d->keep = pd.edge_tables || pd.n_tables;
+    if (pd.n_tables == 0 || d->pool) return GAT_OK;
+    d->tab_size = std::min(g.n, kTabVertices);
+    const long long most = kPoolBytes / (8ll * pd.n_tables * d->tab_size);
+    d->pool_tables = (unsigned)std::max(1ll, std::min<long long>(most, pd.key_edges ? g.m : g.n));
+    d->pool_entries = (long long)pd.n_tables * d->pool_tables * d->tab_size;
+    HIPCHECK(hipMalloc(&d->pool, sizeof(uint2) * d->pool_entries));
+    d->epoch = 255;  // cleared by the first count
+    return GAT_OK;
+}
+
 static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     DeviceInfo di;
     int rc = device_info(&di);
@@ -2706,6 +3006,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     a.err = d->err;
     a.cap = cfg.slot_capacity;
     a.chunk = cfg.queue_chunk;
+    L->chunk = cfg.queue_chunk;
     a.lin_thr = cfg.search_linear_threshold;
     a.gallop_ratio = cfg.gallop_ratio;
     a.strategy = cfg.intersect_strategy;
@@ -2719,6 +3020,15 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     a.sovf_n = d->ovf_n + 8 + kLevels + 1;
     a.sovf_base = kLevels * kSubCap;
     a.sovf_cap = 3 * kSubCap;
+    if (!clique) {
+        rc = ensure_tables(p);
+        if (rc) return rc;
+        for (int k = 0; k < 4; k++) a.edge_tab[k] = d->edge_tab[k];
+        a.pool = d->pool;
+        a.pool_tables = d->pool_tables;
+        a.tab_size = d->tab_size;
+        a.keep = d->keep;
+    }
     a.split_ticks = split ? (long long)cfg.split_us * di.wall_khz / 1000 : 0;
     if (!clique && cfg.hub_degree > 0) {
         rc = ensure_hubs(g, d->dg.get(), cfg.hub_degree);
@@ -2848,6 +3158,23 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
     hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, (unsigned long long *)d->err, 1ll, 0ull);
     gatk::KArgs a = L.a, ao = L.ao;
     a.account = ao.account = account ? 1 : 0;
+    if (account) {  // W_alg is accumulated where the values are computed
+        a.keep = ao.keep = 0;
+    }
+    if (!L.clique && a.keep && a.pool) {
+        // epochs 1 .. 254 for counts in turn; replays of a captured count share
+        // one, so it clears the pool itself, as does the first count of a turn
+        const bool clear = !events || d->epoch >= 254;
+        d->epoch = clear ? 1 : d->epoch + 1;
+        a.epoch = ao.epoch = events ? d->epoch : 255;
+        if (clear)
+            hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, s, (unsigned long long *)d->pool,
+                               d->pool_entries, 0ull);
+    }
+    for (int k = 0; k < 4 && !L.clique && a.keep; k++)
+        if (a.edge_tab[k])
+            hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, s, (unsigned long long *)a.edge_tab[k],
+                               (a.m + 1) / 2, ~0ull);
     a.tl = ao.tl = tl;
     ao.bytes = d->bytes + 1;  // second launch: its own W_alg counter
     const int waves = (int)(L.grid.x * (L.block.x / 64));
@@ -2886,7 +3213,8 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
     } else {
         a.tl_base = tl_take(waves);
         hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, a, d->dargs);
-        hipLaunchKernelGGL(gatk::engine_kernel<false>, L.grid, L.block, L.lds, s, d->dargs, L.wave_bytes);
+        const bool keep = a.keep;
+        hipLaunchKernelGGL((keep ? gatk::engine_kernel<false> : gatk::engine_plain_kernel<false>), L.grid, L.block, L.lds, s, d->dargs, L.wave_bytes);
         if (events) HIPCHECK(hipEventRecord(d->ev[1], s));
         if (a.split_ticks > 0)  // split subtasks, level by level, in LDS like the main launch
             for (int k = 1; k <= kLevels; k++) {
@@ -2899,7 +3227,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
                 sk.bytes = d->bytes + 1;
                 sk.tl_base = tl_take(waves);
                 hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, sk, d->dargs + k);
-                hipLaunchKernelGGL(gatk::engine_sub_kernel<false>, L.grid, L.block, L.lds, s, d->dargs + k,
+                hipLaunchKernelGGL((keep ? gatk::engine_sub_kernel<false> : gatk::engine_plain_sub_kernel<false>), L.grid, L.block, L.lds, s, d->dargs + k,
                                    L.wave_bytes);
             }
         ao.out_n = d->ovf_n + 8 + kLevels + 1;  // the HBM launch splits into the HBM list
@@ -2907,7 +3235,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
         ao.out_cap = 3 * kSubCap;
         ao.tl_base = tl_take((int)L.ovf_grid.x);
         hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, ao, d->dargs + kLevels + 1);
-        hipLaunchKernelGGL(gatk::engine_kernel<true>, L.ovf_grid, dim3(64), L.ovf_lds, s, d->dargs + kLevels + 1,
+        hipLaunchKernelGGL((keep ? gatk::engine_kernel<true> : gatk::engine_plain_kernel<true>), L.ovf_grid, dim3(64), L.ovf_lds, s, d->dargs + kLevels + 1,
                            L.ovf_wave_bytes);
         if (ao.split_ticks > 0) {
             gatk::KArgs sh = ao;
@@ -2918,7 +3246,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
             sh.out_n = nullptr;
             sh.tl_base = tl_take((int)L.ovf_grid.x);
             hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, sh, d->dargs + kLevels + 2);
-            hipLaunchKernelGGL(gatk::engine_sub_kernel<true>, L.ovf_grid, dim3(64), L.ovf_lds, s,
+            hipLaunchKernelGGL((keep ? gatk::engine_sub_kernel<true> : gatk::engine_plain_sub_kernel<true>), L.ovf_grid, dim3(64), L.ovf_lds, s,
                                d->dargs + kLevels + 2, L.ovf_wave_bytes);
         }
         if (events) HIPCHECK(hipEventRecord(d->ev[3], s));

@@ -240,6 +240,66 @@ struct Compiler {
     }
 };
 
+// A KEEP_POOL table: values of one father set and truncation over c. Leaves of
+// different depths may share it (the level of c itself is written as bit 7).
+struct KeptTable {
+    std::vector<int> data;
+    std::vector<Mask> groups;
+    bool operator==(const KeptTable &o) const { return data == o.data && groups == o.groups; }
+};
+
+// Decides whether leaf COUNT `s` of node `node` can be kept in a table (see
+// GATP_KEEP_*), and fills the op's fields. The father's levels must not empty
+// their sets on repeated vertices (reference semantics, HNode::A): the value
+// would then not be a function of the key.
+void keep_count(const Compiler &C, int node, const HSlot &s, GatOp *o, std::vector<KeptTable> *tables) {
+    const HSlot &f = C.slots[s.father];
+    const int d = s.depth;
+    if (d < 2) return;  // every (v_0, c) comes once
+    std::vector<Mask> adj(d + 1, 0), empties(d + 1, 0);  // adj[l]: earlier levels v_l is known to be adjacent to
+    for (int n = node; n >= 0; n = C.nodes[n].parent) {
+        adj[C.nodes[n].depth] = C.nodes[n].L;
+        empties[C.nodes[n].depth] = C.nodes[n].A;
+    }
+    Mask data = 0, groups = 0;
+    for (int l : f.data) data |= Mask(1u << l);
+    if (!s.notrunc)
+        for (Mask g : s.groups) groups |= g;
+    const Mask key = Mask((data | groups) & ~(1u << d));
+    for (int l = 0; l < d; l++)
+        if (data >> l & 1u && empties[l]) return;
+    for (int q = 0; q < d; q++) {
+        if (!(s.X >> q & 1u)) continue;
+        bool in = true;
+        for (int l : f.data) in = in && (l < q ? adj[q] >> l & 1u : adj[l] >> q & 1u);
+        if (in) o->ex_father |= uint8_t(1u << q);
+        if (adj[d] >> q & 1u) o->ex_cand |= uint8_t(1u << q);
+    }
+    o->levels = data;
+    const int j = f.data.back();
+    if (f.data.size() == 1 && C.nodes[node].loop_slot == s.father && (s.notrunc || s.groups.size() == 1) &&
+        !(groups & ~((1u << j) | (1u << d)))) {
+        o->keep = GATP_KEEP_EDGE;
+        o->table = int8_t((groups >> j & 1u) | (groups >> d & 1u) << 1);
+        return;
+    }
+    // the value changes with the parent level (no reuse), or its key is none of
+    // v_0, v_1 and the root edge
+    if (key >> (d - 1) || key > 3) return;
+    KeptTable t;
+    t.data = f.data;
+    if (!s.notrunc)
+        for (Mask g : s.groups) t.groups.push_back(Mask((g & ~(1u << d)) | (g >> d & 1u ? 0x80u : 0u)));
+    size_t k = std::find(tables->begin(), tables->end(), t) - tables->begin();
+    if (k == tables->size()) {
+        if (k >= GATP_MAX_TABLES) return;
+        tables->push_back(t);
+    }
+    o->keep = GATP_KEEP_POOL;
+    o->table = int8_t(k);
+    o->key = key;
+}
+
 }  // namespace
 
 int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOptions &opt, CompiledPlan *out) {
@@ -483,6 +543,7 @@ int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOption
 
     d.n_slots = (int)C.slots.size();
     int nops = 0, nterms = 0, nvids = 0, nsubs = 0, max_leaf = 0;
+    std::vector<KeptTable> tables;
     for (size_t ii = 0; ii < order.size(); ii++) {
         const HNode &h = C.nodes[order[ii]];
         GatNode &g = d.nodes[ii];
@@ -502,6 +563,7 @@ int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOption
             if (it + 1 != sib.end()) g.next_sibling = int16_t(newid[*(it + 1)]);
         }
         g.op_begin = int16_t(nops);
+        g.kept = 1;
         int lists = 0, leafc = 0;
         for (int sid : h.ops) {
             if (nops >= GATP_MAX_OPS) GAT_FAIL(GAT_ELIMIT, "plan needs more than %d ops", GATP_MAX_OPS);
@@ -523,6 +585,12 @@ int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOption
             gs.store = -1;
             if (needs_store(sid)) o.store = gs.store = int8_t(store_base[h.depth] + lists++);
             if ((s.kind == GATP_COUNT || s.kind == GATP_ALIAS) && g.leaf) o.leaf_idx = gs.leaf_idx = int8_t(leafc++);
+            if (s.kind == GATP_COUNT && g.leaf && s.father >= 0) {
+                keep_count(C, order[ii], s, &o, &tables);
+                if (o.keep == GATP_KEEP_NONE) g.kept = 0;
+                if (o.keep == GATP_KEEP_EDGE) d.edge_tables |= 1 << o.table;
+                if (o.keep == GATP_KEEP_POOL && o.key == 3) d.key_edges = 1;
+            }
         }
         if (leafc > GATP_MAX_LEAF_OPS) GAT_FAIL(GAT_ELIMIT, "leaf needs %d counters (> %d)", leafc, GATP_MAX_LEAF_OPS);
         max_leaf = std::max(max_leaf, leafc);
@@ -554,11 +622,23 @@ int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOption
         }
         g.term_count = int16_t(nterms - g.term_begin);
     }
+    for (size_t i = 1; i < order.size(); i++) {
+        GatNode &g = d.nodes[i];
+        if (g.leaf || g.child_count != 1 || g.term_count || g.op_count != 1 || g.ap_levels) continue;
+        const GatNode &c = d.nodes[g.child_begin];
+        if (!c.leaf || c.ap_levels || c.op_count != 1 || c.term_count != 1) continue;
+        const GatOp &list = d.ops[g.op_begin], &cnt = d.ops[c.op_begin];
+        const GatTerm &t = d.terms[c.term_begin];
+        g.pair = list.kind == GATP_ALIAS && c.loop_slot == list.slot && cnt.keep == GATP_KEEP_POOL &&
+                 t.sub_count == 1 && d.subs[t.sub_begin].flag && d.vids[d.subs[t.sub_begin].vid].slot == cnt.slot &&
+                 d.vids[d.subs[t.sub_begin].vid].mode == GATP_VID_COUNT;
+    }
     d.n_nodes = (int)order.size();
     d.n_ops = nops;
     d.n_terms = nterms;
     d.n_vids = nvids;
     d.n_subs = nsubs;
+    d.n_tables = (int)tables.size();
     d.n_patterns = (int)adj.size();
     d.max_leaf_ops = max_leaf;
     d.max_depth = maxd;

@@ -22,6 +22,13 @@
 #define GATP_MAX_STORE 12
 
 enum { GATP_ALIAS = 0, GATP_LIST = 1, GATP_COUNT = 2 };
+// KEEP_EDGE: c runs over N(v_j) and the father is N(v_j), so the value belongs
+// to the edge (v_j, c): one table over the directed edges for the whole launch.
+// KEEP_POOL: the father and the truncation depend on v_0, on v_1 or on the root
+// edge (v_0, v_1) only, which stay fixed while the parent level's vertex
+// changes: a table over c for each of them, in a pool all waves share.
+enum { GATP_KEEP_NONE = 0, GATP_KEEP_EDGE = 1, GATP_KEEP_POOL = 2 };
+#define GATP_MAX_TABLES 8
 enum { GATP_VID_COUNT = 0, GATP_VID_LIST_REF = 1, GATP_VID_LIST_BOUNDED = 2 };
 
 typedef struct GatOp {
@@ -33,7 +40,14 @@ typedef struct GatOp {
     uint8_t excl;      // COUNT: levels whose chosen vertex is excluded per element
     int8_t leaf_idx;   // COUNT evaluated per candidate at a leaf: counter index
     int8_t store;      // LIST: storage region
-    int8_t pad;
+    // COUNT at a leaf: how |N(c) ∩ father| of an unchanged father is kept
+    // within a count instead of being recomputed for every path (GATP_KEEP_*)
+    int8_t keep;
+    int8_t table;      // KEEP_EDGE: truncation (bit 0: t <= v_j, bit 1: t <= c); KEEP_POOL: pool index
+    uint8_t key;       // KEEP_POOL: levels the value depends on besides c (1: v_0, 2: v_1, 3: the edge)
+    uint8_t ex_father; // excluded levels whose vertex is known to lie in the father's untruncated set
+    uint8_t levels;    // levels of the father's prefix
+    uint8_t ex_cand;   // excluded levels whose vertex is known to be adjacent to c
 } GatOp;
 
 typedef struct GatNode {
@@ -49,6 +63,9 @@ typedef struct GatNode {
     int16_t child_begin, child_count; // children are consecutive node ids
     int16_t next_sibling;             // -1 when last child of its parent
     int8_t leaf;                      // no children
+    int8_t kept;                      // leaf: every COUNT with a father is kept in a table
+    int8_t pair;                      // its one child is a leaf over N(v_l) with one KEEP_POOL COUNT, alone in the
+                                      // only term: both levels can be swept together
     int8_t pad;
 } GatNode;
 
@@ -87,7 +104,9 @@ typedef struct GatPlanDev {
     int32_t n_nodes, n_slots, n_ops, n_terms, n_vids, n_subs;
     int32_t n_patterns, n_store, max_leaf_ops, max_depth;
     int32_t root_slot;  // ALIAS slot of prefix [0]
-    int32_t pad;
+    int32_t n_tables;   // KEEP_POOL pools
+    int32_t edge_tables; // bit k: a KEEP_EDGE table of truncation k is used
+    int32_t key_edges;  // some KEEP_POOL op is keyed by the root edge
     GatNode nodes[GATP_MAX_NODES];
     GatSlot slots[GATP_MAX_SLOTS];
     GatOp ops[GATP_MAX_OPS];
