@@ -56,14 +56,18 @@ struct KArgs {
     long long e_lo, e_hi;        // root edges of this count: [e_lo, e_hi)
     const GatPlanDev *plan;
     unsigned long long *counts;  // kCountCopies copies of [GATP_MAX_TERMS]
-    unsigned long long *queue;   // [0] main queue head, [1] overflow head
+    unsigned long long *queue;   // heads of the launches' queues (see queue_next)
+    unsigned int *drained;       // [queue] set once a wave has found the queue empty
     long long *ovf;              // overflow task starts
     unsigned long long *ovf_n;   // overflow task count
     long long ovf_cap;
     int *gstore;                 // HBM set buffers (overflow launch)
     unsigned long long *bytes;   // W_alg accumulator
     unsigned int *err;           // device error flags
-    int cap;                     // entries per set buffer
+    int cap;                     // entries per buffer of an intersection
+    int stage_cap;               // entries per buffer of a staged neighbour list
+    long long store_off[GATP_MAX_STORE];  // first entry of each set buffer
+    int state_bytes;             // LDS of a wave before its set buffers
     int chunk;
     int lin_thr;
     int gallop_ratio;
@@ -146,7 +150,6 @@ struct WaveState {
     int f_node[GATP_MAX_DEPTH + 1];
     int f_cur[GATP_MAX_DEPTH + 1];
     int f_hi[GATP_MAX_DEPTH + 1];
-    int leafcnt[GATP_MAX_LEAF_OPS][W];
     unsigned long long bytes;   // committed W_alg of this wave
     unsigned long long ebytes;  // W_alg of the work not yet committed
     long long t0;               // wall clock at the start of the task
@@ -158,7 +161,8 @@ struct WaveState {
     int base_depth;             // frames exist from this depth on (2, or a subtask's depth)
     int path_pos[GATP_MAX_DEPTH + 1];  // a subtask's positions at depths 2 .. base_depth-1
     int abort;
-    int ex_in[GATP_MAX_LEAF_OPS];                  // leaf: excluded levels whose vertex lies in the op's father
+    int ex_in[GATP_MAX_LEAF_OPS];  // leaf: excluded levels whose vertex lies in the op's father
+    int leafcnt[GATP_MAX_LEAF_OPS][W];  // last: only the plan's max_leaf_ops rows are allocated
 };
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
@@ -280,6 +284,45 @@ __device__ __forceinline__ bool has(P a, int len, int x, int lin_thr) {
         n -= half;
     }
     return a[base] == x;
+}
+
+// Work queues. Atomics on one address are performed one after the other, about
+// 20 ns each on this chip, so one head would feed a launch at most 50 tasks per
+// microsecond and hold back every wave that asks meanwhile (C4 + P4 on a random
+// graph of 1.6M directed edges: 8.8 ms with 16 edges per task and 19 ms with 4;
+// 3.8 and 4.3 ms with 64 heads; a launch without work: 50 and 6 us). A queue has kHeads heads on cache lines of their own; head q hands out the items
+// (r / kRun kHeads + q) kRun + r % kRun, r = 0, 1, ..: runs of kRun neighbouring
+// items, which share a root and the tables kept for it, go to the waves of one
+// head, and waves 8 apart sit on one XCD. A wave whose head is empty moves on to
+// the next one with items left.
+constexpr int kHeads = 64, kHeadStride = 16, kRun = 8;
+enum { kQueueMain = 0, kQueueOverflow = 1, kQueueSub = 1 /* + sub_mode */, kQueues = 6 };
+constexpr int kQueueWords = kQueues * kHeads * kHeadStride;
+__device__ __forceinline__ long long queue_item(unsigned long long r, int q) {
+    return (long long)((r / kRun * kHeads + q) * kRun + r % kRun);
+}
+// The next of the n items of queue id, or -1; *q: this wave's head.
+__device__ __forceinline__ long long queue_next(unsigned long long *queue, unsigned int *drained, int id, long long n,
+                                                int *q, int ln) {
+    if (n <= 0) return -1;
+    unsigned long long *heads = queue + id * kHeads * kHeadStride;
+    for (;;) {
+        unsigned long long r = 0;
+        if (ln == 0) r = atomicAdd(&heads[*q * kHeadStride], 1ull);
+        const long long item = queue_item((unsigned long long)uni64((long long)__shfl(r, 0)), *q);
+        if (item < n) return item;
+        static_assert(kHeads == W, "one head per lane");
+        const unsigned long long at = __hip_atomic_load(&heads[ln * kHeadStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long m = ballot(queue_item(at, ln) < n);
+        if (!m) {
+            if (ln == 0 && !__hip_atomic_load(&drained[id], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                __hip_atomic_store(&drained[id], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return -1;
+        }
+        const int k = (*q + 1) % kHeads;  // the next head from k on that has items
+        const unsigned long long rot = k ? m >> k | m << (kHeads - k) : m;
+        *q = (k + __ffsll((long long)rot) - 1) % kHeads;
+    }
 }
 
 // Counters are kept in kCountCopies copies of GATP_MAX_TERMS, one per group of
@@ -517,7 +560,7 @@ template <bool GS, class F>
 __device__ __forceinline__ auto with_slot(const Ctx &C, int slot, F f) {
     const GatSlot &s = C.P.slots[slot];
     if (s.kind == GATP_ALIAS && (GS || !C.S->staged[slot])) return f(C.a.adj + C.S->sbeg[slot]);
-    return f(C.store + (long long)s.store * C.a.cap);
+    return f(C.store + C.a.store_off[s.store]);
 }
 // Is the slot's content in this wave's LDS buffers?
 template <bool GS>
@@ -539,9 +582,9 @@ __device__ __forceinline__ void exec_op_uniform(const Ctx &C, const GatOp &o, in
     const int slot = o.slot;
     if (o.kind == GATP_ALIAS) {
         // a list that later ops search is staged into LDS when it fits
-        const bool stage = !GS && o.store >= 0 && alen <= a.cap;
+        const bool stage = !GS && o.store >= 0 && alen <= a.stage_cap;
         if (stage) {
-            int *dst = C.store + (long long)o.store * a.cap;
+            int *dst = C.store + a.store_off[o.store];
             for (int k = C.ln; k < alen; k += W) dst[k] = a.adj[ab + k];
         }
         if (C.ln == 0) {
@@ -580,7 +623,7 @@ __device__ __forceinline__ void exec_op_uniform(const Ctx &C, const GatOp &o, in
         }
     }
     const int *A = a.adj + ab;
-    int *out = C.store + (long long)(o.store < 0 ? 0 : o.store) * a.cap;
+    int *out = C.store + a.store_off[o.store < 0 ? 0 : o.store];
     const int hub_a = has_r ? uni(hub_of(a, c)) : -1;
     const bool sa = !has_r || stream_a(a, alen, blen, b_lds || hub_b >= 0, hub_a >= 0);
     const int lin = a.lin_thr;
@@ -604,11 +647,11 @@ __device__ __forceinline__ void exec_op_uniform(const Ctx &C, const GatOp &o, in
     };
     if (sorted_pair) {
         if (b_lds) {
-            const int *B = C.store + (long long)C.P.slots[f].store * a.cap;
+            const int *B = C.store + a.store_off[C.P.slots[f].store];
             result = run2(A, alen, B, blen);
         } else {
             const int *B = C.P.slots[f].kind == GATP_ALIAS ? a.adj + bbeg
-                                                           : C.store + (long long)C.P.slots[f].store * a.cap;
+                                                           : C.store + a.store_off[C.P.slots[f].store];
             result = run2(A, alen, B, blen);
         }
     } else if (!has_r && o.kind == GATP_COUNT) {
@@ -618,14 +661,14 @@ __device__ __forceinline__ void exec_op_uniform(const Ctx &C, const GatOp &o, in
     } else if (sa) {
         // stream A, probe the father: LDS buffer, hub bitmap, or HBM list
         if (b_lds) {
-            const int *B = C.store + (long long)C.P.slots[f].store * a.cap;
+            const int *B = C.store + a.store_off[C.P.slots[f].store];
             result = run(A, alen, [&](int x) { return has(B, blen, x, lin); });
         } else if (hub_b >= 0) {
             const int lim = uni(list_lim(a, bbeg, blen));
             result = run(A, alen, [&](int x) { return hub_has(a, hub_b, x, lim); });
         } else {
             const int *B = C.P.slots[f].kind == GATP_ALIAS ? a.adj + bbeg
-                                                           : C.store + (long long)C.P.slots[f].store * a.cap;
+                                                           : C.store + a.store_off[C.P.slots[f].store];
             result = run(A, alen, [&](int x) { return has(B, blen, x, lin); });
         }
     } else {
@@ -634,11 +677,11 @@ __device__ __forceinline__ void exec_op_uniform(const Ctx &C, const GatOp &o, in
         const int lim_a = hub_a >= 0 ? uni(list_lim(a, ab, alen)) : 0;
         auto probe_hub = [&](int x) { return hub_has(a, hub_a, x, lim_a); };
         if (b_lds) {
-            const int *B = C.store + (long long)C.P.slots[f].store * a.cap;
+            const int *B = C.store + a.store_off[C.P.slots[f].store];
             result = hub_a >= 0 ? run(B, blen, probe_hub) : run(B, blen, probe_a);
         } else {
             const int *B = C.P.slots[f].kind == GATP_ALIAS ? a.adj + bbeg
-                                                           : C.store + (long long)C.P.slots[f].store * a.cap;
+                                                           : C.store + a.store_off[C.P.slots[f].store];
             result = hub_a >= 0 ? run(B, blen, probe_hub) : run(B, blen, probe_a);
         }
     }
@@ -674,16 +717,8 @@ __device__ __noinline__ void cancel_donations(const KArgs &a, WaveState *S, int 
 template <bool GS>
 __device__ __forceinline__ bool queue_drained(const KArgs &a) {
     if (a.split_ticks <= 0 || a.sub_mode >= kSplitLevels) return false;
-    if (GS) {  // the HBM launch: its overflow list is drained
-        const unsigned long long made = __atomic_load_n(a.ovf_n, __ATOMIC_RELAXED);
-        const unsigned long long total = made < (unsigned long long)a.ovf_cap ? made : (unsigned long long)a.ovf_cap;
-        return __atomic_load_n(&a.queue[1], __ATOMIC_RELAXED) >= total;
-    }
-    if (a.sub_mode == 0)
-        return (long long)__atomic_load_n(&a.queue[0], __ATOMIC_RELAXED) >= a.e_hi - a.e_lo;
-    const unsigned long long made = __atomic_load_n(a.in_n, __ATOMIC_RELAXED);
-    const unsigned long long total = made < (unsigned long long)a.in_cap ? made : (unsigned long long)a.in_cap;
-    return __atomic_load_n(&a.queue[1 + a.sub_mode], __ATOMIC_RELAXED) >= total;
+    const int id = GS ? kQueueOverflow : a.sub_mode == 0 ? kQueueMain : kQueueSub + a.sub_mode;
+    return uni((int)__hip_atomic_load(&a.drained[id], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
 }
 template <bool GS>
 __device__ __forceinline__ bool want_split(const KArgs &a, const WaveState *S) {
@@ -834,9 +869,9 @@ __device__ __forceinline__ int sweep_count(const Ctx &C, const GatOp &o, bool ne
     int hub_b = -1, lim_b = 0;
     const GatSlot &fs = C.P.slots[f];
     const bool b_lds = in_lds<GS>(C, f);
-    if (b_lds) Bl = C.store + (long long)fs.store * a.cap;
+    if (b_lds) Bl = C.store + a.store_off[fs.store];
     else if (fs.kind == GATP_ALIAS) Bg = a.adj + S->sbeg[f];
-    else if constexpr (GS) Bg = C.store + (long long)fs.store * a.cap;
+    else if constexpr (GS) Bg = C.store + a.store_off[fs.store];
     const int flen = S->slen[f];
     if (need) blen = t == INT_MAX ? flen : (b_lds ? lbound(Bl, flen, t) : lbound(Bg, flen, t));
     if (!b_lds && fs.kind == GATP_ALIAS) hub_b = uni(hub_of(a, S->val[fs.depth]));
@@ -1405,7 +1440,7 @@ __device__ __forceinline__ void engine_main(const KArgs *__restrict__ ap, int wa
     if (GS)
         store = a.gstore + (long long)(blockIdx.x * wpb + wid) * P.n_store * (long long)a.cap;
     else
-        store = reinterpret_cast<int *>(smem + (size_t)wid * wave_bytes + sizeof(WaveState));
+        store = reinterpret_cast<int *>(smem + (size_t)wid * wave_bytes + a.state_bytes);
     Ctx C{a, P, S, store, ln};
     const int np = P.n_patterns;
     const long long tl_t0 = wall_clock64();
@@ -1416,21 +1451,14 @@ __device__ __forceinline__ void engine_main(const KArgs *__restrict__ ap, int wa
         S->ebytes = 0;
     }
     wsync();
+    int head = (int)((blockIdx.x * wpb + wid) % kHeads);
+    const long long items = GS ? ((long long)*a.ovf_n < a.ovf_cap ? (long long)*a.ovf_n : a.ovf_cap)
+                               : (a.e_hi - a.e_lo + a.chunk - 1) / a.chunk;
     for (;;) {
         long long e0;  // the task: directed edges [e0, e0 + chunk)
-        if (GS) {
-            unsigned long long r = 0;
-            if (ln == 0) r = atomicAdd(&a.queue[1], 1ull);
-            r = (unsigned long long)uni64((long long)__shfl(r, 0));
-            const unsigned long long total = *a.ovf_n;
-            if (r >= total || (long long)r >= a.ovf_cap) break;
-            e0 = uni64(a.ovf[r]);
-        } else {
-            unsigned long long r = 0;
-            if (ln == 0) r = atomicAdd(&a.queue[0], (unsigned long long)a.chunk);
-            e0 = a.e_lo + uni64((long long)__shfl(r, 0));
-            if (e0 >= a.e_hi) break;
-        }
+        const long long r = queue_next(a.queue, a.drained, GS ? kQueueOverflow : kQueueMain, items, &head, ln);
+        if (r < 0) break;
+        e0 = GS ? uni64(a.ovf[r]) : a.e_lo + r * a.chunk;
         tl_items++;
         for (int i = ln; i < np; i += W) S->task_acc[i] = 0;
         if (ln == 0) {
@@ -1483,7 +1511,7 @@ __device__ __forceinline__ void engine_sub(const KArgs *__restrict__ ap, int wav
     if (GS)
         store = a.gstore + (long long)(blockIdx.x * wpb + wid) * P.n_store * (long long)a.cap;
     else
-        store = reinterpret_cast<int *>(smem + (size_t)wid * wave_bytes + sizeof(WaveState));
+        store = reinterpret_cast<int *>(smem + (size_t)wid * wave_bytes + a.state_bytes);
     Ctx C{a, P, S, store, ln};
     const int np = P.n_patterns;
     const long long tl_t0 = wall_clock64();
@@ -1494,14 +1522,13 @@ __device__ __forceinline__ void engine_sub(const KArgs *__restrict__ ap, int wav
         S->ebytes = 0;
     }
     wsync();
+    int head = (int)((blockIdx.x * wpb + wid) % kHeads);
+    const unsigned long long made = *a.in_n;
+    const long long items = (long long)made < a.in_cap ? (long long)made : a.in_cap;
     for (;;) {
-        unsigned long long r = 0;
-        if (ln == 0) r = atomicAdd(&a.queue[1 + a.sub_mode], 1ull);
-        r = (unsigned long long)uni64((long long)__shfl(r, 0));
-        const unsigned long long made = *a.in_n;
-        const unsigned long long total = made < (unsigned long long)a.in_cap ? made : (unsigned long long)a.in_cap;
-        if (r >= total) break;
-        const SplitTask *g = a.subs + a.in_base + (long long)r;
+        const long long r = queue_next(a.queue, a.drained, kQueueSub + a.sub_mode, items, &head, ln);
+        if (r < 0) break;
+        const SplitTask *g = a.subs + a.in_base + r;
         tl_items++;
         for (int i = ln; i < np; i += W) S->task_acc[i] = 0;
         if (ln == 0) {
@@ -2806,11 +2833,16 @@ static int ensure_core(const Graph &g, DeviceGraph *dg) {
 constexpr long long kSubCap = 1ll << 20;
 constexpr int kLevels = gatk::kSplitLevels;
 constexpr int kSplitUs = 2000;
+// queue words of a plan: 16 of the clique store, the array store's heads, and
+// its drained flags
+constexpr int kQueueAlloc = 16 + gatk::kQueueWords + gatk::kQueues;
 // device argument records of one array-store count: the main launch, the
 // LDS subtask levels, the HBM launch and the HBM subtask launch
 constexpr int kArgSlots = kLevels + 3;
 // timeline capacity (records of gatk::kTlFields int64 each)
 constexpr int kTlCap = 1 << 15;
+
+constexpr int64_t kTasksPerWave = 8;
 
 struct Launch {
     gatk::KArgs a;
@@ -2828,6 +2860,8 @@ struct Launch {
     size_t tier_lds[gatk::CTIERS] = {};
     long long tasks = 0;  // root edges of the count
     int chunk = 1;        // queue_chunk
+    int64_t waves = 1;    // waves of the main launch
+    bool edge_grain = false;  // the HBM launch takes single edges
     bool heavy = false;   // clique: some vertex may have more than main_max neighbours below it
 };
 
@@ -2843,10 +2877,18 @@ static int clique_chunk(int configured, long long vertices, long long waves) {
 // Restrict a prepared count to the root vertices [lo, hi): the array store
 // takes the directed edges of those vertices, the bitmap store those top
 // vertices.
+static void set_edges(Launch *L, int64_t lo, int64_t hi) {
+    L->a.e_lo = L->ao.e_lo = lo;
+    L->a.e_hi = L->ao.e_hi = hi;
+    L->tasks = hi - lo;
+    // edges per task: as configured, but at least kTasksPerWave tasks per wave
+    // (few edges: R-MAT s10 with 16 edges per task left two thirds of the waves
+    // without one)
+    L->a.chunk = (int)std::max<int64_t>(1, std::min<int64_t>(L->chunk, (hi - lo) / (kTasksPerWave * L->waves)));
+    L->ao.chunk = L->edge_grain ? 1 : L->a.chunk;
+}
 static void set_roots(Launch *L, const Graph &g, int32_t lo, int32_t hi) {
-    L->a.e_lo = L->ao.e_lo = g.off[lo];
-    L->a.e_hi = L->ao.e_hi = g.off[hi];
-    L->tasks = g.off[hi] - g.off[lo];
+    set_edges(L, g.off[lo], g.off[hi]);
     L->ca.root_lo = lo;
     L->ca.root_hi = hi;
     if (!L->clique) return;
@@ -2945,7 +2987,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         HIPCHECK(hipMalloc(&d->plan, sizeof(GatPlanDev)));
         HIPCHECK(hipMemcpy(d->plan, &pd, sizeof(GatPlanDev), hipMemcpyHostToDevice));
         HIPCHECK(hipMalloc(&d->counts, sizeof(unsigned long long) * GATP_MAX_TERMS * gatk::kCountCopies));
-        HIPCHECK(hipMalloc(&d->queue, sizeof(unsigned long long) * 16));
+        HIPCHECK(hipMalloc(&d->queue, sizeof(unsigned long long) * kQueueAlloc));
         HIPCHECK(hipMalloc(&d->ovf_n, sizeof(unsigned long long) * 16));
         HIPCHECK(hipMalloc(&d->bytes, sizeof(unsigned long long) * 4));
         HIPCHECK(hipMalloc(&d->err, sizeof(unsigned int) * 2));
@@ -2971,7 +3013,9 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     // single-child roots hand over single edges (run_task), others whole tasks
     const bool edge_grain = pd.nodes[0].child_count == 1;
     // overflow entries: edges or tasks, and split subtasks
-    const long long ovf_cap = clique ? 1 : (edge_grain ? g.m + 1 : (g.m + chunk - 1) / chunk + 1);
+    const long long waves = (long long)std::max(1, cfg.waves_per_cu * di.cus);
+    const long long ovf_cap =
+        clique ? 1 : (edge_grain ? g.m + 1 : std::max((g.m + chunk - 1) / chunk, 2 * kTasksPerWave * waves) + 1);
     const bool split = !clique && cfg.split_us > 0;
     // subtask lists: the LDS levels (kSubCap each), then the HBM list (LDS
     // overflow of the levels plus the HBM launch's splits, 3 kSubCap)
@@ -2982,11 +3026,28 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         HIPCHECK(hipMalloc(&d->ovf, sizeof(long long) * ovf_cap));
         d->ovf_cap = ovf_cap;
     }
-    const int wave_bytes = int((sizeof(gatk::WaveState) + size_t(pd.n_store) * cfg.slot_capacity * 4 + 15) / 16 * 16);
+    // A wave's LDS: its state (with the leaf counters the plan needs) and its
+    // set buffers. A neighbour list is staged for binary searches; from
+    // hub_degree entries on its bitmap serves, so its buffer ends there (house:
+    // 17.9 KB per wave with full buffers, 8 waves per CU; 10.6 KB and 14 with
+    // these). Configs are judged by the full size, whatever a plan needs of it.
+    const size_t full = (sizeof(gatk::WaveState) + size_t(pd.n_store) * cfg.slot_capacity * 4 + 15) / 16 * 16;
+    if (full * cfg.block_waves > di.lds_per_block)
+        GAT_FAIL(GAT_EINFEASIBLE, "config needs %zu B of LDS per workgroup (device allows %zu)",
+                 full * cfg.block_waves, di.lds_per_block);
+    const int state_bytes = int((sizeof(gatk::WaveState) -
+                                 size_t(GATP_MAX_LEAF_OPS - pd.max_leaf_ops) * sizeof(int) * 64 + 15) / 16 * 16);
+    const int stage_cap = cfg.hub_degree > 0 ? std::min(cfg.slot_capacity, (cfg.hub_degree + 3) / 4 * 4)
+                                             : cfg.slot_capacity;
+    long long store_off[GATP_MAX_STORE] = {}, entries = 0;
+    for (int r = 0; r < pd.n_store; r++) {
+        bool list = false;  // does some slot keep an intersection here?
+        for (int i = 0; i < pd.n_slots; i++) list |= pd.slots[i].store == r && pd.slots[i].kind == GATP_LIST;
+        store_off[r] = entries;
+        entries += list ? cfg.slot_capacity : stage_cap;
+    }
+    const int wave_bytes = int((size_t(state_bytes) + size_t(entries) * 4 + 15) / 16 * 16);
     const size_t lds = size_t(wave_bytes) * cfg.block_waves;
-    if (lds > di.lds_per_block)
-        GAT_FAIL(GAT_EINFEASIBLE, "config needs %zu B of LDS per workgroup (device allows %zu)", lds,
-                 di.lds_per_block);
     gatk::KArgs a{};
     a.off = d->dg->off;
     a.adj = d->dg->adj;
@@ -2997,7 +3058,8 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     a.e_hi = g.m;
     a.plan = d->plan;
     a.counts = d->counts;
-    a.queue = d->queue;
+    a.queue = d->queue + 16;
+    a.drained = reinterpret_cast<unsigned *>(d->queue + 16 + gatk::kQueueWords);
     a.ovf = d->ovf;
     a.ovf_n = d->ovf_n;
     a.ovf_cap = d->ovf_cap;
@@ -3005,6 +3067,9 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     a.bytes = d->bytes;
     a.err = d->err;
     a.cap = cfg.slot_capacity;
+    a.stage_cap = stage_cap;
+    a.state_bytes = state_bytes;
+    for (int r = 0; r < GATP_MAX_STORE; r++) a.store_off[r] = store_off[r];
     a.chunk = cfg.queue_chunk;
     L->chunk = cfg.queue_chunk;
     a.lin_thr = cfg.search_linear_threshold;
@@ -3045,10 +3110,12 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     L->lds = lds;
     L->wave_bytes = wave_bytes;
     L->ao = a;
+    L->waves = waves;
+    L->edge_grain = edge_grain;
     L->ao.cap = std::max(1, g.max_deg);
-    if (edge_grain) L->ao.chunk = 1;
+    for (int r = 0; r < GATP_MAX_STORE; r++) L->ao.store_off[r] = (long long)r * L->ao.cap;
     L->ovf_grid = dim3(d->ovf_grid);
-    L->ovf_wave_bytes = int((sizeof(gatk::WaveState) + 15) / 16 * 16);
+    L->ovf_wave_bytes = state_bytes;
     L->ovf_lds = L->ovf_wave_bytes;
     L->clique = clique;
     if (clique) {
@@ -3075,7 +3142,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         c.counts = a.counts;
         for (int k = 0; k < 8; k++) c.pat_of_k[k] = p->cp.clique_pattern[k];
         c.kmax = 31 - __builtin_clz(p->cp.clique_ks);
-        c.queue = a.queue;
+        c.queue = d->queue;
         c.ovf_n = a.ovf_n;
         c.bytes = a.bytes;
         c.err = a.err;
@@ -3152,7 +3219,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
     }
     hipLaunchKernelGGL(gatk::fill_u64, dim3(4), dim3(256), 0, s, d->counts,
                        (long long)GATP_MAX_TERMS * gatk::kCountCopies, 0ull);
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->queue, 16ll, 0ull);
+    hipLaunchKernelGGL(gatk::fill_u64, dim3(8), dim3(256), 0, s, d->queue, (long long)kQueueAlloc, 0ull);
     hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->ovf_n, 16ll, 0ull);
     hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->bytes, 4ll, 0ull);
     hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, (unsigned long long *)d->err, 1ll, 0ull);
@@ -3398,9 +3465,7 @@ extern "C" int gat_count_shard_edges(gat_plan *p, const gat_kernel_config *cfg, 
                                    "shards by top vertex (gat_count_shard)");
     // the array store's queue runs over root edges; every task finds its
     // root by binary search, so any edge range is a shard
-    L.a.e_lo = L.ao.e_lo = edge_begin;
-    L.a.e_hi = L.ao.e_hi = edge_end;
-    L.tasks = edge_end - edge_begin;
+    set_edges(&L, edge_begin, edge_end);
     rc = enqueue(p->dev, L, (flags & GAT_FLAG_ACCOUNT) != 0, true, (flags & GAT_FLAG_TIMELINE) != 0);
     if (rc) return rc;
     return finish(p, L, raw_out, stats, true, true);
