@@ -765,6 +765,8 @@ __device__ __noinline__ bool donate(const Ctx C, int d, int node, int lo, int hi
     return true;
 }
 
+constexpr int kPairChunk = 8;  // least candidates of a subtask at a pair node (pair_leaf)
+
 // Donates the rest of the shallowest frame (depth >= base_depth, up to d)
 // that has two or more candidates left; true if it did. The frame is closed
 // by lowering its end to its cursor: f_cur[k] - 1 stays the position of the
@@ -776,7 +778,7 @@ __device__ __noinline__ bool split_shallowest(const Ctx C, int d) {
     for (int k = uni(S->base_depth); k <= d; k++) {
         const int cur = uni(S->f_cur[k]), fh = uni(S->f_hi[k]);
         if (fh - cur < 2) continue;
-        if (!donate(C, k, uni(S->f_node[k]), cur, fh, C.P.nodes[uni(S->f_node[k])].leaf ? W : 1, !GS)) return false;
+        if (!donate(C, k, uni(S->f_node[k]), cur, fh, C.P.nodes[uni(S->f_node[k])].leaf ? W : C.P.nodes[uni(S->f_node[k])].pair ? kPairChunk : 1, !GS)) return false;
         if (C.ln == 0) S->f_hi[k] = cur;
         wsync();
         return true;
@@ -917,9 +919,10 @@ __device__ __forceinline__ int sweep_count(const Ctx &C, const GatOp &o, bool ne
     *blen_out = blen;
     return cnt;
 }
-// The same from the candidate alone, out of line (rare calls).
+// The same from the candidate alone. (Out of line, this and pair_leaf cost C5
+// on R-MAT s13 a third: 19.9 against 14.7 ms.)
 template <bool GS>
-__device__ __noinline__ int sweep_kept(const Ctx C, int op, bool need, int c, int t) {
+__device__ __forceinline__ int sweep_kept(const Ctx C, int op, bool need, int c, int t) {
     const long long ab = need ? C.a.off[c] : 0;
     const int alen = need ? trunc_len(C.a, c, ab, (int)(C.a.off[c + 1] - ab), t) : 0;
     int blen;
@@ -938,10 +941,12 @@ __device__ __forceinline__ uint2 *pool_table(const Ctx &C, const GatOp &o, unsig
     return a.pool + ((long long)o.table * a.pool_tables + key % a.pool_tables) * a.tab_size;
 }
 
-// Is x adjacent to y? x is the same in every lane.
-__device__ __forceinline__ bool adjacent(const KArgs &a, int x, int y) {
-    const int hx = uni(hub_of(a, x));
-    if (hx >= 0) return hub_has(a, hx, y, INT_MAX);
+// Is x adjacent to y, for the lanes in `need`? x, its hub row hx (hub_of) and
+// so the branches on it are the same in every lane; hx is found outside, by the
+// whole wave, so that no cross-lane read stands under a lane's condition.
+__device__ __forceinline__ bool adjacent(const KArgs &a, int x, int hx, int y, bool need) {
+    if (hx >= 0) return need && hub_has(a, hx, y, INT_MAX);
+    if (!need) return false;
     const int hy = hub_of(a, y);
     if (hy >= 0) return hub_has(a, hy, x, INT_MAX);
     const long long b = a.off[x];
@@ -965,8 +970,9 @@ __device__ __forceinline__ void leaf_exclusions(const Ctx &C, const GatNode &N, 
             for (int g = 0; g < f; g++) yes &= !((o.excl >> g & 1u) && S->val[g] == x);
             if (yes && !(o.ex_father >> f & 1u)) {
                 // the father's set is the intersection of N(v_l) over its levels
-                for (int l = 0; l < GATP_MAX_DEPTH && yes; l++)
-                    if (o.levels >> l & 1u) yes = adjacent(a, x, uni(S->val[l]));
+                const int hx = uni(hub_of(a, x));
+                for (int l = 0; l < GATP_MAX_DEPTH; l++)
+                    if (o.levels >> l & 1u) yes = adjacent(a, x, hx, uni(S->val[l]), yes);
             }
             if (uni((int)yes)) in |= 1 << f;
         }
@@ -1074,7 +1080,9 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
                 for (int f = 0; f < d; f++) {
                     if (!(in >> f & 1)) continue;
                     const int x = uni(S->val[f]);
-                    if (live && x < t && ((o.ex_cand >> f & 1u) || adjacent(a, x, c))) cnt--;
+                    const bool below = live && x < t;
+                    if (o.ex_cand >> f & 1u) cnt -= below;
+                    else cnt -= adjacent(a, x, uni(hub_of(a, x)), c, below);
                 }
             }
             S->leafcnt[o.leaf_idx][ln] = live ? cnt : 0;
@@ -1100,14 +1108,14 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
 // a time, and below them all their candidates c in N(v), flattened over the
 // lanes. A leaf frame of its own per v cost a visit, a frame and a chunk of 64
 // lanes for about 40 candidates: 35 us a chunk on R-MAT s13's C5, most of it
-// the chain of dependent reads from v to the table (285 ms with
-// tables and leaf frames, 108 ms with this, 820 ms without either).
+// the chain of dependent reads from v to the table (820 ms without
+// tables; of this step alone 285 to 108).
 // Every c takes its value from the kept table; what is missing is computed by
 // sweep_kept. Chunks of v are cut where they would hold more than kPairMax
 // elements, so that the tail of a launch can still be split.
 constexpr int kPairMax = 1 << 14;
 template <bool GS>
-__device__ __noinline__ void pair_leaf(const Ctx C, int d, int node, int cur, int hi, bool can_split) {
+__device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur, int hi, bool can_split) {
     const KArgs &a = C.a;
     WaveState *S = C.S;
     const int ln = C.ln;
@@ -1115,10 +1123,37 @@ __device__ __noinline__ void pair_leaf(const Ctx C, int d, int node, int cur, in
     const GatOp &list = C.P.ops[N.op_begin], &o = C.P.ops[M.op_begin];
     const GatTerm &Tm = C.P.terms[M.term_begin];
     leaf_exclusions(C, M, d);
-    const int in = uni(S->ex_in[o.leaf_idx]);
     unsigned tag;
     uint2 *tab = pool_table(C, o, &tag);
     const bool ex_v = o.excl >> d & 1u;
+    // what the chosen vertices of the levels below d mean for every c: skip[],
+    // the vertices c must differ from; less[], those to subtract where c is
+    // adjacent to them (whether that is known: less_known) and they lie below t
+    int skip[GATP_MAX_DEPTH], less[GATP_MAX_DEPTH], less_hub[GATP_MAX_DEPTH], n_skip = 0, n_less = 0;
+    unsigned less_known = 0;
+    const int in = uni(S->ex_in[o.leaf_idx]);
+#pragma unroll
+    for (int i = 0; i < GATP_MAX_DEPTH; i++) skip[i] = less[i] = less_hub[i] = 0;
+    for (int f = 0; f < d; f++) {
+        const int x = uni(S->val[f]), hx = uni(hub_of(a, x));
+#pragma unroll
+        for (int i = 0; i < GATP_MAX_DEPTH; i++) {  // constant indexes keep the arrays in registers
+            if ((M.excl >> f & 1u) && i == n_skip) skip[i] = x;
+            if ((in >> f & 1) && i == n_less) {
+                less[i] = x;
+                less_hub[i] = hx;
+            }
+        }
+        if (M.excl >> f & 1u) n_skip++;
+        if (in >> f & 1) {
+            if (o.ex_cand >> f & 1u) less_known |= 1u << n_less;
+            n_less++;
+        }
+    }
+    unsigned levels = 0;
+    for (int i = 0; i < o.ngroups; i++) levels |= o.groups[i];
+    const bool t_lane = levels >> (d + 1) & 1u;  // the truncation depends on c
+    const int t_all = t_lane ? 0 : uni(group_bound(S, o.groups, o.ngroups, d + 1, 0));
     unsigned long long sum = 0;
     int nl = W;
     for (int cb = cur; cb < hi; cb += nl) {
@@ -1137,7 +1172,10 @@ __device__ __noinline__ void pair_leaf(const Ctx C, int d, int node, int cur, in
         }
         if (ex_v && !(o.ex_father >> d & 1u))
             for (int l = 0; l < d; l++)
-                if (o.levels >> l & 1u) in_v = in_v && adjacent(a, uni(S->val[l]), v);
+                if (o.levels >> l & 1u) {
+                    const int x = uni(S->val[l]);
+                    in_v = adjacent(a, x, uni(hub_of(a, x)), v, in_v);
+                }
         int T = 0;
         int myoff = excl_scan(len, &T);
         nl = W;
@@ -1168,19 +1206,26 @@ __device__ __noinline__ void pair_leaf(const Ctx C, int d, int node, int cur, in
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                live[u] = live[u] && !equals_any(S, M.excl, d, c[u]) && !((M.excl >> d & 1u) && c[u] == w[u]);
+#pragma unroll
+                for (int i = 0; i < GATP_MAX_DEPTH; i++) {
+                    if (i >= n_skip) break;
+                    live[u] = live[u] && c[u] != skip[i];
+                }
+                live[u] = live[u] && !((M.excl >> d & 1u) && c[u] == w[u]);
                 e[u] = make_uint2(0, 0);
                 if (live[u] && c[u] < a.tab_size) e[u] = tab[c[u]];
-                t[u] = group_bound(S, o.groups, o.ngroups, d + 1, c[u]);
+                t[u] = t_lane ? group_bound(S, o.groups, o.ngroups, d + 1, c[u]) : t_all;
             }
             int cnt[U];
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 cnt[u] = 0;
-                for (int f = 0; f < d; f++) {
-                    if (!(in >> f & 1)) continue;
-                    const int x = uni(S->val[f]);
-                    if (live[u] && x < t[u] && ((o.ex_cand >> f & 1u) || adjacent(a, x, c[u]))) cnt[u]--;
+#pragma unroll
+                for (int i = 0; i < GATP_MAX_DEPTH; i++) {
+                    if (i >= n_less) break;
+                    const bool below = live[u] && less[i] < t[u];
+                    if (less_known >> i & 1u) cnt[u] -= below;
+                    else cnt[u] -= adjacent(a, less[i], less_hub[i], c[u], below);
                 }
                 if (live[u] && wex[u] && w[u] < t[u]) cnt[u]--;  // c lies in N(w)
             }
@@ -1253,7 +1298,7 @@ __device__ __forceinline__ void drop_pending(WaveState *S, int np, int ln) {
 // an edge whose sets outgrow the LDS buffers is handed alone to the HBM
 // launch and the walk goes on with the next edge; otherwise the whole task
 // is abandoned and re-run there.
-template <bool GS, bool KEEP>
+template <bool GS, bool KEEP, bool PAIR>
 __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e1) {
     const KArgs &a = C.a;
     const GatPlanDev &P = C.P;
@@ -1292,7 +1337,7 @@ __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e
             if (N.leaf) {
                 leaf<GS, KEEP>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node);
                 exhausted = true;
-            } else if (KEEP && N.pair && d >= 2) {
+            } else if (PAIR && N.pair && d >= 2) {
                 const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
                 if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
                 pair_leaf<GS>(C, d, node, cur, fh, can_split);
@@ -1342,7 +1387,7 @@ __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e
 // path are rebuilt (neither counted nor accounted again), then the walk
 // covers candidates [lo, hi) of its node and their subtrees only. A set that
 // outgrows its LDS buffer leaves S->abort set (the HBM launch re-runs it).
-template <bool GS, bool KEEP>
+template <bool GS, bool KEEP, bool PAIR>
 __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
     const KArgs &a = C.a;
     const GatPlanDev &P = C.P;
@@ -1390,7 +1435,7 @@ __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
         if (N.leaf) {
             leaf<GS, KEEP>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node);
             exhausted = true;
-        } else if (KEEP && N.pair) {
+        } else if (PAIR && N.pair) {
             const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
             if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
             pair_leaf<GS>(C, d, node, cur, fh, can_split);
@@ -1429,7 +1474,7 @@ __global__ void put_kargs(KArgs a, KArgs *dst) {
     if (threadIdx.x == 0) *dst = a;
 }
 
-template <bool GS, bool KEEP>
+template <bool GS, bool KEEP, bool PAIR>
 __device__ __forceinline__ void engine_main(const KArgs *__restrict__ ap, int wave_bytes, unsigned char *smem) {
     const KArgs &a = *ap;
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
@@ -1467,7 +1512,7 @@ __device__ __forceinline__ void engine_main(const KArgs *__restrict__ ap, int wa
             S->t0 = wall_clock64();
         }
         wsync();
-        run_task<GS, KEEP>(C, e0, e0 + a.chunk < a.e_hi ? e0 + a.chunk : a.e_hi);
+        run_task<GS, KEEP, PAIR>(C, e0, e0 + a.chunk < a.e_hi ? e0 + a.chunk : a.e_hi);
         wsync();
         if (S->abort) {
             if (GS) {
@@ -1500,7 +1545,7 @@ __device__ __forceinline__ void engine_main(const KArgs *__restrict__ ap, int wa
 // Subtask launches: list sub_mode (1 .. kSplitLevels: LDS buffers; then the
 // HBM list with HBM buffers). A subtask that outgrows LDS is copied to the
 // HBM list for the last launch.
-template <bool GS, bool KEEP>
+template <bool GS, bool KEEP, bool PAIR>
 __device__ __forceinline__ void engine_sub(const KArgs *__restrict__ ap, int wave_bytes, unsigned char *smem) {
     const KArgs &a = *ap;
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
@@ -1537,7 +1582,7 @@ __device__ __forceinline__ void engine_sub(const KArgs *__restrict__ ap, int wav
             S->t0 = wall_clock64();
         }
         wsync();
-        if (uni(g->lo) < uni(g->hi)) run_sub<GS, KEEP>(C, g);
+        if (uni(g->lo) < uni(g->hi)) run_sub<GS, KEEP, PAIR>(C, g);
         wsync();
         if (S->abort) {
             if (GS) {
@@ -1576,27 +1621,37 @@ __device__ __forceinline__ void engine_sub(const KArgs *__restrict__ ap, int wav
 
 // Kernels of plans that keep COUNT values in tables, and of those that do not
 // (and of W_alg accounting, which charges every value): the code of the tables
-// costs the others 8 % (C4 + P4 on a sparse random graph). Four waves per SIMD
-// are worth the spills around the calls.
+// costs the others 8 % (C4 + P4 on a sparse random graph), and that of
+// pair_leaf costs plans without pair nodes 15 % (house on Chung-Lu 65,536).
 template <bool GS>
 __global__ void __launch_bounds__(256, 4) engine_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
     extern __shared__ __align__(16) unsigned char smem[];
-    engine_main<GS, true>(ap, wave_bytes, smem);
+    engine_main<GS, true, false>(ap, wave_bytes, smem);
 }
 template <bool GS>
 __global__ void __launch_bounds__(256, 4) engine_sub_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
     extern __shared__ __align__(16) unsigned char smem[];
-    engine_sub<GS, true>(ap, wave_bytes, smem);
+    engine_sub<GS, true, false>(ap, wave_bytes, smem);
+}
+template <bool GS>
+__global__ void __launch_bounds__(256, 4) engine_pair_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    engine_main<GS, true, true>(ap, wave_bytes, smem);
+}
+template <bool GS>
+__global__ void __launch_bounds__(256, 4) engine_pair_sub_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    engine_sub<GS, true, true>(ap, wave_bytes, smem);
 }
 template <bool GS>
 __global__ void __launch_bounds__(256) engine_plain_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
     extern __shared__ __align__(16) unsigned char smem[];
-    engine_main<GS, false>(ap, wave_bytes, smem);
+    engine_main<GS, false, false>(ap, wave_bytes, smem);
 }
 template <bool GS>
 __global__ void __launch_bounds__(256) engine_plain_sub_kernel(const KArgs *__restrict__ ap, int wave_bytes) {
     extern __shared__ __align__(16) unsigned char smem[];
-    engine_sub<GS, false>(ap, wave_bytes, smem);
+    engine_sub<GS, false, false>(ap, wave_bytes, smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -2657,8 +2712,10 @@ struct DeviceGraph {
     // core bitmap of the clique store (core_n < 0: not built)
     unsigned *core = nullptr;
     int core_n = -1;
-    // hub bitmaps, built for the threshold hub_degree (0 = not built)
+    // hub bitmaps, built for the threshold hub_degree (0: the default)
+    bool hub_built = false;
     int hub_degree = 0;
+    int hub_full = INT_MAX;
     int n_hubs = 0;
     long long hub_words = 0;
     unsigned *hub_bits = nullptr;
@@ -2671,6 +2728,8 @@ struct DeviceGraph {
         hub_map = hub_vertex = nullptr;
         n_hubs = 0;
         hub_degree = 0;
+        hub_full = INT_MAX;
+        hub_built = false;
     }
     ~DeviceGraph() {
         free_hubs();
@@ -2751,30 +2810,50 @@ static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
     return GAT_OK;
 }
 
-// Neighbourhood bitmaps for every vertex of degree >= thr, most connected
-// first, within kHubBytes. Built once per (graph, threshold) outside the
+// Neighbourhood bitmaps, most connected vertices first, within kHubBytes: of
+// every vertex of degree >= the configured threshold, or by default of those of
+// degree >= kHubDegree and, within kHubMoreBytes, of further ones down to
+// hub_default(n). One word of a bitmap replaces a search of about log2(degree)
+// dependent reads, but in many sparse rows every word is a cache line of its
+// own. ms with a threshold of 256 / 64 / 16: house on Chung-Lu 65,536 22.0 /
+// 19.1 / 19.1, C5 on R-MAT s13 24.3 / 22.0 / 21.8, 21 patterns on R-MAT s10
+// 11.1 / 8.8 / 7.3, C4 + P4 on a random graph of 100,000 vertices and mean
+// degree 16 3.8 / 3.8 / 5.6. Built once per (graph, threshold) outside the
 // timed count, like the graph upload itself.
-constexpr double kHubBytes = 8.0 * (1ull << 30);
+constexpr double kHubBytes = 8.0 * (1ull << 30), kHubMoreBytes = 1.0 * (1ull << 30);
+constexpr int kHubDegree = 256;
+static int hub_default(int64_t n) { return n <= 16384 ? 16 : 64; }
 
+// thr: the configured threshold, 0 for the default. dg->hub_full: every vertex
+// from this degree on has a bitmap.
 static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr) {
-    if (dg->hub_degree == thr) return GAT_OK;
+    if (dg->hub_built && dg->hub_degree == thr) return GAT_OK;
     dg->free_hubs();
     const long long words = ((long long)g.n + 31) / 32;
     bool ordered = true;  // degree-ordered graphs keep hubs as a prefix
     for (int32_t v = 1; v < g.n && ordered; v++) ordered = g.deg(v) <= g.deg(v - 1);
+    const int least = thr ? thr : hub_default(g.n);
     std::vector<int32_t> hubs;
     if (ordered) {
         int32_t h = 0;
-        while (h < g.n && g.deg(h) >= thr) h++;
+        while (h < g.n && g.deg(h) >= least) h++;
         hubs.resize(h);
         std::iota(hubs.begin(), hubs.end(), 0);
     } else {
         for (int32_t v = 0; v < g.n; v++)
-            if (g.deg(v) >= thr) hubs.push_back(v);
+            if (g.deg(v) >= least) hubs.push_back(v);
         std::stable_sort(hubs.begin(), hubs.end(), [&](int32_t x, int32_t y) { return g.deg(x) > g.deg(y); });
     }
-    const long long max_hubs = (long long)(kHubBytes / (4.0 * std::max(1ll, words)));
-    if ((long long)hubs.size() > max_hubs) hubs.resize(max_hubs);
+    const size_t found = hubs.size();
+    const double row_bytes = 4.0 * std::max(1ll, words);
+    size_t always = hubs.size();  // rows that only kHubBytes limits
+    if (!thr)
+        always = std::partition_point(hubs.begin(), hubs.end(), [&](int32_t v) { return g.deg(v) >= kHubDegree; }) -
+                 hubs.begin();
+    hubs.resize(std::min(hubs.size(), std::max(always, (size_t)(kHubMoreBytes / row_bytes))));
+    hubs.resize(std::min(hubs.size(), (size_t)(kHubBytes / row_bytes)));
+    dg->hub_full = hubs.size() == found ? least : hubs.empty() ? INT_MAX : g.deg(hubs.back()) + 1;
+    dg->hub_built = true;
     dg->hub_degree = thr;
     dg->hub_words = words;
     if (hubs.empty()) return GAT_OK;
@@ -2862,6 +2941,7 @@ struct Launch {
     int chunk = 1;        // queue_chunk
     int64_t waves = 1;    // waves of the main launch
     bool edge_grain = false;  // the HBM launch takes single edges
+    bool pair = false;        // the plan has nodes swept with their leaf (GatNode::pair)
     bool heavy = false;   // clique: some vertex may have more than main_max neighbours below it
 };
 
@@ -2903,7 +2983,6 @@ static void fill_defaults(gat_kernel_config *c) {
     if (c->intersect_strategy < 0 || c->intersect_strategy > 4) c->intersect_strategy = 0;
     if (c->gallop_ratio <= 0) c->gallop_ratio = 32;
     if (c->search_linear_threshold < 0) c->search_linear_threshold = 0;
-    if (c->hub_degree == 0) c->hub_degree = 256;
     if (c->split_us == 0) c->split_us = kSplitUs;
 }
 
@@ -3027,18 +3106,22 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         d->ovf_cap = ovf_cap;
     }
     // A wave's LDS: its state (with the leaf counters the plan needs) and its
-    // set buffers. A neighbour list is staged for binary searches; from
-    // hub_degree entries on its bitmap serves, so its buffer ends there (house:
-    // 17.9 KB per wave with full buffers, 8 waves per CU; 10.6 KB and 14 with
-    // these). Configs are judged by the full size, whatever a plan needs of it.
+    // set buffers. A neighbour list is staged for binary searches; where
+    // every vertex of its length has a bitmap, that serves, so the buffer ends
+    // there (house: 17.9 KB per wave with full buffers, 8 waves per CU; 9 KB and
+    // 16 with these). Configs are judged by the full size, whatever a plan needs of it.
     const size_t full = (sizeof(gatk::WaveState) + size_t(pd.n_store) * cfg.slot_capacity * 4 + 15) / 16 * 16;
     if (full * cfg.block_waves > di.lds_per_block)
         GAT_FAIL(GAT_EINFEASIBLE, "config needs %zu B of LDS per workgroup (device allows %zu)",
                  full * cfg.block_waves, di.lds_per_block);
     const int state_bytes = int((sizeof(gatk::WaveState) -
                                  size_t(GATP_MAX_LEAF_OPS - pd.max_leaf_ops) * sizeof(int) * 64 + 15) / 16 * 16);
-    const int stage_cap = cfg.hub_degree > 0 ? std::min(cfg.slot_capacity, (cfg.hub_degree + 3) / 4 * 4)
-                                             : cfg.slot_capacity;
+    if (!clique && cfg.hub_degree >= 0) {
+        rc = ensure_hubs(g, d->dg.get(), cfg.hub_degree);
+        if (rc) return rc;
+    }
+    const int staged = !clique && cfg.hub_degree >= 0 ? std::min(cfg.slot_capacity, d->dg->hub_full) : cfg.slot_capacity;
+    const int stage_cap = std::min(cfg.slot_capacity, (staged + 3) / 4 * 4);
     long long store_off[GATP_MAX_STORE] = {}, entries = 0;
     for (int r = 0; r < pd.n_store; r++) {
         bool list = false;  // does some slot keep an intersection here?
@@ -3095,9 +3178,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         a.keep = d->keep;
     }
     a.split_ticks = split ? (long long)cfg.split_us * di.wall_khz / 1000 : 0;
-    if (!clique && cfg.hub_degree > 0) {
-        rc = ensure_hubs(g, d->dg.get(), cfg.hub_degree);
-        if (rc) return rc;
+    if (!clique && cfg.hub_degree >= 0) {
         a.hub_bits = d->dg->hub_bits;
         a.hub_map = d->dg->hub_map;
         a.hub_words = d->dg->hub_words;
@@ -3112,6 +3193,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     L->ao = a;
     L->waves = waves;
     L->edge_grain = edge_grain;
+    for (int i = 0; i < pd.n_nodes; i++) L->pair |= pd.nodes[i].pair != 0;
     L->ao.cap = std::max(1, g.max_deg);
     for (int r = 0; r < GATP_MAX_STORE; r++) L->ao.store_off[r] = (long long)r * L->ao.cap;
     L->ovf_grid = dim3(d->ovf_grid);
@@ -3280,8 +3362,15 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
     } else {
         a.tl_base = tl_take(waves);
         hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, a, d->dargs);
-        const bool keep = a.keep;
-        hipLaunchKernelGGL((keep ? gatk::engine_kernel<false> : gatk::engine_plain_kernel<false>), L.grid, L.block, L.lds, s, d->dargs, L.wave_bytes);
+        const bool pair = a.keep && L.pair;
+        auto pick = [&](auto plain, auto kept, auto paired) { return pair ? paired : a.keep ? kept : plain; };
+        const auto main_k = pick(gatk::engine_plain_kernel<false>, gatk::engine_kernel<false>, gatk::engine_pair_kernel<false>);
+        const auto sub_k = pick(gatk::engine_plain_sub_kernel<false>, gatk::engine_sub_kernel<false>,
+                                gatk::engine_pair_sub_kernel<false>);
+        const auto main_hbm_k = pick(gatk::engine_plain_kernel<true>, gatk::engine_kernel<true>, gatk::engine_pair_kernel<true>);
+        const auto sub_hbm_k = pick(gatk::engine_plain_sub_kernel<true>, gatk::engine_sub_kernel<true>,
+                                    gatk::engine_pair_sub_kernel<true>);
+        hipLaunchKernelGGL(main_k, L.grid, L.block, L.lds, s, d->dargs, L.wave_bytes);
         if (events) HIPCHECK(hipEventRecord(d->ev[1], s));
         if (a.split_ticks > 0)  // split subtasks, level by level, in LDS like the main launch
             for (int k = 1; k <= kLevels; k++) {
@@ -3294,7 +3383,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
                 sk.bytes = d->bytes + 1;
                 sk.tl_base = tl_take(waves);
                 hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, sk, d->dargs + k);
-                hipLaunchKernelGGL((keep ? gatk::engine_sub_kernel<false> : gatk::engine_plain_sub_kernel<false>), L.grid, L.block, L.lds, s, d->dargs + k,
+                hipLaunchKernelGGL(sub_k, L.grid, L.block, L.lds, s, d->dargs + k,
                                    L.wave_bytes);
             }
         ao.out_n = d->ovf_n + 8 + kLevels + 1;  // the HBM launch splits into the HBM list
@@ -3302,7 +3391,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
         ao.out_cap = 3 * kSubCap;
         ao.tl_base = tl_take((int)L.ovf_grid.x);
         hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, ao, d->dargs + kLevels + 1);
-        hipLaunchKernelGGL((keep ? gatk::engine_kernel<true> : gatk::engine_plain_kernel<true>), L.ovf_grid, dim3(64), L.ovf_lds, s, d->dargs + kLevels + 1,
+        hipLaunchKernelGGL(main_hbm_k, L.ovf_grid, dim3(64), L.ovf_lds, s, d->dargs + kLevels + 1,
                            L.ovf_wave_bytes);
         if (ao.split_ticks > 0) {
             gatk::KArgs sh = ao;
@@ -3313,7 +3402,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
             sh.out_n = nullptr;
             sh.tl_base = tl_take((int)L.ovf_grid.x);
             hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, sh, d->dargs + kLevels + 2);
-            hipLaunchKernelGGL((keep ? gatk::engine_sub_kernel<true> : gatk::engine_plain_sub_kernel<true>), L.ovf_grid, dim3(64), L.ovf_lds, s,
+            hipLaunchKernelGGL(sub_hbm_k, L.ovf_grid, dim3(64), L.ovf_lds, s,
                                d->dargs + kLevels + 2, L.ovf_wave_bytes);
         }
         if (events) HIPCHECK(hipEventRecord(d->ev[3], s));

@@ -155,7 +155,8 @@ typedef struct gat_kernel_config {
     int32_t hub_degree;       /* array store: vertices of at least this degree
                                  get a dense neighbourhood bitmap in HBM that
                                  replaces binary search in their lists
-                                 (0 = 256, negative = none)                   */
+                                 (0: 256, and within 1 GiB of bitmaps 64, or 16
+                                 up to 16,384 vertices; negative = none)      */
     int32_t split_us;         /* array store: a task still running after this
                                  many microseconds, once its launch's queue
                                  is drained, hands the unfinished rest of its
@@ -377,7 +378,8 @@ int gat_plan_timeline(const gat_plan *p, int64_t *out, int64_t cap, int64_t *n_o
  * the full length of the text (which may exceed cap) or an error code. */
 int gat_plan_describe(const gat_plan *p, char *buf, size_t cap);
 
-/* Default configuration the engine uses for zero fields. */
+/* Default configuration the engine uses for zero fields (a zero hub_degree
+ * also takes vertices below the 256 reported here, see there). */
 int gat_default_config(gat_kernel_config *out);
 
 /* ---- learned cost model (tuner) ------------------------------------- */
