@@ -850,18 +850,17 @@ __device__ __forceinline__ bool visit(const Ctx &C, const GatNode &N, int d, int
     return true;
 }
 
-// |N(c) ∩ father ∩ [0,t)| without the nex values ex, for the lanes in `need`
+// |N(c) ∩ father ∩ [0,t)|, father the set of slot f, without the nex values ex, for the lanes in `need`
 // (0 in the others): the (candidate, element) pairs of the wave's lanes form one
 // flattened index space. alen: the length of N(c) below t; *blen_out: that of
 // the father.
 template <bool GS>
-__device__ __forceinline__ int sweep_count(const Ctx &C, const GatOp &o, bool need, int c, long long ab, int alen, int t,
+__device__ __forceinline__ int sweep_count(const Ctx &C, int f, bool need, int c, long long ab, int alen, int t,
                                            const int *ex, int nex, int *blen_out) {
     const KArgs &a = C.a;
     WaveState *S = C.S;
     const int ln = C.ln;
     int cnt = 0;
-    const int f = o.father;
     int blen = 0;
     // Bg: father in HBM (a neighbour list, or any set in the overflow
     // launch); Bl: father in this wave's LDS buffers. hub_b: the
@@ -922,11 +921,11 @@ __device__ __forceinline__ int sweep_count(const Ctx &C, const GatOp &o, bool ne
 // The same from the candidate alone. (Out of line, this and pair_leaf cost C5
 // on R-MAT s13 a third: 19.9 against 14.7 ms.)
 template <bool GS>
-__device__ __forceinline__ int sweep_kept(const Ctx C, int op, bool need, int c, int t) {
+__device__ __forceinline__ int sweep_kept(const Ctx &C, int f, bool need, int c, int t) {
     const long long ab = need ? C.a.off[c] : 0;
     const int alen = need ? trunc_len(C.a, c, ab, (int)(C.a.off[c + 1] - ab), t) : 0;
     int blen;
-    return sweep_count<GS>(C, C.P.ops[op], need, c, ab, alen, t, nullptr, 0, &blen);
+    return sweep_count<GS>(C, f, need, c, ab, alen, t, nullptr, 0, &blen);
 }
 
 // The table of a KEEP_POOL op for the chosen v_0, v_1 or root edge, and the tag
@@ -961,7 +960,7 @@ __device__ __forceinline__ void leaf_exclusions(const Ctx &C, const GatNode &N, 
     WaveState *S = C.S;
     for (int k = 0; k < N.op_count; k++) {
         const GatOp &o = C.P.ops[N.op_begin + k];
-        if (o.kind != GATP_COUNT || o.keep == GATP_KEEP_NONE) continue;
+        if (o.kind != GATP_COUNT || o.keep == GATP_KEEP_NONE || o.keep == GATP_KEEP_SUM) continue;
         int in = 0;
         for (int f = 0; f < upto; f++) {
             if (!(o.excl >> f & 1u)) continue;
@@ -981,6 +980,84 @@ __device__ __forceinline__ void leaf_exclusions(const Ctx &C, const GatNode &N, 
     wsync();
 }
 
+// Does every table of the leaf node hold the value of c, the ci-th candidate?
+__device__ __forceinline__ bool leaf_known(const Ctx &C, const GatNode &N, int c, int ci) {
+    const KArgs &a = C.a;
+    bool known = true;
+    for (int k = 0; k < N.op_count; k++) {
+        const GatOp &o = C.P.ops[N.op_begin + k];
+        if (o.kind != GATP_COUNT) continue;
+        if (o.keep == GATP_KEEP_EDGE) known = known && a.edge_tab[o.table][C.S->sbeg[N.loop_slot] + ci] >= 0;
+        if (o.keep == GATP_KEEP_POOL) {
+            unsigned key = 0;  // pool_table without its cross-lane reads
+            if (o.key == 3) key = (unsigned)(C.S->sub_edge >= 0 ? C.S->sub_edge : C.S->rb + (C.S->f_cur[1] - 1));
+            else key = (unsigned)C.S->val[o.key == 2 ? 1 : 0];
+            if (c >= a.tab_size) return false;
+            const uint2 e = a.pool[((long long)o.table * a.pool_tables + key % a.pool_tables) * a.tab_size + c];
+            known = known && e.x == key + 1 && e.y >> 24 == a.epoch;
+        }
+    }
+    return known;
+}
+
+// The KEEP_SUM ops of leaf node N at depth d: their sums over all candidates
+// of the frame, added to the terms that use them.
+template <bool GS>
+__device__ __forceinline__ void leaf_sums(const Ctx &C, const GatNode &N, int d) {
+    const KArgs &a = C.a;
+    WaveState *S = C.S;
+    const int ln = C.ln;
+    for (int k = 0; k < N.op_count; k++) {
+        const GatOp &o = C.P.ops[N.op_begin + k];
+        if (o.kind != GATP_COUNT || o.keep != GATP_KEEP_SUM) continue;
+        const int v = uni(S->val[C.P.slots[N.loop_slot].depth]);  // v_j
+        const long long vb = a.off[v];
+        const int deg = (int)(a.off[v + 1] - vb), b = o.table ? v : INT_MAX;
+        const int t = uni(group_bound(S, o.groups, o.ngroups, d, 0));
+        int *edge = a.edge_tab[o.table] + vb;
+        const int len = uni(S->slen[o.father]);
+        unsigned long long sum = 0;
+        for (int base = 0; base < len; base += W) {
+            const int i = base + ln;
+            int x = INT_MAX;
+            if (i < len) x = with_slot<GS>(C, o.father, [&](auto p) { return p[i]; });
+            bool use = i < len && x < t;
+            for (int f = 0; f < d; f++)
+                if (o.excl >> f & 1u) use = use && x != S->val[f];
+            int cnt = 0;
+            const int pos = use ? lbound(a.adj + vb, deg, x) : 0;
+            if (use) cnt = edge[pos];
+            const bool need = use && cnt < 0;
+            if (ballot(need)) {
+                const int fresh = sweep_kept<GS>(C, N.loop_slot, need, x, b);
+                if (need) edge[pos] = cnt = fresh;
+            }
+            // candidates that are skipped or empty although they lie in N(v_j)
+            // below b: chosen vertices (each once)
+            for (int f = 0; f < d; f++) {
+                const unsigned out = N.excl | N.ap_levels;
+                if (!(out >> f & 1u)) continue;
+                const int y = uni(S->val[f]), hy = uni(hub_of(a, y));
+                bool once = y < b;
+                for (int h = 0; h < f; h++) once = once && !((out >> h & 1u) && S->val[h] == y);
+                once = adjacent(a, y, hy, v, once);
+                if (uni((int)once)) cnt -= adjacent(a, y, hy, x, use);
+            }
+            if (use) sum += (unsigned long long)(long long)cnt;
+        }
+        sum = wave_sum64(sum);
+        if (ln == 0)
+            for (int u = 0; u < N.term_count; u++) {
+                const GatTerm &T = C.P.terms[N.term_begin + u];
+                for (int q = 0; q < T.sub_count; q++) {
+                    const GatSub &sb = C.P.subs[T.sub_begin + q];
+                    if (C.P.vids[sb.vid].slot == o.slot) S->task_acc[T.pattern] += sum * (unsigned long long)(long long)sb.coef;
+                }
+            }
+    }
+    wsync();
+}
+
 // All candidates of a leaf frame, flattened across lanes.
 // With can_split, a wave that is due to split (want_split) hands the
 // batches after the current one to the next split launch.
@@ -992,6 +1069,10 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
     const int ln = C.ln;
     unsigned long long bytes = 0;
     if (KEEP) leaf_exclusions(C, N, d);
+    // Parts of a frame that was split have cur > 0; a frame handed on whole is
+    // left empty here. So the part with the first candidate adds the sums, and
+    // an empty frame has none.
+    if (KEEP && d >= 2 && cur == 0 && hi > 0) leaf_sums<GS>(C, N, d);
     for (int cb = cur; cb < hi; cb += W) {
         const int ci = cb + ln;
         int c = 0;
@@ -1004,9 +1085,11 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
         // for one donation record). With none left, the leaf's candidates
         // after the first go, in about as many parts as the chunk holds
         // budgets of work (at most 64), so that whole waves sweep their lists
-        // in parallel; the wave keeps the first candidate.
-        if (can_split && !(KEEP && N.kept) && hi - cb > 1 && queue_drained<GS>(a)) {
-            const long long lw = ci < hi ? a.off[c + 1] - a.off[c] : 0;
+        // in parallel; the wave keeps the first candidate. Candidates whose values
+        // are all in the tables are not swept.
+        if (can_split && hi - cb > 1 && queue_drained<GS>(a)) {
+            long long lw = 0;
+            if (ci < hi && !(KEEP && N.kept && leaf_known(C, N, c, ci))) lw = a.off[c + 1] - a.off[c];
             const long long tot = uni64((long long)wave_sum64((unsigned long long)lw));
             if (3 * tot > a.split_ticks && !split_shallowest<GS>(C, d - 1)) {
                 const long long budgets = 3 * tot / a.split_ticks + 1;
@@ -1030,6 +1113,10 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
             int *edge = nullptr;
             uint2 *slot = nullptr;
             unsigned tag = 0;
+            if (KEEP && o.keep == GATP_KEEP_SUM) {  // added by leaf_sums
+                S->leafcnt[o.leaf_idx][ln] = 0;
+                continue;
+            }
             if (KEEP && o.keep == GATP_KEEP_EDGE) edge = a.edge_tab[o.table];
             if (KEEP && edge) {
                 edge += S->sbeg[N.loop_slot] + ci;
@@ -1067,7 +1154,7 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
                 continue;
             }
             int blen = 0;
-            cnt = sweep_count<GS>(C, o, need, c, ab, alen, t, ex, nex, &blen);
+            cnt = sweep_count<GS>(C, o.father, need, c, ab, alen, t, ex, nex, &blen);
             if (a.account && live)
                 bytes += 4ull * (alen + blen) + 16ull + (C.P.slots[o.father].kind == GATP_ALIAS ? 16ull : 0ull);
             if (need && edge) *edge = cnt;
@@ -1234,7 +1321,7 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
                 const bool need = live[u] && (e[u].x != tag || e[u].y >> 24 != a.epoch);
                 int x = (int)(e[u].y & 0xffffffu);
                 if (ballot(need)) {
-                    const int fresh = sweep_kept<GS>(C, M.op_begin, need, c[u], t[u]);
+                    const int fresh = sweep_kept<GS>(C, o.father, need, c[u], t[u]);
                     if (need) {
                         x = fresh;
                         if (c[u] < a.tab_size) tab[c[u]] = make_uint2(tag, (unsigned)fresh | a.epoch << 24);

@@ -300,6 +300,33 @@ void keep_count(const Compiler &C, int node, const HSlot &s, GatOp *o, std::vect
     o->key = key;
 }
 
+// Turns leaf COUNT `o` of node `node` (device node g) into a KEEP_SUM where its
+// loop set, father and terms allow it.
+void sum_count(const Compiler &C, int node, const GatPlanDev &d, const GatNode &g, GatOp *o) {
+    const HSlot &f = C.slots[o->father], &loop = C.slots[g.loop_slot];
+    if (g.depth < 2 || f.kind != GATP_LIST || loop.data.size() != 1) return;
+    const int j = loop.data[0];
+    Mask data = 0;
+    for (int l : f.data) data |= Mask(1u << l);
+    if (!(data >> j & 1u) || (g.bound && g.bound != 1u << j)) return;
+    for (int k = 0; k < o->ngroups; k++)
+        if (o->groups[k] >> g.depth & 1u) return;  // the truncation must not depend on c
+    for (int n = node; n >= 0; n = C.nodes[n].parent)
+        if (data >> C.nodes[n].depth & 1u && C.nodes[n].A) return;  // see keep_count
+    for (int t = g.term_begin; t < g.term_begin + g.term_count; t++) {
+        int first = 0;  // of the factors of one product
+        for (int k = 0; k < d.terms[t].sub_count; k++) {
+            const GatSub &sb = d.subs[d.terms[t].sub_begin + k];
+            const GatVid &v = d.vids[sb.vid];
+            if (v.slot == o->slot && (v.mode != GATP_VID_COUNT || k != first || !sb.flag)) return;
+            if (sb.flag) first = k + 1;
+        }
+    }
+    o->keep = GATP_KEEP_SUM;
+    o->table = g.bound ? 1 : 0;
+    o->levels = data;
+}
+
 }  // namespace
 
 int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOptions &opt, CompiledPlan *out) {
@@ -587,8 +614,6 @@ int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOption
             if ((s.kind == GATP_COUNT || s.kind == GATP_ALIAS) && g.leaf) o.leaf_idx = gs.leaf_idx = int8_t(leafc++);
             if (s.kind == GATP_COUNT && g.leaf && s.father >= 0) {
                 keep_count(C, order[ii], s, &o, &tables);
-                if (o.keep == GATP_KEEP_NONE) g.kept = 0;
-                if (o.keep == GATP_KEEP_EDGE) d.edge_tables |= 1 << o.table;
                 if (o.keep == GATP_KEEP_POOL && o.key == 3) d.key_edges = 1;
             }
         }
@@ -621,6 +646,17 @@ int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOption
             }
         }
         g.term_count = int16_t(nterms - g.term_begin);
+    }
+    for (size_t i = 1; i < order.size(); i++) {
+        GatNode &g = d.nodes[i];
+        if (!g.leaf) continue;
+        for (int k = g.op_begin; k < g.op_begin + g.op_count; k++) {
+            GatOp &o = d.ops[k];
+            if (o.kind != GATP_COUNT || o.father < 0) continue;
+            if (o.keep == GATP_KEEP_NONE) sum_count(C, order[i], d, g, &o);
+            if (o.keep == GATP_KEEP_NONE) g.kept = 0;
+            if (o.keep == GATP_KEEP_EDGE || o.keep == GATP_KEEP_SUM) d.edge_tables |= 1 << o.table;
+        }
     }
     for (size_t i = 1; i < order.size(); i++) {
         GatNode &g = d.nodes[i];

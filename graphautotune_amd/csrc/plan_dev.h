@@ -27,7 +27,11 @@ enum { GATP_ALIAS = 0, GATP_LIST = 1, GATP_COUNT = 2 };
 // KEEP_POOL: the father and the truncation depend on v_0, on v_1 or on the root
 // edge (v_0, v_1) only, which stay fixed while the parent level's vertex
 // changes: a table over c for each of them, in a pool all waves share.
-enum { GATP_KEEP_NONE = 0, GATP_KEEP_EDGE = 1, GATP_KEEP_POOL = 2 };
+// KEEP_SUM: every term uses the value alone (no product), so only its sum over
+// the leaf's candidates matters. With c in N(v_j), c < b, and a father F inside
+// N(v_j), sum_c |N(c) ∩ F| = sum_{x in F} |N(x) ∩ N(v_j) ∩ [0,b)|: a KEEP_EDGE
+// value of the edge (v_j, x) for each x in F, once per leaf frame.
+enum { GATP_KEEP_NONE = 0, GATP_KEEP_EDGE = 1, GATP_KEEP_POOL = 2, GATP_KEEP_SUM = 3 };
 #define GATP_MAX_TABLES 8
 enum { GATP_VID_COUNT = 0, GATP_VID_LIST_REF = 1, GATP_VID_LIST_BOUNDED = 2 };
 
@@ -43,7 +47,7 @@ typedef struct GatOp {
     // COUNT at a leaf: how |N(c) ∩ father| of an unchanged father is kept
     // within a count instead of being recomputed for every path (GATP_KEEP_*)
     int8_t keep;
-    int8_t table;      // KEEP_EDGE: truncation (bit 0: t <= v_j, bit 1: t <= c); KEEP_POOL: pool index
+    int8_t table;      // KEEP_EDGE, KEEP_SUM: truncation (bit 0: t <= v_j, bit 1: t <= c); KEEP_POOL: pool index
     uint8_t key;       // KEEP_POOL: levels the value depends on besides c (1: v_0, 2: v_1, 3: the edge)
     uint8_t ex_father; // excluded levels whose vertex is known to lie in the father's untruncated set
     uint8_t levels;    // levels of the father's prefix
