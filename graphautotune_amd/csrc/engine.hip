@@ -1554,11 +1554,18 @@ __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
 }
 
 // The array-store kernels read their arguments from device memory (written
-// by put_kargs just before the launch): the walk hands a reference to them
+// by put_kargs before the count's launches): the walk hands a reference to them
 // to out-of-line helpers, and a reference to a by-value kernel argument
 // would make every lane copy the whole record to scratch first.
-__global__ void put_kargs(KArgs a, KArgs *dst) {
-    if (threadIdx.x == 0) *dst = a;
+constexpr int kArgSlots = kSplitLevels + 3;  // the main launch, the LDS subtask levels, the HBM launch and its subtasks
+struct KArgsSet {
+    KArgs a[kArgSlots];
+};
+static_assert(sizeof(KArgsSet) <= 4000, "kernel arguments");
+__global__ void put_kargs(KArgsSet set, KArgsSet *dst) {
+    const int *src = reinterpret_cast<const int *>(&set);
+    for (int i = threadIdx.x; i < (int)(sizeof(KArgsSet) / sizeof(int)); i += blockDim.x)
+        reinterpret_cast<int *>(dst)[i] = src[i];
 }
 
 template <bool GS, bool KEEP, bool PAIR>
@@ -2830,11 +2837,11 @@ struct DeviceGraph {
 struct PlanDevice {
     hipStream_t stream = nullptr;
     GatPlanDev *plan = nullptr;
-    unsigned long long *counts = nullptr, *queue = nullptr, *ovf_n = nullptr, *bytes = nullptr;
-    unsigned int *err = nullptr;
+    unsigned long long *ctl = nullptr;      // control words (kCtl*)
+    unsigned long long *result = nullptr;   // the first kCtlResult of them in pinned host memory
     long long *ovf = nullptr;
     gatk::SplitTask *subs = nullptr;  // split subtasks (array store)
-    gatk::KArgs *dargs = nullptr;     // arguments of the array-store launches of a count
+    gatk::KArgsSet *dargs = nullptr;  // arguments of the array-store launches of a count
     long long *tl = nullptr;          // timeline records of the last GAT_FLAG_TIMELINE count
     int tl_n = 0;                     // records that count reserved (0: none)
     int *tier[gatk::CTIERS] = {};  // clique vertices of the workgroup tiers
@@ -2866,12 +2873,12 @@ void destroy_plan_device(PlanDevice *d) {
     if (d->graph) (void)hipGraphDestroy(d->graph);
     for (auto &e : d->ev)
         if (e) (void)hipEventDestroy(e);
-    for (void *p : {(void *)d->plan, (void *)d->dargs, (void *)d->tl, (void *)d->counts, (void *)d->queue, (void *)d->ovf_n, (void *)d->bytes,
-                    (void *)d->err, (void *)d->ovf, (void *)d->subs, (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2], (void *)d->tier[3],
+    for (void *p : {(void *)d->plan, (void *)d->dargs, (void *)d->tl, (void *)d->ctl, (void *)d->ovf, (void *)d->subs, (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2], (void *)d->tier[3],
                     (void *)d->gstore, (void *)d->edge_tab[0], (void *)d->edge_tab[1], (void *)d->edge_tab[2],
                     (void *)d->edge_tab[3], (void *)d->pool, (void *)d->grows,
                     (void *)d->goff})
         if (p) (void)hipFree(p);
+    if (d->result) (void)hipHostFree(d->result);
     if (d->stream) (void)hipStreamDestroy(d->stream);
     delete d;
 }
@@ -2999,12 +3006,15 @@ static int ensure_core(const Graph &g, DeviceGraph *dg) {
 constexpr long long kSubCap = 1ll << 20;
 constexpr int kLevels = gatk::kSplitLevels;
 constexpr int kSplitUs = 2000;
-// queue words of a plan: 16 of the clique store, the array store's heads, and
-// its drained flags
-constexpr int kQueueAlloc = 16 + gatk::kQueueWords + gatk::kQueues;
-// device argument records of one array-store count: the main launch, the
-// LDS subtask levels, the HBM launch and the HBM subtask launch
-constexpr int kArgSlots = kLevels + 3;
+// Control words of a count, one allocation: first what the host reads back (the
+// copies of the counts, 16 list sizes, 4 W_alg sums, the error flags), then the
+// clique store's queues, and for the array store the queue heads and drained
+// flags. One launch clears them and one copy into pinned memory reads them: five
+// fills and four copies were 50 us of a small count.
+constexpr int kCtlOvf = GATP_MAX_TERMS * gatk::kCountCopies, kCtlBytes = kCtlOvf + 16, kCtlErr = kCtlBytes + 4;
+constexpr int kCtlResult = kCtlErr + 1, kCtlQueue = (kCtlResult + 15) / 16 * 16, kCtlHeads = kCtlQueue + 16;
+constexpr int kCtlDrained = kCtlHeads + gatk::kQueueWords, kCtlWords = kCtlDrained + gatk::kQueues;
+static_assert(kCtlQueue % 16 == 0 && kCtlHeads % 16 == 0, "queue heads on cache lines of their own");
 // timeline capacity (records of gatk::kTlFields int64 each)
 constexpr int kTlCap = 1 << 15;
 
@@ -3028,6 +3038,7 @@ struct Launch {
     int chunk = 1;        // queue_chunk
     int64_t waves = 1;    // waves of the main launch
     bool edge_grain = false;  // the HBM launch takes single edges
+    bool may_overflow = true; // some intersection may outgrow its LDS buffer
     bool pair = false;        // the plan has nodes swept with their leaf (GatNode::pair)
     bool heavy = false;   // clique: some vertex may have more than main_max neighbours below it
 };
@@ -3152,12 +3163,9 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         HIPCHECK(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
         HIPCHECK(hipMalloc(&d->plan, sizeof(GatPlanDev)));
         HIPCHECK(hipMemcpy(d->plan, &pd, sizeof(GatPlanDev), hipMemcpyHostToDevice));
-        HIPCHECK(hipMalloc(&d->counts, sizeof(unsigned long long) * GATP_MAX_TERMS * gatk::kCountCopies));
-        HIPCHECK(hipMalloc(&d->queue, sizeof(unsigned long long) * kQueueAlloc));
-        HIPCHECK(hipMalloc(&d->ovf_n, sizeof(unsigned long long) * 16));
-        HIPCHECK(hipMalloc(&d->bytes, sizeof(unsigned long long) * 4));
-        HIPCHECK(hipMalloc(&d->err, sizeof(unsigned int) * 2));
-        HIPCHECK(hipMalloc(&d->dargs, sizeof(gatk::KArgs) * kArgSlots));
+        HIPCHECK(hipMalloc(&d->ctl, sizeof(unsigned long long) * kCtlWords));
+        HIPCHECK(hipHostMalloc((void **)&d->result, sizeof(unsigned long long) * kCtlResult, hipHostMallocDefault));
+        HIPCHECK(hipMalloc(&d->dargs, sizeof(gatk::KArgsSet)));
         for (auto &e : d->ev) HIPCHECK(hipEventCreate(&e));
     }
     PlanDevice *d = p->dev;
@@ -3227,15 +3235,15 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     a.e_lo = 0;
     a.e_hi = g.m;
     a.plan = d->plan;
-    a.counts = d->counts;
-    a.queue = d->queue + 16;
-    a.drained = reinterpret_cast<unsigned *>(d->queue + 16 + gatk::kQueueWords);
+    a.counts = d->ctl;
+    a.queue = d->ctl + kCtlHeads;
+    a.drained = reinterpret_cast<unsigned *>(d->ctl + kCtlDrained);
     a.ovf = d->ovf;
-    a.ovf_n = d->ovf_n;
+    a.ovf_n = d->ctl + kCtlOvf;
     a.ovf_cap = d->ovf_cap;
     a.gstore = d->gstore;
-    a.bytes = d->bytes;
-    a.err = d->err;
+    a.bytes = d->ctl + kCtlBytes;
+    a.err = reinterpret_cast<unsigned *>(d->ctl + kCtlErr);
     a.cap = cfg.slot_capacity;
     a.stage_cap = stage_cap;
     a.state_bytes = state_bytes;
@@ -3249,10 +3257,10 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     a.sub_mode = 0;
     a.subs = d->subs;
     a.in_n = nullptr;
-    a.out_n = d->ovf_n + 8 + 1;  // the main launch splits into level 1
+    a.out_n = a.ovf_n + 8 + 1;  // the main launch splits into level 1
     a.in_base = a.out_base = 0;
     a.in_cap = a.out_cap = kSubCap;
-    a.sovf_n = d->ovf_n + 8 + kLevels + 1;
+    a.sovf_n = a.ovf_n + 8 + kLevels + 1;
     a.sovf_base = kLevels * kSubCap;
     a.sovf_cap = 3 * kSubCap;
     if (!clique) {
@@ -3280,6 +3288,9 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     L->ao = a;
     L->waves = waves;
     L->edge_grain = edge_grain;
+    bool lists = false;
+    for (int i = 0; i < pd.n_ops; i++) lists |= pd.ops[i].kind == GATP_LIST;
+    L->may_overflow = lists && g.max_deg > cfg.slot_capacity;
     for (int i = 0; i < pd.n_nodes; i++) L->pair |= pd.nodes[i].pair != 0;
     L->ao.cap = std::max(1, g.max_deg);
     for (int r = 0; r < GATP_MAX_STORE; r++) L->ao.store_off[r] = (long long)r * L->ao.cap;
@@ -3311,7 +3322,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         c.counts = a.counts;
         for (int k = 0; k < 8; k++) c.pat_of_k[k] = p->cp.clique_pattern[k];
         c.kmax = 31 - __builtin_clz(p->cp.clique_ks);
-        c.queue = d->queue;
+        c.queue = d->ctl + kCtlQueue;
         c.ovf_n = a.ovf_n;
         c.bytes = a.bytes;
         c.err = a.err;
@@ -3386,22 +3397,18 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
                            (long long)gatk::kTlFields * kTlCap, ~0ull);
         tl = d->tl;
     }
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(4), dim3(256), 0, s, d->counts,
-                       (long long)GATP_MAX_TERMS * gatk::kCountCopies, 0ull);
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(8), dim3(256), 0, s, d->queue, (long long)kQueueAlloc, 0ull);
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->ovf_n, 16ll, 0ull);
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, d->bytes, 4ll, 0ull);
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(1), dim3(64), 0, s, (unsigned long long *)d->err, 1ll, 0ull);
+    hipLaunchKernelGGL(gatk::fill_u64, dim3(8), dim3(256), 0, s, d->ctl, (long long)(L.clique ? kCtlHeads : kCtlWords),
+                       0ull);
     gatk::KArgs a = L.a, ao = L.ao;
     a.account = ao.account = account ? 1 : 0;
     if (account) {  // W_alg is accumulated where the values are computed
         a.keep = ao.keep = 0;
     }
     if (!L.clique && a.keep && a.pool) {
-        // epochs 1 .. 254 for counts in turn; replays of a captured count share
-        // one, so it clears the pool itself, as does the first count of a turn
+        // epochs 1 .. 254 for counts in turn, with the pool cleared before the
+        // first; the replays of a captured count share one, so each clears it
         const bool clear = !events || d->epoch >= 254;
-        d->epoch = clear ? 1 : d->epoch + 1;
+        if (events) d->epoch = clear ? 1 : d->epoch + 1;
         a.epoch = ao.epoch = events ? d->epoch : 255;
         if (clear)
             hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, s, (unsigned long long *)d->pool,
@@ -3412,7 +3419,7 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
             hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, s, (unsigned long long *)a.edge_tab[k],
                                (a.m + 1) / 2, ~0ull);
     a.tl = ao.tl = tl;
-    ao.bytes = d->bytes + 1;  // second launch: its own W_alg counter
+    ao.bytes = a.bytes + 1;  // second launch: its own W_alg counter
     const int waves = (int)(L.grid.x * (L.block.x / 64));
     if (events) HIPCHECK(hipEventRecord(d->ev[0], s));
     gatk::CArgs c = L.ca;
@@ -3428,11 +3435,11 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
             c.tl_base = tl_take(waves);
             hipLaunchKernelGGL(gatk::clique_kernel<T>, L.grid, L.block, L.clique_lds, s, c);
             if (events) HIPCHECK(hipEventRecord(d->ev[1], s));
-            c.bytes = d->bytes + 1;  // tiers 0 and 1: their own W_alg counter
+            c.bytes = a.bytes + 1;  // tiers 0 and 1: their own W_alg counter
             launch_tier<T, gatk::CT0W, 0, gatk::CNW0>(L, c, s, tl_take);
             launch_tier<T, gatk::CT1W, 1, gatk::CNW1>(L, c, s, tl_take);
             if (events) HIPCHECK(hipEventRecord(d->ev[3], s));
-            c.bytes = d->bytes + 2;  // tiers 2 and 3
+            c.bytes = a.bytes + 2;  // tiers 2 and 3
             launch_tier<T, gatk::CT2W, 2, gatk::CNW2>(L, c, s, tl_take);
             if (L.tier_grid[3].x) {
                 c.tl_base = tl_take((int)L.tier_grid[3].x);
@@ -3447,8 +3454,6 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
                                    : run(std::integral_constant<int, 3>{});
         if (rc) return rc;
     } else {
-        a.tl_base = tl_take(waves);
-        hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, a, d->dargs);
         const bool pair = a.keep && L.pair;
         auto pick = [&](auto plain, auto kept, auto paired) { return pair ? paired : a.keep ? kept : plain; };
         const auto main_k = pick(gatk::engine_plain_kernel<false>, gatk::engine_kernel<false>, gatk::engine_pair_kernel<false>);
@@ -3457,40 +3462,43 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
         const auto main_hbm_k = pick(gatk::engine_plain_kernel<true>, gatk::engine_kernel<true>, gatk::engine_pair_kernel<true>);
         const auto sub_hbm_k = pick(gatk::engine_plain_sub_kernel<true>, gatk::engine_sub_kernel<true>,
                                     gatk::engine_pair_sub_kernel<true>);
-        hipLaunchKernelGGL(main_k, L.grid, L.block, L.lds, s, d->dargs, L.wave_bytes);
-        if (events) HIPCHECK(hipEventRecord(d->ev[1], s));
-        if (a.split_ticks > 0)  // split subtasks, level by level, in LDS like the main launch
-            for (int k = 1; k <= kLevels; k++) {
-                gatk::KArgs sk = a;
-                sk.sub_mode = k;
-                sk.in_n = d->ovf_n + 8 + k;
-                sk.in_base = (k - 1) * kSubCap;
-                sk.out_n = k < kLevels ? d->ovf_n + 8 + k + 1 : nullptr;  // the last level does not split
-                sk.out_base = k * kSubCap;
-                sk.bytes = d->bytes + 1;
-                sk.tl_base = tl_take(waves);
-                hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, sk, d->dargs + k);
-                hipLaunchKernelGGL(sub_k, L.grid, L.block, L.lds, s, d->dargs + k,
-                                   L.wave_bytes);
-            }
-        ao.out_n = d->ovf_n + 8 + kLevels + 1;  // the HBM launch splits into the HBM list
+        const bool split = a.split_ticks > 0;
+        gatk::KArgsSet set;
+        a.tl_base = tl_take(waves);
+        set.a[0] = a;
+        for (int k = 1; k <= kLevels; k++) {
+            gatk::KArgs &sk = set.a[k] = a;
+            sk.sub_mode = k;
+            sk.in_n = a.ovf_n + 8 + k;
+            sk.in_base = (k - 1) * kSubCap;
+            sk.out_n = k < kLevels ? a.ovf_n + 8 + k + 1 : nullptr;  // the last level does not split
+            sk.out_base = k * kSubCap;
+            sk.bytes = a.bytes + 1;
+            sk.tl_base = split ? tl_take(waves) : 0;
+        }
+        ao.out_n = a.ovf_n + 8 + kLevels + 1;  // the HBM launch splits into the HBM list
         ao.out_base = kLevels * kSubCap;
         ao.out_cap = 3 * kSubCap;
         ao.tl_base = tl_take((int)L.ovf_grid.x);
-        hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, ao, d->dargs + kLevels + 1);
-        hipLaunchKernelGGL(main_hbm_k, L.ovf_grid, dim3(64), L.ovf_lds, s, d->dargs + kLevels + 1,
-                           L.ovf_wave_bytes);
-        if (ao.split_ticks > 0) {
-            gatk::KArgs sh = ao;
-            sh.sub_mode = kLevels + 1;  // HBM buffers, no further splitting
-            sh.in_n = d->ovf_n + 8 + kLevels + 1;
-            sh.in_base = kLevels * kSubCap;
-            sh.in_cap = 3 * kSubCap;
-            sh.out_n = nullptr;
-            sh.tl_base = tl_take((int)L.ovf_grid.x);
-            hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(64), 0, s, sh, d->dargs + kLevels + 2);
-            hipLaunchKernelGGL(sub_hbm_k, L.ovf_grid, dim3(64), L.ovf_lds, s,
-                               d->dargs + kLevels + 2, L.ovf_wave_bytes);
+        set.a[kLevels + 1] = ao;
+        gatk::KArgs &sh = set.a[kLevels + 2] = ao;
+        sh.sub_mode = kLevels + 1;  // HBM buffers, no further splitting
+        sh.in_n = a.ovf_n + 8 + kLevels + 1;
+        sh.in_base = kLevels * kSubCap;
+        sh.in_cap = 3 * kSubCap;
+        sh.out_n = nullptr;
+        sh.tl_base = split ? tl_take((int)L.ovf_grid.x) : 0;
+        hipLaunchKernelGGL(gatk::put_kargs, dim3(1), dim3(256), 0, s, set, d->dargs);
+        const gatk::KArgs *args = d->dargs->a;
+        hipLaunchKernelGGL(main_k, L.grid, L.block, L.lds, s, args, L.wave_bytes);
+        if (events) HIPCHECK(hipEventRecord(d->ev[1], s));
+        for (int k = 1; k <= kLevels && split; k++)  // split subtasks, level by level, in LDS like the main launch
+            hipLaunchKernelGGL(sub_k, L.grid, L.block, L.lds, s, args + k, L.wave_bytes);
+        if (L.may_overflow) {
+            hipLaunchKernelGGL(main_hbm_k, L.ovf_grid, dim3(64), L.ovf_lds, s, args + kLevels + 1, L.ovf_wave_bytes);
+            if (split)
+                hipLaunchKernelGGL(sub_hbm_k, L.ovf_grid, dim3(64), L.ovf_lds, s, args + kLevels + 2,
+                                   L.ovf_wave_bytes);
         }
         if (events) HIPCHECK(hipEventRecord(d->ev[3], s));
     }
@@ -3506,14 +3514,12 @@ static int finish(gat_plan *p, const Launch &L, uint64_t *counts_out, gat_count_
                   bool raw_sums = false) {
     PlanDevice *d = p->dev;
     const int np = p->cp.dev.n_patterns;
-    unsigned long long raw[GATP_MAX_TERMS] = {}, ovf[16] = {}, bytes[3] = {0, 0, 0};
-    unsigned long long copies[gatk::kCountCopies * GATP_MAX_TERMS];
-    unsigned int err = 0;
-    HIPCHECK(hipMemcpyAsync(copies, d->counts, sizeof(copies), hipMemcpyDeviceToHost, d->stream));
-    HIPCHECK(hipMemcpyAsync(ovf, d->ovf_n, sizeof(ovf), hipMemcpyDeviceToHost, d->stream));
-    HIPCHECK(hipMemcpyAsync(bytes, d->bytes, sizeof(bytes), hipMemcpyDeviceToHost, d->stream));
-    HIPCHECK(hipMemcpyAsync(&err, d->err, sizeof(err), hipMemcpyDeviceToHost, d->stream));
+    unsigned long long raw[GATP_MAX_TERMS] = {};
+    HIPCHECK(hipMemcpyAsync(d->result, d->ctl, sizeof(unsigned long long) * kCtlResult, hipMemcpyDeviceToHost,
+                            d->stream));
     HIPCHECK(hipStreamSynchronize(d->stream));
+    const unsigned long long *copies = d->result, *ovf = copies + kCtlOvf, *bytes = copies + kCtlBytes;
+    const unsigned int err = (unsigned)copies[kCtlErr];
     for (int c = 0; c < gatk::kCountCopies; c++)
         for (int i = 0; i < np; i++) raw[i] += copies[c * GATP_MAX_TERMS + i];
     // flags 2 and 4: a device work list (overflow tasks, subtasks, clique
@@ -3758,12 +3764,11 @@ extern "C" int gat_count_cliques_noalloc(const int64_t *d_offsets, const int32_t
         launch_tier<0, gatk::CT2W, 2, gatk::CNW2>(L, c, s, no_tl);
     }
     HIPCHECK(hipGetLastError());
-    unsigned long long copies[gatk::kCountCopies * GATP_MAX_TERMS], raw[8] = {}, heavy = 0;
-    unsigned int err = 0;
-    HIPCHECK(hipMemcpyAsync(copies, c.counts, sizeof(copies), hipMemcpyDeviceToHost, s));
-    HIPCHECK(hipMemcpyAsync(&heavy, h + 24 + 5, sizeof(heavy), hipMemcpyDeviceToHost, s));
-    HIPCHECK(hipMemcpyAsync(&err, h + 44, sizeof(err), hipMemcpyDeviceToHost, s));
+    unsigned long long head[kNaHead], raw[8] = {};
+    HIPCHECK(hipMemcpyAsync(head, h, sizeof(head), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
+    const unsigned long long *copies = head + 64, heavy = head[24 + 5];
+    const unsigned int err = (unsigned)head[44];
     if (err & 16u)
         GAT_FAIL(GAT_ELIMIT, "a vertex has more than %d neighbours below it; the allocation-free count has no HBM tier",
                  c.lds_dmax);
