@@ -1796,9 +1796,9 @@ __device__ __forceinline__ int clique_parts(int kmax, unsigned long long vertice
 // Waves per workgroup: enough to share one vertex's work, few enough that
 // the workgroups of a CU (bounded by LDS, 11, 39 and 160 KB each, and by registers) overlap
 // one's row build with another's counting.
-constexpr int CNW0 = 4, CNW1 = 4, CNW2 = 12, CNW3 = 16;
+constexpr int CNW0 = 4, CNW1 = 4, CNW2 = 8, CNW3 = 16;
 // Waves per SIMD the tiers' registers leave room for.
-constexpr int clique_occupancy(int tier) { return tier == 0 ? 4 : 3; }
+constexpr int clique_occupancy(int tier) { return tier == 0 ? 4 : tier == 1 ? 3 : 2; }
 // Words per bit row of a list of d vertices: enough for d bits, rounded up
 // to an odd number so that lanes reading the same word of different rows
 // hit different LDS banks (an even stride folds them onto a few banks).
@@ -1986,8 +1986,10 @@ __device__ __forceinline__ unsigned long long vtx_rows(const CArgs &a, LP L, int
 // 16 cycles and about half as many cycles of vector instructions. R-MAT s20,
 // K4 + K5, tiers 0 to 2: 28.0 ms with the pair walk and swept rows, 10.6 ms
 // with this (rows 2.6 ms of it); K6 on R-MAT s16: 840 ms against 5.4 ms. The
-// tiles in registers are what counts: two row tiles instead of four in tier 1
-// cost 2 ms, because every column tile is read and unpacked once per group.
+// tiles in registers are what counts, because every column tile is read and
+// unpacked once per group: two row tiles instead of four cost 2 ms in tier 1
+// and 0.25 ms in tier 2 (in spite of 12 waves per CU instead of 8); eight in
+// tier 1, with two waves per SIMD instead of three, cost 1 ms.
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kFp4 = 4;  // operand format of the instruction: 4-bit float
@@ -2554,7 +2556,7 @@ __global__ void __launch_bounds__(64 * NW, clique_occupancy(TIER)) clique_block_
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
     constexpr int lcap = 32 * MW;
     constexpr int KC = MW / 4;            // chunks of 128 positions
-    constexpr int RT = MW <= 16 ? 4 : 2;  // row tiles held at once (registers)
+    constexpr int RT = 4;  // row tiles held at once
     unsigned *rows = reinterpret_cast<unsigned *>(smem);
     int *L = reinterpret_cast<int *>(rows + tier_row_words(MW));
     unsigned *buf = reinterpret_cast<unsigned *>(L) + wid * 2 * CCOLS;
