@@ -43,8 +43,12 @@ HBM_PEAK_GBPS = 8000.0
 # (two wave64 instructions per CU per cycle; rocprofv3 counts the clique
 # tier-0 launch at 1.05 per CU-cycle, above what 16-lane SIMDs could issue).
 VALU_PEAK_TOPS = 256 * 4 * 32 * 2.4e9 / 1e12
-CLIQUE_KERNELS = ("gatk::clique_kernel<0>", "gatk::clique_block_kernel<16, true, 0, 8, 0>",
-                  "gatk::clique_block_kernel<32, true, 1, 16, 0>")
+CLIQUE_KERNELS = ("gatk::clique_kernel<0>", "gatk::clique_block_kernel<8, 0, 4, 0>",
+                  "gatk::clique_block_kernel<16, 1, 4, 0>", "gatk::clique_block_kernel<32, 2, 8, 0>")
+# launch groups of the clique store's count, the heaviest kernel first: the main
+# launch, tiers 0 and 1 (second_kernel_ms), tier 2 and the tier in memory
+CLIQUE_GROUPS = {CLIQUE_KERNELS[0]: (CLIQUE_KERNELS[0],), "tiers 0 and 1": (CLIQUE_KERNELS[2], CLIQUE_KERNELS[1]),
+                 "tiers 2 and 3": (CLIQUE_KERNELS[3], "gatk::clique_hbm_kernel<0>")}
 
 
 def load_profile(name, cfg):
@@ -60,8 +64,9 @@ def load_profile(name, cfg):
 
 def clique_roofline(kernel, ms, walg, prof):
     """Bitmap clique store: its operands are bit rows in LDS, its work is
-    integer bit operations on the vector ALU (rocprofv3 counters in the
-    profile give the VALU issue rate, lane use and LDS use beside it).
+    integer bit operations, priced against the vector ALU (the tiers count
+    them on the matrix cores; rocprofv3 counters in the profile give the VALU
+    issue rate, lane use and LDS use beside it).
     Algorithmic integer operations = W_alg / 4: every 4-byte operand word of
     an AND of rows is one AND (or one three-input bit op) or one
     popcount-accumulate."""
@@ -73,16 +78,18 @@ def clique_roofline(kernel, ms, walg, prof):
            "peak_source": "MI355X 157.3 TFLOP/s FP32 vector peak / 2 flops per FMA (256 CUs x 4 SIMDs x 32 "
                           "lanes x 2.4 GHz)"}
     if prof:
-        hbm = prof.get("hbm_bytes_per_launch", {}).get(kernel)
+        names = CLIQUE_GROUPS.get(kernel, (kernel,))
+        hbm = sum(prof.get("hbm_bytes_per_launch", {}).get(n, 0) for n in names)
         if hbm:
             out["traffic"] = hbm
             out["hbm_achieved_gbps"] = hbm / (ms * 1e-3) / 1e9
             out["hbm_frac"] = out["hbm_achieved_gbps"] / HBM_PEAK_GBPS
-        low = prof.get("hbm_bytes_per_launch_unscaled_fetch", {}).get(kernel)
+        low = sum(prof.get("hbm_bytes_per_launch_unscaled_fetch", {}).get(n, 0) for n in names)
         if low:
             out["hbm_frac_unscaled_fetch"] = low / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS
-        d = prof.get("derived", {}).get(kernel)
+        d = prof.get("derived", {}).get(names[0])
         if d:
+            out["counters_kernel"] = names[0]
             out["counters"] = {k: d[k] for k in ("valu_issue", "valu_lane_util", "lds_util", "lds_conflict_share",
                                                  "wait_share", "waves_per_cu") if k in d}
     return out
@@ -102,10 +109,12 @@ def hbm_roofline(kernel, ms, walg, prof):
 
 
 # launch groups of the array store's count: the main launch, and the split
-# subtask levels with the HBM overflow launch and its subtasks
-IEP_GROUPS = {"gatk::engine_kernel<false>": ("gatk::engine_kernel<false>",),
+# subtask levels with the HBM overflow launch and its subtasks (a plan has one
+# of two kernels per launch: the pair kernels sweep its last two levels together)
+IEP_GROUPS = {"gatk::engine_kernel<false>": ("gatk::engine_kernel<false>", "gatk::engine_pair_kernel<false>"),
               "split and HBM launches": ("gatk::engine_sub_kernel<false>", "gatk::engine_kernel<true>",
-                                         "gatk::engine_sub_kernel<true>")}
+                                         "gatk::engine_sub_kernel<true>", "gatk::engine_pair_sub_kernel<false>",
+                                         "gatk::engine_pair_kernel<true>", "gatk::engine_pair_sub_kernel<true>")}
 
 
 def iep_traffic(prof, group, key="hbm_bytes_per_launch"):
@@ -115,7 +124,7 @@ def iep_traffic(prof, group, key="hbm_bytes_per_launch"):
     the group's longest kernel and that kernel's counters."""
     calls = {k["kernel"]: k["calls"] for k in prof["kernel_stats"]}
     total = {k["kernel"]: k["total_ms"] for k in prof["kernel_stats"]}
-    counts = calls.get("gatk::engine_kernel<false>")
+    counts = sum(calls.get(n, 0) for n in IEP_GROUPS["gatk::engine_kernel<false>"])
     hb = prof.get(key, {})
     names = IEP_GROUPS[group]
     if not counts or not all(n in hb for n in names if calls.get(n)):
@@ -480,8 +489,7 @@ def main():
     walg_rest = walg - walg_main - walg_second
     rest_ms = t_b * 1e3 - main_ms - second_ms
     if bitmap:
-        launches = [(CLIQUE_KERNELS[0], main_ms, walg_main), (CLIQUE_KERNELS[1], second_ms, walg_second),
-                    (CLIQUE_KERNELS[2] + " and tier 2", rest_ms, walg_rest)]
+        launches = list(zip(CLIQUE_GROUPS, (main_ms, second_ms, rest_ms), (walg_main, walg_second, walg_rest)))
     else:
         launches = [("gatk::engine_kernel<false>", main_ms, walg_main),
                     ("split and HBM launches", second_ms, walg_second)]
@@ -551,7 +559,7 @@ def main():
     if args.timeline:
         _, tst = batched.count(cfg, timeline=True)
         names = {0: "clique_kernel", 1: "clique_block_kernel tier 0", 2: "clique_block_kernel tier 1",
-                 3: "clique_block_kernel tier 2"} if bitmap else \
+                 3: "clique_block_kernel tier 2", 4: "clique_hbm_kernel"} if bitmap else \
                 {0: "engine_kernel", 1: "subtasks level 1", 2: "subtasks level 2", 3: "subtasks level 3",
                  4: "HBM launch", 5: "HBM subtasks"}
         summ = {"workload": out["config"]["workload"], "kernel_config": cfg, "device_ms": tst["seconds"] * 1e3,
