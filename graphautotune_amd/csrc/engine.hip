@@ -2805,6 +2805,7 @@ struct DeviceGraph {
     long long *off = nullptr;
     int *adj = nullptr;
     int *split = nullptr;
+    std::mutex mu;  // held while the bitmaps are built
     // core bitmap of the clique store (core_n < 0: not built)
     unsigned *core = nullptr;
     int core_n = -1;
@@ -2906,6 +2907,21 @@ static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
     return GAT_OK;
 }
 
+// Memory that a count can do without: false, and *p null, if there is none left.
+template <class T>
+static bool try_malloc(T **p, size_t bytes, int *rc) {
+    *p = nullptr;
+    const hipError_t e = hipMalloc((void **)p, bytes);
+    if (e == hipSuccess) return true;
+    *p = nullptr;
+    (void)hipGetLastError();
+    if (e != hipErrorOutOfMemory) {
+        gat::set_error("hipMalloc failed: %s", hipGetErrorString(e));
+        *rc = GAT_ENODEV;
+    }
+    return false;
+}
+
 // Neighbourhood bitmaps, most connected vertices first, within kHubBytes: of
 // every vertex of degree >= the configured threshold, or by default of those of
 // degree >= kHubDegree and, within kHubMoreBytes, of further ones down to
@@ -2923,6 +2939,7 @@ static int hub_default(int64_t n) { return n <= 16384 ? 16 : 64; }
 // thr: the configured threshold, 0 for the default. dg->hub_full: every vertex
 // from this degree on has a bitmap.
 static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr) {
+    std::lock_guard<std::mutex> lk(dg->mu);
     if (dg->hub_built && dg->hub_degree == thr) return GAT_OK;
     dg->free_hubs();
     const long long words = ((long long)g.n + 31) / 32;
@@ -2948,13 +2965,21 @@ static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr) {
                  hubs.begin();
     hubs.resize(std::min(hubs.size(), std::max(always, (size_t)(kHubMoreBytes / row_bytes))));
     hubs.resize(std::min(hubs.size(), (size_t)(kHubBytes / row_bytes)));
+    long long n_u32 = (long long)hubs.size() * words;
+    if (hubs.size() > always) {  // the rows beyond kHubDegree only where there is room
+        int rc = GAT_OK;
+        if (!try_malloc(&dg->hub_bits, sizeof(unsigned) * (size_t)((n_u32 + 1) / 2 * 2), &rc)) {
+            if (rc) return rc;
+            hubs.resize(always);
+            n_u32 = (long long)always * words;
+        }
+    }
     dg->hub_full = hubs.size() == found ? least : hubs.empty() ? INT_MAX : g.deg(hubs.back()) + 1;
     dg->hub_built = true;
     dg->hub_degree = thr;
     dg->hub_words = words;
     if (hubs.empty()) return GAT_OK;
-    const long long n_u32 = (long long)hubs.size() * words;
-    HIPCHECK(hipMalloc(&dg->hub_bits, sizeof(unsigned) * (size_t)((n_u32 + 1) / 2 * 2)));
+    if (!dg->hub_bits) HIPCHECK(hipMalloc(&dg->hub_bits, sizeof(unsigned) * (size_t)((n_u32 + 1) / 2 * 2)));
     hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, nullptr, (unsigned long long *)dg->hub_bits,
                        (n_u32 + 1) / 2, 0ull);
     if (!ordered) {
@@ -2987,10 +3012,18 @@ static int core_vertices(int64_t n, long long words) {
 }
 
 static int ensure_core(const Graph &g, DeviceGraph *dg) {
+    std::lock_guard<std::mutex> lk(dg->mu);  // plans of one graph may be first counted on different threads
     if (dg->core_n >= 0) return GAT_OK;
-    const int h = core_vertices(g.n, std::max<long long>(1 << 21, 4ll * g.m));
-    const size_t words = gatk::core_row(h);
-    HIPCHECK(hipMalloc(&dg->core, sizeof(unsigned) * std::max<size_t>(words, 16)));
+    long long budget = std::max<long long>(1 << 21, 4ll * g.m);
+    int h = core_vertices(g.n, budget);
+    int rc = GAT_OK;
+    // fewer core vertices where memory is short
+    while (!try_malloc(&dg->core, sizeof(unsigned) * std::max<size_t>(gatk::core_row(h), 16), &rc)) {
+        if (rc) return rc;
+        if (budget <= 1 << 21) GAT_FAIL(GAT_ENODEV, "no device memory for the core bitmap (%d rows)", h);
+        budget = std::max<long long>(1 << 21, budget / 4);
+        h = core_vertices(g.n, budget);
+    }
     if (h > 0) {
         hipLaunchKernelGGL(gatk::core_rows_kernel, dim3(std::min((h + 3) / 4, 4096)), dim3(256), 0, nullptr, dg->off,
                            dg->adj, dg->split, h, dg->core);
@@ -3130,17 +3163,23 @@ static int ensure_tables(gat_plan *p) {
     const GatPlanDev &pd = p->cp.dev;
     const Graph &g = *p->graph;
     if (g.m == 0 || g.max_deg >= 1 << 24 || g.m >= (1ll << 32) - 1) return GAT_OK;
+    d->keep = 0;
+    int rc = GAT_OK;
     for (int k = 0; k < 4; k++)
-        if ((pd.edge_tables >> k & 1) && !d->edge_tab[k])
-            HIPCHECK(hipMalloc(&d->edge_tab[k], sizeof(int) * (((size_t)g.m + 1) / 2 * 2)));
-    d->keep = pd.edge_tables || pd.n_tables;
-    if (pd.n_tables == 0 || d->pool) return GAT_OK;
+        if ((pd.edge_tables >> k & 1) && !d->edge_tab[k] &&
+            !try_malloc(&d->edge_tab[k], sizeof(int) * (((size_t)g.m + 1) / 2 * 2), &rc))
+            return rc;
+    if (pd.n_tables == 0 || d->pool) {
+        d->keep = pd.edge_tables || pd.n_tables;
+        return GAT_OK;
+    }
     d->tab_size = std::min(g.n, kTabVertices);
     const long long most = kPoolBytes / (8ll * pd.n_tables * d->tab_size);
     d->pool_tables = (unsigned)std::max(1ll, std::min<long long>(most, pd.key_edges ? g.m : g.n));
     d->pool_entries = (long long)pd.n_tables * d->pool_tables * d->tab_size;
-    HIPCHECK(hipMalloc(&d->pool, sizeof(uint2) * d->pool_entries));
+    if (!try_malloc(&d->pool, sizeof(uint2) * d->pool_entries, &rc)) return rc;
     d->epoch = 255;  // cleared by the first count
+    d->keep = 1;
     return GAT_OK;
 }
 
