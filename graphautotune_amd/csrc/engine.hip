@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "handles.hpp"
+#include "kept.h"
 #include "plan_dev.h"
 
 namespace gatk {
@@ -101,13 +102,13 @@ struct KArgs {
     // there are many (R-MAT s13's C5: 1.3e9 paths over 6.7e7 pairs of vertices).
     // edge_tab[k][e] is the value of directed edge e with truncation k, or -1.
     // Pool i holds tables of tab_size entries from pool + i pool_tables
-    // tab_size on; key x uses table x % pool_tables, whose entry c is {x + 1,
-    // value | epoch << 24} for the key that wrote it last. Every count has its
+    // tab_size on; key x uses table x % pool_tables, whose entry c holds the tag
+    // x + 1, the value and the epoch for the key that wrote it last. Every count has its
     // own epoch, so nothing of an earlier one is taken. One pool for all waves:
     // with a table per wave the subtasks of one root each filled their own
     // (C5 108 ms, now 56; house on Chung-Lu 65,536 46 ms, now 36).
-    int *edge_tab[4];
-    uint2 *pool;
+    KeptEdge *edge_tab[4];
+    KeptEntry *pool;
     unsigned pool_tables;
     int tab_size;
     unsigned epoch;
@@ -930,7 +931,7 @@ __device__ __forceinline__ int sweep_kept(const Ctx &C, int f, bool need, int c,
 
 // The table of a KEEP_POOL op for the chosen v_0, v_1 or root edge, and the tag
 // of its entries.
-__device__ __forceinline__ uint2 *pool_table(const Ctx &C, const GatOp &o, unsigned *tag) {
+__device__ __forceinline__ KeptEntry *pool_table(const Ctx &C, const GatOp &o, unsigned *tag) {
     const KArgs &a = C.a;
     const WaveState *S = C.S;
     unsigned key;
@@ -987,14 +988,14 @@ __device__ __forceinline__ bool leaf_known(const Ctx &C, const GatNode &N, int c
     for (int k = 0; k < N.op_count; k++) {
         const GatOp &o = C.P.ops[N.op_begin + k];
         if (o.kind != GATP_COUNT) continue;
-        if (o.keep == GATP_KEEP_EDGE) known = known && a.edge_tab[o.table][C.S->sbeg[N.loop_slot] + ci] >= 0;
+        if (o.keep == GATP_KEEP_EDGE) known = known && a.edge_tab[o.table][C.S->sbeg[N.loop_slot] + ci].read() >= 0;
         if (o.keep == GATP_KEEP_POOL) {
             unsigned key = 0;  // pool_table without its cross-lane reads
             if (o.key == 3) key = (unsigned)(C.S->sub_edge >= 0 ? C.S->sub_edge : C.S->rb + (C.S->f_cur[1] - 1));
             else key = (unsigned)C.S->val[o.key == 2 ? 1 : 0];
             if (c >= a.tab_size) return false;
-            const uint2 e = a.pool[((long long)o.table * a.pool_tables + key % a.pool_tables) * a.tab_size + c];
-            known = known && e.x == key + 1 && e.y >> 24 == a.epoch;
+            const long long table = (long long)o.table * a.pool_tables + key % a.pool_tables;
+            known = known && a.pool[table * a.tab_size + c].read().serves(key + 1, a.epoch);
         }
     }
     return known;
@@ -1014,7 +1015,7 @@ __device__ __forceinline__ void leaf_sums(const Ctx &C, const GatNode &N, int d)
         const long long vb = a.off[v];
         const int deg = (int)(a.off[v + 1] - vb), b = o.table ? v : INT_MAX;
         const int t = uni(group_bound(S, o.groups, o.ngroups, d, 0));
-        int *edge = a.edge_tab[o.table] + vb;
+        KeptEdge *edge = a.edge_tab[o.table] + vb;
         const int len = uni(S->slen[o.father]);
         unsigned long long sum = 0;
         for (int base = 0; base < len; base += W) {
@@ -1026,11 +1027,14 @@ __device__ __forceinline__ void leaf_sums(const Ctx &C, const GatNode &N, int d)
                 if (o.excl >> f & 1u) use = use && x != S->val[f];
             int cnt = 0;
             const int pos = use ? lbound(a.adj + vb, deg, x) : 0;
-            if (use) cnt = edge[pos];
+            if (use) cnt = edge[pos].read();
             const bool need = use && cnt < 0;
             if (ballot(need)) {
                 const int fresh = sweep_kept<GS>(C, N.loop_slot, need, x, b);
-                if (need) edge[pos] = cnt = fresh;
+                if (need) {
+                    cnt = fresh;
+                    edge[pos].write(fresh);
+                }
             }
             // candidates that are skipped or empty although they lie in N(v_j)
             // below b: chosen vertices (each once)
@@ -1110,8 +1114,8 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
             const bool live = pass && !dup;
             bool need = live;
             int kept = 0;
-            int *edge = nullptr;
-            uint2 *slot = nullptr;
+            KeptEdge *edge = nullptr;
+            KeptEntry *slot = nullptr;
             unsigned tag = 0;
             if (KEEP && o.keep == GATP_KEEP_SUM) {  // added by leaf_sums
                 S->leafcnt[o.leaf_idx][ln] = 0;
@@ -1120,14 +1124,14 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
             if (KEEP && o.keep == GATP_KEEP_EDGE) edge = a.edge_tab[o.table];
             if (KEEP && edge) {
                 edge += S->sbeg[N.loop_slot] + ci;
-                if (live) kept = *edge;
+                if (live) kept = edge->read();
                 need = live && kept < 0;
             } else if (KEEP && o.keep == GATP_KEEP_POOL) {
                 slot = pool_table(C, o, &tag) + c;
                 if (live && c < a.tab_size) {
-                    const uint2 e = *slot;
-                    kept = (int)(e.y & 0xffffffu);
-                    need = e.x != tag || e.y >> 24 != a.epoch;
+                    const KeptEntry::Read e = slot->read();
+                    kept = e.value();
+                    need = !e.serves(tag, a.epoch);
                 }
             }
             const bool by_table = KEEP && (edge || slot);
@@ -1157,8 +1161,8 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
             cnt = sweep_count<GS>(C, o.father, need, c, ab, alen, t, ex, nex, &blen);
             if (a.account && live)
                 bytes += 4ull * (alen + blen) + 16ull + (C.P.slots[o.father].kind == GATP_ALIAS ? 16ull : 0ull);
-            if (need && edge) *edge = cnt;
-            if (need && slot && c < a.tab_size) *slot = make_uint2(tag, (unsigned)cnt | a.epoch << 24);
+            if (need && edge) edge->write(cnt);
+            if (need && slot && c < a.tab_size) slot->write(tag, cnt, a.epoch);
             }
             if (by_table) {
                 if (!need) cnt = kept;
@@ -1211,7 +1215,7 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
     const GatTerm &Tm = C.P.terms[M.term_begin];
     leaf_exclusions(C, M, d);
     unsigned tag;
-    uint2 *tab = pool_table(C, o, &tag);
+    KeptEntry *tab = pool_table(C, o, &tag);
     const bool ex_v = o.excl >> d & 1u;
     // what the chosen vertices of the levels below d mean for every c: skip[],
     // the vertices c must differ from; less[], those to subtract where c is
@@ -1274,7 +1278,7 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
         constexpr int U = 2;  // steps in flight
         for (int k0 = 0; k0 < T; k0 += U * W) {
             int c[U], w[U], t[U];
-            uint2 e[U];
+            KeptEntry::Read e[U];
             bool live[U], wex[U];
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -1299,8 +1303,8 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
                     live[u] = live[u] && c[u] != skip[i];
                 }
                 live[u] = live[u] && !((M.excl >> d & 1u) && c[u] == w[u]);
-                e[u] = make_uint2(0, 0);
-                if (live[u] && c[u] < a.tab_size) e[u] = tab[c[u]];
+                e[u] = {0, 0};  // tags start at 1
+                if (live[u] && c[u] < a.tab_size) e[u] = tab[c[u]].read();
                 t[u] = t_lane ? group_bound(S, o.groups, o.ngroups, d + 1, c[u]) : t_all;
             }
             int cnt[U];
@@ -1318,13 +1322,13 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const bool need = live[u] && (e[u].x != tag || e[u].y >> 24 != a.epoch);
-                int x = (int)(e[u].y & 0xffffffu);
+                const bool need = live[u] && !e[u].serves(tag, a.epoch);
+                int x = e[u].value();
                 if (ballot(need)) {
                     const int fresh = sweep_kept<GS>(C, o.father, need, c[u], t[u]);
                     if (need) {
                         x = fresh;
-                        if (c[u] < a.tab_size) tab[c[u]] = make_uint2(tag, (unsigned)fresh | a.epoch << 24);
+                        if (c[u] < a.tab_size) tab[c[u]].write(tag, fresh, a.epoch);
                     }
                 }
                 if (live[u]) sum += (unsigned long long)(long long)(x + cnt[u]);
@@ -2852,8 +2856,8 @@ struct PlanDevice {
     int *gstore = nullptr;
     size_t gstore_bytes = 0;
     // kept COUNT values (array store)
-    int *edge_tab[4] = {};
-    uint2 *pool = nullptr;
+    gatk::KeptEdge *edge_tab[4] = {};
+    gatk::KeptEntry *pool = nullptr;
     long long pool_entries = 0;
     unsigned pool_tables = 0, epoch = 0;
     int tab_size = 0;
@@ -3167,7 +3171,7 @@ static int ensure_tables(gat_plan *p) {
     int rc = GAT_OK;
     for (int k = 0; k < 4; k++)
         if ((pd.edge_tables >> k & 1) && !d->edge_tab[k] &&
-            !try_malloc(&d->edge_tab[k], sizeof(int) * (((size_t)g.m + 1) / 2 * 2), &rc))
+            !try_malloc(&d->edge_tab[k], sizeof(gatk::KeptEdge) * (((size_t)g.m + 1) / 2 * 2), &rc))
             return rc;
     if (pd.n_tables == 0 || d->pool) {
         d->keep = pd.edge_tables || pd.n_tables;
@@ -3177,7 +3181,7 @@ static int ensure_tables(gat_plan *p) {
     const long long most = kPoolBytes / (8ll * pd.n_tables * d->tab_size);
     d->pool_tables = (unsigned)std::max(1ll, std::min<long long>(most, pd.key_edges ? g.m : g.n));
     d->pool_entries = (long long)pd.n_tables * d->pool_tables * d->tab_size;
-    if (!try_malloc(&d->pool, sizeof(uint2) * d->pool_entries, &rc)) return rc;
+    if (!try_malloc(&d->pool, sizeof(gatk::KeptEntry) * d->pool_entries, &rc)) return rc;
     d->epoch = 255;  // cleared by the first count
     d->keep = 1;
     return GAT_OK;
