@@ -154,12 +154,14 @@ struct WaveState {
     unsigned long long bytes;   // committed W_alg of this wave
     unsigned long long ebytes;  // W_alg of the work not yet committed
     long long t0;               // wall clock at the start of the task
+    long long f_t0[GATP_MAX_DEPTH + 1];  // and of the frames above the leaves (see rest_is_long)
     long long rb;               // first edge of the task's root v0
     long long sub_edge;         // root edge of the running subtask, or -1
     long long don_base[kMaxDonations];  // subtask blocks donated since the last commit
     int don_cnt[kMaxDonations];
     int n_don;
     int base_depth;             // frames exist from this depth on (2, or a subtask's depth)
+    int base_lo;                // first position of that depth's frame
     int path_pos[GATP_MAX_DEPTH + 1];  // a subtask's positions at depths 2 .. base_depth-1
     int abort;
     int ex_in[GATP_MAX_LEAF_OPS];  // leaf: excluded levels whose vertex lies in the op's father
@@ -728,6 +730,29 @@ __device__ __forceinline__ bool want_split(const KArgs &a, const WaveState *S) {
     return queue_drained<GS>(a);
 }
 
+// A loop whose first `done` candidates took `ticks`: will the other `left` take
+// more than 1 / kTailShare of the split budget? In the tail such a rest does not
+// wait for the budget: idle waves are there to take it, and one subtask costs 10
+// to 20 us. (Counts of a few roots are tails from their start: C5 of one light
+// root of Chung-Lu 1M, 1.7 to 5.3 ms in the mean of eight, 4.8 when every level
+// of subtasks waited for the budget.)
+constexpr int kTailShare = 8;
+__device__ __forceinline__ bool rest_is_long(const KArgs &a, long long ticks, int done, int left) {
+    return done > 0 && ticks * left * kTailShare > a.split_ticks * done;
+}
+// The same for the depth-d frame, above the leaves, with candidates [cur, fh)
+// left; or the task has outrun its budget (want_split).
+template <bool GS>
+__device__ __forceinline__ bool due_to_split(const KArgs &a, WaveState *S, int d, int cur, int fh, int ln) {
+    if (a.split_ticks <= 0 || a.sub_mode >= kSplitLevels) return false;
+    const long long now = uni64(wall_clock64());
+    const int done = cur - (d == uni(S->base_depth) ? uni(S->base_lo) : 0);
+    if (done == 0 && ln == 0) S->f_t0[d] = now;
+    const bool spent = now - S->t0 > a.split_ticks;
+    if (!spent && !rest_is_long(a, now - S->f_t0[d], done, fh - cur)) return false;
+    return queue_drained<GS>(a);
+}
+
 // Hands candidates [lo, hi) of the depth-d frame's node to the next split
 // launch, in at most 64 chunks of at least min_chunk. False, with nothing
 // handed on, when the wave's record of donations or the list is full
@@ -1203,8 +1228,10 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
 // tables; of this step alone 285 to 108).
 // Every c takes its value from the kept table; what is missing is computed by
 // sweep_kept. Chunks of v are cut where they would hold more than kPairMax
-// elements, so that the tail of a launch can still be split.
-constexpr int kPairMax = 1 << 14;
+// elements, so that the tail of a launch can still be split. Once the queue is
+// drained they end at kPairTail elements, and a rest that would be long at the
+// pace of the chunk just done is handed on (rest_is_long).
+constexpr int kPairMax = 1 << 14, kPairTail = 1 << 11;
 template <bool GS>
 __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur, int hi, bool can_split) {
     const KArgs &a = C.a;
@@ -1248,6 +1275,9 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
     unsigned long long sum = 0;
     int nl = W;
     for (int cb = cur; cb < hi; cb += nl) {
+        const bool tail = can_split && queue_drained<GS>(a);
+        const long long c0 = tail ? uni64(wall_clock64()) : 0;
+        const int most = tail ? kPairTail : kPairMax;
         const int vi = cb + ln;
         int v = 0;
         if (vi < hi) v = with_slot<GS>(C, N.loop_slot, [&](auto p) { return p[vi]; });
@@ -1270,8 +1300,8 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
         int T = 0;
         int myoff = excl_scan(len, &T);
         nl = W;
-        if (T > kPairMax) {
-            nl = max(1, __popcll(ballot(myoff + len <= kPairMax)));  // a prefix of the lanes
+        if (T > most) {
+            nl = max(1, __popcll(ballot(myoff + len <= most)));  // a prefix of the lanes
             T = __shfl(myoff + len, nl - 1);
             if (ln >= nl) myoff = T;
         }
@@ -1334,7 +1364,11 @@ __device__ __forceinline__ void pair_leaf(const Ctx C, int d, int node, int cur,
                 if (live[u]) sum += (unsigned long long)(long long)(x + cnt[u]);
             }
         }
-        if (can_split && hi - (cb + nl) >= 2 && want_split<GS>(a, S) && donate(C, d, node, cb + nl, hi, 1, !GS)) break;
+        const int left = hi - (cb + nl);
+        if (!can_split || left < 2) continue;
+        const bool long_rest = tail && rest_is_long(a, uni64(wall_clock64()) - c0, nl, left);
+        if (long_rest && split_shallowest<GS>(C, d - 1)) continue;
+        if ((long_rest || want_split<GS>(a, S)) && donate(C, d, node, cb + nl, hi, 1, !GS)) break;
     }
     sum = wave_sum64(sum);
     if (ln == 0) S->task_acc[Tm.pattern] += sum * (unsigned long long)(long long)C.P.subs[Tm.sub_begin].coef;
@@ -1412,6 +1446,7 @@ __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e
             S->rb = rb;
             S->sub_edge = -1;
             S->base_depth = 2;
+            S->base_lo = 0;
         }
         wsync();
         for (int k = 0; k < root.op_count; k++) exec_op_uniform<GS>(C, P.ops[root.op_begin + k], 0, v0, false);
@@ -1430,12 +1465,12 @@ __device__ __forceinline__ void run_task(const Ctx &C, long long e0, long long e
                 exhausted = true;
             } else if (PAIR && N.pair && d >= 2) {
                 const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
-                if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
+                if (can_split && cur < fh && due_to_split<GS>(a, S, d, cur, fh, C.ln) && split_shallowest<GS>(C, d)) continue;
                 pair_leaf<GS>(C, d, node, cur, fh, can_split);
                 exhausted = true;
             } else {
                 const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
-                if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
+                if (can_split && cur < fh && due_to_split<GS>(a, S, d, cur, fh, C.ln) && split_shallowest<GS>(C, d)) continue;
                 if (cur < fh) {
                     const int c = uni(with_slot<GS>(C, N.loop_slot, [&](auto p) { return p[cur]; }));
                     if (C.ln == 0) S->f_cur[d] = cur + 1;
@@ -1498,6 +1533,7 @@ __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
         S->rb = rb;
         S->sub_edge = e;
         S->base_depth = D;
+        S->base_lo = max(sub_lo, 0);
     }
     for (int j = 2 + C.ln; j < D; j += W) S->path_pos[j] = g->pos[j];
     wsync();
@@ -1528,12 +1564,12 @@ __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
             exhausted = true;
         } else if (PAIR && N.pair) {
             const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
-            if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
+            if (can_split && cur < fh && due_to_split<GS>(a, S, d, cur, fh, C.ln) && split_shallowest<GS>(C, d)) continue;
             pair_leaf<GS>(C, d, node, cur, fh, can_split);
             exhausted = true;
         } else {
             const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
-            if (can_split && cur < fh && want_split<GS>(a, S) && split_shallowest<GS>(C, d)) continue;
+            if (can_split && cur < fh && due_to_split<GS>(a, S, d, cur, fh, C.ln) && split_shallowest<GS>(C, d)) continue;
             if (cur < fh) {
                 const int c = uni(with_slot<GS>(C, N.loop_slot, [&](auto p) { return p[cur]; }));
                 if (C.ln == 0) S->f_cur[d] = cur + 1;

@@ -161,9 +161,10 @@ typedef struct gat_kernel_config {
                                  many microseconds, once its launch's queue
                                  is drained, hands the unfinished rest of its
                                  shallowest loop at depth >= 2 to subtask
-                                 launches in up to 64 parts (0 = 2000,
-                                 negative = never); counts and W_alg do not
-                                 change                                       */
+                                 launches in up to 64 parts, and before that
+                                 where the rest of a loop would take an eighth
+                                 of it at the pace so far (0 = 2000, negative
+                                 = never); counts and W_alg do not change     */
 } gat_kernel_config;
 
 /* Per-call statistics filled by gat_count (any pointer may be NULL). */
