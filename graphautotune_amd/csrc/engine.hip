@@ -76,7 +76,8 @@ struct KArgs {
     int account;
     // Dense neighbourhood bitmaps of high-degree vertices ("hubs"): row h
     // holds bit x set iff x is a neighbour of hub h. hub_map == nullptr means
-    // the graph is degree-ordered and the hubs are vertices [0, n_hubs).
+    // the graph is degree-ordered and the hubs are vertices [0, n_hubs); else
+    // it gives a vertex's row, or -1, and rows from n_hubs on are not used.
     const unsigned *hub_bits;
     const int *hub_map;
     long long hub_words;  // words per row: (n + 31) / 32
@@ -382,8 +383,8 @@ __device__ __forceinline__ int trunc_len(const KArgs &a, int v, long long beg, i
 // Hub row of vertex v, or -1.
 __device__ __forceinline__ int hub_of(const KArgs &a, int v) {
     if (a.n_hubs == 0) return -1;
-    if (a.hub_map) return a.hub_map[v];
-    return v < a.n_hubs ? v : -1;
+    const int h = a.hub_map ? a.hub_map[v] : v;
+    return h < a.n_hubs ? h : -1;
 }
 // Membership of x in the first len entries of hub h's sorted neighbour
 // list, whose last kept entry is lim: one bitmap word instead of a search.
@@ -2787,10 +2788,15 @@ __global__ void copy_kernel(const int4 *__restrict__ src, int4 *__restrict__ dst
 // ===========================================================================
 namespace gat {
 
+// (The runtime keeps an error until it is asked for: read here, it does not
+// turn up in the next count's check of its launches.)
 #define HIPCHECK(x)                                                                                  \
     do {                                                                                             \
         hipError_t e_ = (x);                                                                         \
-        if (e_ != hipSuccess) GAT_FAIL(GAT_ENODEV, "%s failed: %s", #x, hipGetErrorString(e_));      \
+        if (e_ != hipSuccess) {                                                                      \
+            (void)hipGetLastError();                                                                 \
+            GAT_FAIL(GAT_ENODEV, "%s failed: %s", #x, hipGetErrorString(e_));                        \
+        }                                                                                            \
     } while (0)
 
 struct DeviceInfo {
@@ -2841,6 +2847,21 @@ static int device_info(DeviceInfo *out) {
     return GAT_OK;
 }
 
+// Bitmap rows of the n most connected vertices of a graph, in the order of
+// degree (descending, then id). A count that needs fewer uses the first of
+// them, so plans of different thresholds share one set. It is shared: whoever
+// replaces it leaves it to the counts that were prepared with it.
+struct HubRows {
+    size_t n = 0;
+    unsigned *bits = nullptr;
+    int *map = nullptr;  // null when the graph is degree-ordered
+    int *vertex = nullptr;
+    ~HubRows() {
+        for (void *p : {(void *)bits, (void *)map, (void *)vertex})
+            if (p) (void)hipFree(p);
+    }
+};
+
 struct DeviceGraph {
     long long *off = nullptr;
     int *adj = nullptr;
@@ -2849,27 +2870,11 @@ struct DeviceGraph {
     // core bitmap of the clique store (core_n < 0: not built)
     unsigned *core = nullptr;
     int core_n = -1;
-    // hub bitmaps, built for the threshold hub_degree (0: the default)
-    bool hub_built = false;
-    int hub_degree = 0;
-    int hub_full = INT_MAX;
-    int n_hubs = 0;
-    long long hub_words = 0;
-    unsigned *hub_bits = nullptr;
-    int *hub_map = nullptr;     // null when the graph is degree-ordered
-    int *hub_vertex = nullptr;
-    void free_hubs() {
-        for (void *p : {(void *)hub_bits, (void *)hub_map, (void *)hub_vertex})
-            if (p) (void)hipFree(p);
-        hub_bits = nullptr;
-        hub_map = hub_vertex = nullptr;
-        n_hubs = 0;
-        hub_degree = 0;
-        hub_full = INT_MAX;
-        hub_built = false;
-    }
+    std::shared_ptr<HubRows> hubs;
+    std::vector<int> at_least;     // at_least[d]: vertices of degree >= d, d <= max_deg + 1
+    bool ordered = false;          // ids by descending degree
+    size_t hubs_short = SIZE_MAX;  // a set of so many rows found no memory
     ~DeviceGraph() {
-        free_hubs();
         if (off) (void)hipFree(off);
         if (adj) (void)hipFree(adj);
         if (split) (void)hipFree(split);
@@ -2970,71 +2975,91 @@ static bool try_malloc(T **p, size_t bytes, int *rc) {
 // own. ms with a threshold of 256 / 64 / 16: house on Chung-Lu 65,536 22.0 /
 // 19.1 / 19.1, C5 on R-MAT s13 24.3 / 22.0 / 21.8, 21 patterns on R-MAT s10
 // 11.1 / 8.8 / 7.3, C4 + P4 on a random graph of 100,000 vertices and mean
-// degree 16 3.8 / 3.8 / 5.6. Built once per (graph, threshold) outside the
-// timed count, like the graph upload itself.
+// degree 16 3.8 / 3.8 / 5.6. Built outside the timed count, like the graph
+// upload itself, when a graph's first count needs them or a later one needs more.
 constexpr double kHubBytes = 8.0 * (1ull << 30), kHubMoreBytes = 1.0 * (1ull << 30);
 constexpr int kHubDegree = 256;
 static int hub_default(int64_t n) { return n <= 16384 ? 16 : 64; }
 
-// thr: the configured threshold, 0 for the default. dg->hub_full: every vertex
-// from this degree on has a bitmap.
-static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr) {
-    std::lock_guard<std::mutex> lk(dg->mu);
-    if (dg->hub_built && dg->hub_degree == thr) return GAT_OK;
-    dg->free_hubs();
-    const long long words = ((long long)g.n + 31) / 32;
-    bool ordered = true;  // degree-ordered graphs keep hubs as a prefix
-    for (int32_t v = 1; v < g.n && ordered; v++) ordered = g.deg(v) <= g.deg(v - 1);
-    const int least = thr ? thr : hub_default(g.n);
-    std::vector<int32_t> hubs;
-    if (ordered) {
-        int32_t h = 0;
-        while (h < g.n && g.deg(h) >= least) h++;
-        hubs.resize(h);
-        std::iota(hubs.begin(), hubs.end(), 0);
-    } else {
+// What a count uses of them: the first n rows. full: every vertex from this
+// degree on has one.
+struct HubUse {
+    std::shared_ptr<HubRows> rows;
+    int n = 0, full = INT_MAX;
+};
+
+static int build_hubs(const Graph &g, DeviceGraph *dg, size_t n, int least, std::shared_ptr<HubRows> *out) {
+    const long long words = ((long long)g.n + 31) / 32, n_u64 = ((long long)n * words + 1) / 2;
+    auto h = std::make_shared<HubRows>();
+    h->n = n;
+    int rc = GAT_OK;
+    if (!try_malloc(&h->bits, 8 * (size_t)n_u64, &rc)) return rc;  // *out stays empty
+    hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, nullptr, (unsigned long long *)h->bits, n_u64, 0ull);
+    if (!dg->ordered) {
+        std::vector<int32_t> hubs, map(size_t(g.n), -1);
         for (int32_t v = 0; v < g.n; v++)
             if (g.deg(v) >= least) hubs.push_back(v);
         std::stable_sort(hubs.begin(), hubs.end(), [&](int32_t x, int32_t y) { return g.deg(x) > g.deg(y); });
+        hubs.resize(n);
+        for (size_t k = 0; k < n; k++) map[hubs[k]] = int32_t(k);
+        HIPCHECK(hipMalloc(&h->map, sizeof(int) * size_t(g.n)));
+        HIPCHECK(hipMalloc(&h->vertex, sizeof(int) * n));
+        HIPCHECK(hipMemcpy(h->map, map.data(), sizeof(int) * size_t(g.n), hipMemcpyHostToDevice));
+        HIPCHECK(hipMemcpy(h->vertex, hubs.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     }
-    const size_t found = hubs.size();
-    const double row_bytes = 4.0 * std::max(1ll, words);
-    size_t always = hubs.size();  // rows that only kHubBytes limits
-    if (!thr)
-        always = std::partition_point(hubs.begin(), hubs.end(), [&](int32_t v) { return g.deg(v) >= kHubDegree; }) -
-                 hubs.begin();
-    hubs.resize(std::min(hubs.size(), std::max(always, (size_t)(kHubMoreBytes / row_bytes))));
-    hubs.resize(std::min(hubs.size(), (size_t)(kHubBytes / row_bytes)));
-    long long n_u32 = (long long)hubs.size() * words;
-    if (hubs.size() > always) {  // the rows beyond kHubDegree only where there is room
-        int rc = GAT_OK;
-        if (!try_malloc(&dg->hub_bits, sizeof(unsigned) * (size_t)((n_u32 + 1) / 2 * 2), &rc)) {
-            if (rc) return rc;
-            hubs.resize(always);
-            n_u32 = (long long)always * words;
-        }
-    }
-    dg->hub_full = hubs.size() == found ? least : hubs.empty() ? INT_MAX : g.deg(hubs.back()) + 1;
-    dg->hub_built = true;
-    dg->hub_degree = thr;
-    dg->hub_words = words;
-    if (hubs.empty()) return GAT_OK;
-    if (!dg->hub_bits) HIPCHECK(hipMalloc(&dg->hub_bits, sizeof(unsigned) * (size_t)((n_u32 + 1) / 2 * 2)));
-    hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, nullptr, (unsigned long long *)dg->hub_bits,
-                       (n_u32 + 1) / 2, 0ull);
-    if (!ordered) {
-        std::vector<int32_t> map(size_t(g.n), -1);
-        for (size_t h = 0; h < hubs.size(); h++) map[hubs[h]] = int32_t(h);
-        HIPCHECK(hipMalloc(&dg->hub_map, sizeof(int) * size_t(g.n)));
-        HIPCHECK(hipMalloc(&dg->hub_vertex, sizeof(int) * hubs.size()));
-        HIPCHECK(hipMemcpy(dg->hub_map, map.data(), sizeof(int) * size_t(g.n), hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(dg->hub_vertex, hubs.data(), sizeof(int) * hubs.size(), hipMemcpyHostToDevice));
-    }
-    hipLaunchKernelGGL(gatk::hub_rows_kernel, dim3((unsigned)std::min<size_t>(hubs.size(), 65535)), dim3(256), 0,
-                       nullptr, dg->off, dg->adj, dg->hub_vertex, (int)hubs.size(), dg->hub_bits, words);
+    hipLaunchKernelGGL(gatk::hub_rows_kernel, dim3((unsigned)std::min<size_t>(n, 65535)), dim3(256), 0, nullptr, dg->off,
+                       dg->adj, h->vertex, (int)n, h->bits, words);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipDeviceSynchronize());
-    dg->n_hubs = (int)hubs.size();
+    *out = h;
+    return GAT_OK;
+}
+
+// thr: the configured threshold, 0 for the default. The graph's rows serve if
+// there are enough of them; else they are built anew, and on a failure the
+// graph is left without any, for the next count to build.
+static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr, HubUse *out) {
+    std::lock_guard<std::mutex> lk(dg->mu);
+    if (dg->at_least.empty()) {
+        std::vector<int> c((size_t)g.max_deg + 2, 0);
+        bool ordered = true;
+        for (int32_t v = 0; v < g.n; v++) {
+            c[g.deg(v)]++;
+            ordered = ordered && (v == 0 || g.deg(v) <= g.deg(v - 1));
+        }
+        for (size_t d = c.size() - 1; d-- > 0;) c[d] += c[d + 1];
+        dg->ordered = ordered;
+        dg->at_least = std::move(c);
+    }
+    const std::vector<int> &at_least = dg->at_least;
+    auto vertices = [&](int degree) -> size_t { return degree < (int)at_least.size() ? at_least[degree] : 0; };
+    const int least = thr ? thr : hub_default(g.n);
+    const double row_bytes = 4.0 * (double)std::max(1ll, ((long long)g.n + 31) / 32);
+    const size_t found = vertices(least), most = (size_t)(kHubBytes / row_bytes);
+    const size_t always = std::min(thr ? found : vertices(std::max(least, kHubDegree)), most);  // rows that only kHubBytes limits
+    size_t n = std::min({found, std::max(always, (size_t)(kHubMoreBytes / row_bytes)), most});
+    if (n > always && n >= dg->hubs_short) n = always;
+    if (n && (!dg->hubs || dg->hubs->n < n)) {
+        dg->hubs.reset();
+        std::shared_ptr<HubRows> rows;
+        int rc = build_hubs(g, dg, n, least, &rows);
+        if (!rc && !rows && n > always) {  // the rows beyond kHubDegree only where there is room
+            dg->hubs_short = n;
+            n = always;
+            rc = n ? build_hubs(g, dg, n, least, &rows) : GAT_OK;
+        }
+        if (rc) return rc;
+        if (!rows && n) GAT_FAIL(GAT_ENODEV, "no device memory for the bitmaps of %zu vertices", n);
+        dg->hubs = rows;
+    }
+    out->rows = dg->hubs;
+    out->n = (int)n;
+    // one more than the degree of the last row's vertex, if some are left without
+    out->full = n == found ? least
+                : n == 0   ? INT_MAX
+                           : (int)(std::partition_point(at_least.begin(), at_least.end(),
+                                                        [&](int c) { return (size_t)c >= n; }) -
+                                   at_least.begin());
     return GAT_OK;
 }
 
@@ -3115,6 +3140,7 @@ struct Launch {
     bool edge_grain = false;  // the HBM launch takes single edges
     bool may_overflow = true; // some intersection may outgrow its LDS buffer
     bool pair = false;        // the plan has nodes swept with their leaf (GatNode::pair)
+    HubUse hubs;              // kept for as long as the count may read them
     bool heavy = false;   // clique: some vertex may have more than main_max neighbours below it
 };
 
@@ -3293,10 +3319,10 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     const int state_bytes = int((sizeof(gatk::WaveState) -
                                  size_t(GATP_MAX_LEAF_OPS - pd.max_leaf_ops) * sizeof(int) * 64 + 15) / 16 * 16);
     if (!clique && cfg.hub_degree >= 0) {
-        rc = ensure_hubs(g, d->dg.get(), cfg.hub_degree);
+        rc = ensure_hubs(g, d->dg.get(), cfg.hub_degree, &L->hubs);
         if (rc) return rc;
     }
-    const int staged = !clique && cfg.hub_degree >= 0 ? std::min(cfg.slot_capacity, d->dg->hub_full) : cfg.slot_capacity;
+    const int staged = !clique && cfg.hub_degree >= 0 ? std::min(cfg.slot_capacity, L->hubs.full) : cfg.slot_capacity;
     const int stage_cap = std::min(cfg.slot_capacity, (staged + 3) / 4 * 4);
     long long store_off[GATP_MAX_STORE] = {}, entries = 0;
     for (int r = 0; r < pd.n_store; r++) {
@@ -3354,11 +3380,11 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         a.keep = d->keep;
     }
     a.split_ticks = split ? (long long)cfg.split_us * di.wall_khz / 1000 : 0;
-    if (!clique && cfg.hub_degree >= 0) {
-        a.hub_bits = d->dg->hub_bits;
-        a.hub_map = d->dg->hub_map;
-        a.hub_words = d->dg->hub_words;
-        a.n_hubs = d->dg->n_hubs;
+    if (L->hubs.n) {
+        a.hub_bits = L->hubs.rows->bits;
+        a.hub_map = L->hubs.rows->map;
+        a.hub_words = ((long long)g.n + 31) / 32;
+        a.n_hubs = L->hubs.n;
     }
     L->a = a;
     L->block = dim3(64 * cfg.block_waves);
