@@ -2932,6 +2932,7 @@ void destroy_plan_device(PlanDevice *d) {
 }
 
 static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
+    std::lock_guard<std::mutex> lk(*g.dev_mu);
     if (g.dev) {
         *out = std::static_pointer_cast<DeviceGraph>(g.dev);
         return GAT_OK;
@@ -2950,6 +2951,20 @@ static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
     g.dev = dg;
     *out = dg;
     return GAT_OK;
+}
+
+// The largest number of neighbours below a vertex.
+static int32_t max_out_degree(Graph &g) {
+    std::lock_guard<std::mutex> lk(*g.dev_mu);
+    if (g.max_out < 0) {
+        int32_t mo = 0;
+        for (int32_t v = 0; v < g.n; v++) {
+            const int32_t *b = g.adj.data() + g.off[v], *en = g.adj.data() + g.off[v + 1];
+            mo = std::max(mo, int32_t(std::lower_bound(b, en, v) - b));
+        }
+        g.max_out = mo;
+    }
+    return g.max_out;
 }
 
 // Memory that a count can do without: false, and *p null, if there is none left.
@@ -3406,14 +3421,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     L->ovf_lds = L->ovf_wave_bytes;
     L->clique = clique;
     if (clique) {
-        if (g.max_out < 0) {
-            int32_t mo = 0;
-            for (int32_t v = 0; v < g.n; v++) {
-                const int32_t *b = g.adj.data() + g.off[v], *en = g.adj.data() + g.off[v + 1];
-                mo = std::max(mo, int32_t(std::lower_bound(b, en, v) - b));
-            }
-            g.max_out = mo;
-        }
+        const int max_out = max_out_degree(g);
         rc = ensure_core(g, d->dg.get());
         if (rc) return rc;
         gatk::CArgs c{};
@@ -3434,7 +3442,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         c.bytes = a.bytes;
         c.err = a.err;
         L->ca = c;
-        rc = clique_shape(di, cfg, g.max_out, L);
+        rc = clique_shape(di, cfg, max_out, L);
         if (rc) return rc;
         for (int t = 0; t < gatk::CTIERS; t++) {
             if (L->tier_grid[t].x && !d->tier[t]) HIPCHECK(hipMalloc(&d->tier[t], sizeof(int) * ((size_t)g.n + 1)));
@@ -3443,7 +3451,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         }
         if (L->tier_grid[3].x) {
             // HBM tier: one scratch area per workgroup, sized by the maximum out-degree
-            const int hcap = std::max(32, g.max_out), ws = gatk::row_words(hcap);
+            const int hcap = std::max(32, max_out), ws = gatk::row_words(hcap);
             int groups = (int)L->tier_grid[3].x;
             while (groups > 64 && (double)groups * hcap * ws * 4 > 16e9) groups /= 2;
             if (d->big_cap < hcap || d->big_groups < groups) {

@@ -3,6 +3,7 @@
 #include <cstdint>
 #include <functional>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -21,8 +22,11 @@ struct Graph {
     std::vector<int64_t> off;
     std::vector<int32_t> adj;
     int32_t max_deg = 0;
-    int32_t max_out = -1;       // max #neighbours below the vertex (computed on demand)
-    std::shared_ptr<void> dev;  // device copy, created by the engine on first use
+    // What plans of the graph, on one thread or several, make on first use and
+    // share; dev_mu is held meanwhile.
+    std::unique_ptr<std::mutex> dev_mu = std::make_unique<std::mutex>();
+    int32_t max_out = -1;       // max #neighbours below the vertex
+    std::shared_ptr<void> dev;  // device copy, created by the engine
 
     int32_t deg(int32_t v) const { return int32_t(off[v + 1] - off[v]); }
     void finish();  // recompute max_deg

@@ -3,12 +3,14 @@
 // RTLD_GLOBAL before libgat.so, so that its symbols are taken for the real ones.
 #include <hip/hip_runtime_api.h>
 
+#include <chrono>
 #include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 
 namespace {
 std::mutex mu;
@@ -18,7 +20,7 @@ std::map<void *, size_t> live;
 std::map<const void *, std::string> kernels;
 size_t live_bytes = 0, limit = SIZE_MAX, refuse_from = SIZE_MAX;
 int refusals = 0;  // the next allocations of at least refuse_from bytes to refuse (-1: all)
-int hold = 0, held = 0;
+int hold = 0, held = 0, copy_ms = 0;
 hipError_t last = hipSuccess;
 struct Config {
     dim3 grid, block;
@@ -48,6 +50,7 @@ size_t fake_live() {
     std::lock_guard<std::mutex> lk(mu);
     return live_bytes;
 }
+void fake_slow_copies(int ms) { copy_ms = ms; }  // every copy takes so long
 // While held, the first stream to be waited for does not finish.
 void fake_hold() { hold = 1; }
 int fake_held() {
@@ -114,6 +117,7 @@ hipError_t hipHostFree(void *p) {
     return hipSuccess;
 }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
+    if (copy_ms) std::this_thread::sleep_for(std::chrono::milliseconds(copy_ms));
     std::memcpy(d, s, n);
     std::lock_guard<std::mutex> lk(mu);
     say("copy " + std::to_string(n));
