@@ -41,7 +41,9 @@ constexpr int kLevelsHbm = kSplitLevels + 1;  // timeline id of the HBM launch (
 // A split subtask: candidates [lo, hi) of the loop of node `node` (at depth
 // `depth` >= 2) below root edge `edge` (directed edge index: v0 = its row,
 // v1 = its entry), with the candidates of depths 2 .. depth-1 taken from
-// loop positions pos[2 ..]. lo >= hi marks an empty or cancelled entry.
+// loop positions pos[2 ..]. lo >= hi marks an empty or cancelled entry. With
+// pos[0] = k + 1 the range is not one of the loop but of the father of the
+// node's KEEP_SUM op k (leaf_sum).
 struct SplitTask {
     long long edge;
     int node, depth, lo, hi;
@@ -760,7 +762,9 @@ __device__ __forceinline__ bool due_to_split(const KArgs &a, WaveState *S, int d
 // (reserved entries past the end of the list are left empty). Donations are
 // recorded for cancellation only where the donor can still abort (LDS
 // buffers); the HBM launch's tasks cannot, so their donations are unlimited.
-__device__ __noinline__ bool donate(const Ctx C, int d, int node, int lo, int hi, int min_chunk, bool record) {
+// sum_op: the op of a KEEP_SUM's range, or -1.
+__device__ __noinline__ bool donate(const Ctx C, int d, int node, int lo, int hi, int min_chunk, bool record,
+                                    int sum_op = -1) {
     const KArgs &a = C.a;
     WaveState *S = C.S;
     if (record && S->n_don >= kMaxDonations) return false;
@@ -780,6 +784,7 @@ __device__ __noinline__ bool donate(const Ctx C, int d, int node, int lo, int hi
         t->depth = d;
         t->lo = fit == parts ? lo + k * chunk : 0;
         t->hi = fit == parts ? min(hi, lo + (k + 1) * chunk) : 0;
+        t->pos[0] = sum_op + 1;
         for (int j = 2; j < d; j++) t->pos[j] = j < S->base_depth ? S->path_pos[j] : S->f_cur[j] - 1;
     }
     if (fit < parts) return false;
@@ -1027,64 +1032,76 @@ __device__ __forceinline__ bool leaf_known(const Ctx &C, const GatNode &N, int c
     return known;
 }
 
-// The KEEP_SUM ops of leaf node N at depth d: their sums over all candidates
-// of the frame, added to the terms that use them.
+// The KEEP_SUM op k of leaf node N (number `node`) at depth d: its sum over all
+// candidates of the frame, taken over the entries [lo, hi) of its father and
+// added to the terms that use it. In the tail, a rest that one wave would sweep
+// for more than 1 / kTailShare of the split budget (3 ticks an element, as in
+// leaf()) goes to the next split launch in up to 64 parts. (One edge between two hubs of Chung-Lu 1M, house: 4.1 ms with the
+// sum on one wave, 2.5 when the leaf that it replaces was split.)
 template <bool GS>
-__device__ __forceinline__ void leaf_sums(const Ctx &C, const GatNode &N, int d) {
+__device__ __forceinline__ void leaf_sum(const Ctx &C, const GatNode &N, int d, int node, int k, int lo, int hi,
+                                         bool can_split) {
     const KArgs &a = C.a;
     WaveState *S = C.S;
     const int ln = C.ln;
-    for (int k = 0; k < N.op_count; k++) {
-        const GatOp &o = C.P.ops[N.op_begin + k];
-        if (o.kind != GATP_COUNT || o.keep != GATP_KEEP_SUM) continue;
-        const int v = uni(S->val[C.P.slots[N.loop_slot].depth]);  // v_j
-        const long long vb = a.off[v];
-        const int deg = (int)(a.off[v + 1] - vb), b = o.table ? v : INT_MAX;
-        const int t = uni(group_bound(S, o.groups, o.ngroups, d, 0));
-        KeptEdge *edge = a.edge_tab[o.table] + vb;
-        const int len = uni(S->slen[o.father]);
-        unsigned long long sum = 0;
-        for (int base = 0; base < len; base += W) {
-            const int i = base + ln;
-            int x = INT_MAX;
-            if (i < len) x = with_slot<GS>(C, o.father, [&](auto p) { return p[i]; });
-            bool use = i < len && x < t;
-            for (int f = 0; f < d; f++)
-                if (o.excl >> f & 1u) use = use && x != S->val[f];
-            int cnt = 0;
-            const int pos = use ? lbound(a.adj + vb, deg, x) : 0;
-            if (use) cnt = edge[pos].read();
-            const bool need = use && cnt < 0;
-            if (ballot(need)) {
-                const int fresh = sweep_kept<GS>(C, N.loop_slot, need, x, b);
-                if (need) {
-                    cnt = fresh;
-                    edge[pos].write(fresh);
-                }
+    const GatOp &o = C.P.ops[N.op_begin + k];
+    const int v = uni(S->val[C.P.slots[N.loop_slot].depth]);  // v_j
+    const long long vb = a.off[v];
+    const int deg = (int)(a.off[v + 1] - vb), b = o.table ? v : INT_MAX;
+    const int t = uni(group_bound(S, o.groups, o.ngroups, d, 0));
+    KeptEdge *edge = a.edge_tab[o.table] + vb;
+    unsigned long long sum = 0;
+    for (int base = lo; base < hi; base += W) {
+        const int i = base + ln;
+        int x = INT_MAX;
+        if (i < hi) x = with_slot<GS>(C, o.father, [&](auto p) { return p[i]; });
+        bool use = i < hi && x < t;
+        for (int f = 0; f < d; f++)
+            if (o.excl >> f & 1u) use = use && x != S->val[f];
+        int cnt = 0;
+        const int pos = use ? lbound(a.adj + vb, deg, x) : 0;
+        if (use) cnt = edge[pos].read();
+        bool need = use && cnt < 0;
+        if (ballot(need) && can_split && hi - base > 1 && queue_drained<GS>(a)) {
+            const long long lw = need ? min((long long)deg, a.off[x + 1] - a.off[x]) : 0;
+            const long long tot = uni64((long long)wave_sum64((unsigned long long)lw));
+            const int kept = 3 * tot * kTailShare > a.split_ticks ? base + 1 : base + W;
+            if (kept < hi && 3 * tot * kTailShare * (hi - base) > a.split_ticks * W &&
+                donate(C, d, node, kept, hi, 1, !GS, k)) {
+                hi = kept;
+                use = use && i < hi;
+                need = need && i < hi;
             }
-            // candidates that are skipped or empty although they lie in N(v_j)
-            // below b: chosen vertices (each once)
-            for (int f = 0; f < d; f++) {
-                const unsigned out = N.excl | N.ap_levels;
-                if (!(out >> f & 1u)) continue;
-                const int y = uni(S->val[f]), hy = uni(hub_of(a, y));
-                bool once = y < b;
-                for (int h = 0; h < f; h++) once = once && !((out >> h & 1u) && S->val[h] == y);
-                once = adjacent(a, y, hy, v, once);
-                if (uni((int)once)) cnt -= adjacent(a, y, hy, x, use);
-            }
-            if (use) sum += (unsigned long long)(long long)cnt;
         }
-        sum = wave_sum64(sum);
-        if (ln == 0)
-            for (int u = 0; u < N.term_count; u++) {
-                const GatTerm &T = C.P.terms[N.term_begin + u];
-                for (int q = 0; q < T.sub_count; q++) {
-                    const GatSub &sb = C.P.subs[T.sub_begin + q];
-                    if (C.P.vids[sb.vid].slot == o.slot) S->task_acc[T.pattern] += sum * (unsigned long long)(long long)sb.coef;
-                }
+        if (ballot(need)) {
+            const int fresh = sweep_kept<GS>(C, N.loop_slot, need, x, b);
+            if (need) {
+                cnt = fresh;
+                edge[pos].write(fresh);
             }
+        }
+        // candidates that are skipped or empty although they lie in N(v_j)
+        // below b: chosen vertices (each once)
+        for (int f = 0; f < d; f++) {
+            const unsigned out = N.excl | N.ap_levels;
+            if (!(out >> f & 1u)) continue;
+            const int y = uni(S->val[f]), hy = uni(hub_of(a, y));
+            bool once = y < b;
+            for (int h = 0; h < f; h++) once = once && !((out >> h & 1u) && S->val[h] == y);
+            once = adjacent(a, y, hy, v, once);
+            if (uni((int)once)) cnt -= adjacent(a, y, hy, x, use);
+        }
+        if (use) sum += (unsigned long long)(long long)cnt;
     }
+    sum = wave_sum64(sum);
+    if (ln == 0)
+        for (int u = 0; u < N.term_count; u++) {
+            const GatTerm &T = C.P.terms[N.term_begin + u];
+            for (int q = 0; q < T.sub_count; q++) {
+                const GatSub &sb = C.P.subs[T.sub_begin + q];
+                if (C.P.vids[sb.vid].slot == o.slot) S->task_acc[T.pattern] += sum * (unsigned long long)(long long)sb.coef;
+            }
+        }
     wsync();
 }
 
@@ -1102,7 +1119,11 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
     // Parts of a frame that was split have cur > 0; a frame handed on whole is
     // left empty here. So the part with the first candidate adds the sums, and
     // an empty frame has none.
-    if (KEEP && d >= 2 && cur == 0 && hi > 0) leaf_sums<GS>(C, N, d);
+    for (int k = 0; KEEP && d >= 2 && cur == 0 && hi > 0 && k < N.op_count; k++) {
+        const GatOp &o = C.P.ops[N.op_begin + k];
+        if (o.kind == GATP_COUNT && o.keep == GATP_KEEP_SUM)
+            leaf_sum<GS>(C, N, d, node, k, 0, uni(S->slen[o.father]), can_split);
+    }
     for (int cb = cur; cb < hi; cb += W) {
         const int ci = cb + ln;
         int c = 0;
@@ -1143,7 +1164,7 @@ __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int 
             KeptEdge *edge = nullptr;
             KeptEntry *slot = nullptr;
             unsigned tag = 0;
-            if (KEEP && o.keep == GATP_KEEP_SUM) {  // added by leaf_sums
+            if (KEEP && o.keep == GATP_KEEP_SUM) {  // added by leaf_sum
                 S->leafcnt[o.leaf_idx][ln] = 0;
                 continue;
             }
@@ -1554,6 +1575,11 @@ __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
     wsync();
     if (!ok) return;
     const bool can_split = !GS && a.sub_mode < kSplitLevels;
+    const int sum_op = KEEP ? uni(g->pos[0]) - 1 : -1;
+    if (KEEP && sum_op >= 0) {
+        leaf_sum<GS>(C, P.nodes[sub_node], D, sub_node, sum_op, sub_lo, sub_hi, can_split);
+        return;
+    }
     push_frame<GS>(C, D, sub_node, sub_lo, sub_hi);
     int d = D;
     while (d >= D) {

@@ -29,3 +29,23 @@ def test_long_rest_is_handed_on_before_the_budget(gat, gpu, mode):
     got, st = plan.count_shard_edges(e, e + 1, {"split_us": int(budget_ms * 1e3)})
     assert got == want
     assert st["main_kernel_ms"] < budget_ms and st["split_tasks"] > 0, (budget_ms, st)
+
+
+def test_sum_over_the_father_is_split(gat, gpu):
+    """A leaf whose count is summed over the father set of one edge between two
+    hubs (about 7 of the 29 ms that one wave takes): its entries go to several
+    waves, in the LDS launches and, with small set buffers, in the HBM launch."""
+    pattern = "0010100011100110110111110"
+    g = gat.Graph.chung_lu(300007, 24.0, 2.1, 20000, 1)
+    plan = gat.Plan(g, [pattern], "unique")
+    e = int(plan.run_offsets()[1000])
+    plan.count_shard_edges(e, e + 1)
+    want, alone = plan.count_shard_edges(e, e + 1, {"split_us": -1})
+    budget_ms = alone["main_kernel_ms"] / 8
+    assert alone["overflow_tasks"] == 0
+    got, st = plan.count_shard_edges(e, e + 1, {"split_us": int(budget_ms * 1e3)})
+    assert got == want
+    assert st["main_kernel_ms"] < budget_ms, (budget_ms, st)
+    for us in (1, 100, 2000):
+        got, st = plan.count_shard_edges(e, e + 1, {"split_us": us, "slot_capacity": 16})
+        assert got == want and st["overflow_tasks"] == 1 and st["split_tasks"] > 0, (us, got, st)
