@@ -1107,23 +1107,25 @@ __device__ __forceinline__ void leaf_sum(const Ctx &C, const GatNode &N, int d, 
 
 // All candidates of a leaf frame, flattened across lanes.
 // With can_split, a wave that is due to split (want_split) hands the
-// batches after the current one to the next split launch.
+// batches after the current one to the next split launch. With sum_op, the
+// range is one of that op's father (see SplitTask) and nothing else is done.
 template <bool GS, bool KEEP>
 __device__ __forceinline__ void leaf(const Ctx &C, const GatNode &N, int d, int cur, int hi, bool can_split = false,
-                                     int node = -1) {
+                                     int node = -1, int sum_op = -1) {
     const KArgs &a = C.a;
     WaveState *S = C.S;
     const int ln = C.ln;
     unsigned long long bytes = 0;
-    if (KEEP) leaf_exclusions(C, N, d);
+    if (KEEP && sum_op < 0) leaf_exclusions(C, N, d);
     // Parts of a frame that was split have cur > 0; a frame handed on whole is
     // left empty here. So the part with the first candidate adds the sums, and
     // an empty frame has none.
-    for (int k = 0; KEEP && d >= 2 && cur == 0 && hi > 0 && k < N.op_count; k++) {
+    for (int k = 0; KEEP && d >= 2 && (sum_op >= 0 || (cur == 0 && hi > 0)) && k < N.op_count; k++) {
         const GatOp &o = C.P.ops[N.op_begin + k];
-        if (o.kind == GATP_COUNT && o.keep == GATP_KEEP_SUM)
-            leaf_sum<GS>(C, N, d, node, k, 0, uni(S->slen[o.father]), can_split);
+        if (o.kind != GATP_COUNT || o.keep != GATP_KEEP_SUM || (sum_op >= 0 && k != sum_op)) continue;
+        leaf_sum<GS>(C, N, d, node, k, sum_op >= 0 ? cur : 0, sum_op >= 0 ? hi : uni(S->slen[o.father]), can_split);
     }
+    if (KEEP && sum_op >= 0) return;
     for (int cb = cur; cb < hi; cb += W) {
         const int ci = cb + ln;
         int c = 0;
@@ -1577,17 +1579,22 @@ __device__ __forceinline__ void run_sub(const Ctx &C, const SplitTask *g) {
     const bool can_split = !GS && a.sub_mode < kSplitLevels;
     const int sum_op = KEEP ? uni(g->pos[0]) - 1 : -1;
     if (KEEP && sum_op >= 0) {
-        leaf_sum<GS>(C, P.nodes[sub_node], D, sub_node, sum_op, sub_lo, sub_hi, can_split);
-        return;
+        if (C.ln == 0) {
+            S->f_node[D] = sub_node;
+            S->f_cur[D] = sub_lo;
+            S->f_hi[D] = sub_hi;
+        }
+        wsync();
+    } else {
+        push_frame<GS>(C, D, sub_node, sub_lo, sub_hi);
     }
-    push_frame<GS>(C, D, sub_node, sub_lo, sub_hi);
     int d = D;
     while (d >= D) {
         const int node = uni(S->f_node[d]);
         const GatNode &N = P.nodes[node];
         bool exhausted = false;
         if (N.leaf) {
-            leaf<GS, KEEP>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node);
+            leaf<GS, KEEP>(C, N, d, uni(S->f_cur[d]), uni(S->f_hi[d]), can_split, node, sum_op);
             exhausted = true;
         } else if (PAIR && N.pair) {
             const int cur = uni(S->f_cur[d]), fh = uni(S->f_hi[d]);
