@@ -25,6 +25,7 @@
 #include <cstdio>
 #include <cstring>
 #include <numeric>
+#include <set>
 #include <type_traits>
 #include <vector>
 
@@ -2895,27 +2896,62 @@ struct HubRows {
     }
 };
 
+// Core bitmap of the clique store: the rows of the vertices [0, n), shared like
+// the hub rows.
+struct CoreRows {
+    int n = 0;
+    unsigned *bits = nullptr;
+    ~CoreRows() {
+        if (bits) (void)hipFree(bits);
+    }
+};
+
+// Memory that makes counts faster and that they can do without (bitmaps of a
+// graph, tables of kept counts of a plan) stays with the graph or plan. What
+// holds some of it is listed here: an allocation that a count cannot do without
+// and that finds no memory takes it from those that no count is using (need_malloc).
+struct PlanDevice;
+struct DeviceGraph;
+struct Holders {
+    std::mutex mu;
+    std::set<PlanDevice *> plans;
+    std::set<DeviceGraph *> graphs;
+};
+static Holders &holders() {
+    static Holders *h = new Holders;  // plans may be freed after this file's statics
+    return *h;
+}
+// After an optional allocation found no memory, the next kRetry counts do not
+// ask for it again.
+constexpr int kRetry = 64;
+
 struct DeviceGraph {
     long long *off = nullptr;
     int *adj = nullptr;
     int *split = nullptr;
-    std::mutex mu;  // held while the bitmaps are built
-    // core bitmap of the clique store (core_n < 0: not built)
-    unsigned *core = nullptr;
-    int core_n = -1;
+    std::mutex mu;  // guards what follows; held while the bitmaps are built
+    std::shared_ptr<CoreRows> core;
     std::shared_ptr<HubRows> hubs;
-    std::vector<int> at_least;     // at_least[d]: vertices of degree >= d, d <= max_deg + 1
-    bool ordered = false;          // ids by descending degree
-    size_t hubs_short = SIZE_MAX;  // a set of so many rows found no memory
+    std::vector<int> at_least;  // at_least[d]: vertices of degree >= d, d <= max_deg + 1
+    bool ordered = false;       // ids by descending degree
+    int hubs_wait = 0;          // counts until the optional rows are asked for again
+    DeviceGraph() {
+        std::lock_guard<std::mutex> lk(holders().mu);
+        holders().graphs.insert(this);
+    }
     ~DeviceGraph() {
+        {
+            std::lock_guard<std::mutex> lk(holders().mu);
+            holders().graphs.erase(this);
+        }
         if (off) (void)hipFree(off);
         if (adj) (void)hipFree(adj);
         if (split) (void)hipFree(split);
-        if (core) (void)hipFree(core);
     }
 };
 
 struct PlanDevice {
+    std::mutex busy;  // held by a count from its preparation to its end
     hipStream_t stream = nullptr;
     GatPlanDev *plan = nullptr;
     unsigned long long *ctl = nullptr;      // control words (kCtl*)
@@ -2936,6 +2972,7 @@ struct PlanDevice {
     unsigned pool_tables = 0, epoch = 0;
     int tab_size = 0;
     bool keep = false;
+    int tables_wait = 0;  // counts until tables are asked for again
     int ovf_grid = 0;
     hipEvent_t ev[4] = {};
     // clique HBM-tier rows and pair offsets
@@ -2946,22 +2983,102 @@ struct PlanDevice {
     // captured graph
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
+    PlanDevice() {
+        std::lock_guard<std::mutex> lk(holders().mu);
+        holders().plans.insert(this);
+    }
+    // Frees the tables of kept counts; true if there were any.
+    bool drop_tables() {
+        bool any = false;
+        for (auto &t : edge_tab)
+            if (t) {
+                (void)hipFree(t);
+                t = nullptr;
+                any = true;
+            }
+        if (pool) {
+            (void)hipFree(pool);
+            pool = nullptr;
+            any = true;
+        }
+        keep = false;
+        return any;
+    }
 };
 
 void destroy_plan_device(PlanDevice *d) {
     if (!d) return;
+    {
+        std::lock_guard<std::mutex> lk(holders().mu);
+        holders().plans.erase(d);
+    }
+    d->drop_tables();
     if (d->gexec) (void)hipGraphExecDestroy(d->gexec);
     if (d->graph) (void)hipGraphDestroy(d->graph);
     for (auto &e : d->ev)
         if (e) (void)hipEventDestroy(e);
     for (void *p : {(void *)d->plan, (void *)d->dargs, (void *)d->tl, (void *)d->ctl, (void *)d->ovf, (void *)d->subs, (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2], (void *)d->tier[3],
-                    (void *)d->gstore, (void *)d->edge_tab[0], (void *)d->edge_tab[1], (void *)d->edge_tab[2],
-                    (void *)d->edge_tab[3], (void *)d->pool, (void *)d->grows,
-                    (void *)d->goff})
+                    (void *)d->gstore, (void *)d->grows, (void *)d->goff})
         if (p) (void)hipFree(p);
     if (d->result) (void)hipHostFree(d->result);
     if (d->stream) (void)hipStreamDestroy(d->stream);
     delete d;
+}
+
+// Memory that a count can do without: false, and *p null, if there is none left.
+template <class T>
+static bool try_malloc(T **p, size_t bytes, int *rc) {
+    *p = nullptr;
+    const hipError_t e = hipMalloc((void **)p, bytes);
+    if (e == hipSuccess) return true;
+    *p = nullptr;
+    (void)hipGetLastError();
+    if (e != hipErrorOutOfMemory) {
+        gat::set_error("hipMalloc failed: %s", hipGetErrorString(e));
+        *rc = GAT_ENODEV;
+    }
+    return false;
+}
+
+// Frees what idle plans and graphs can do without; true if that was anything.
+// mine, if given, is a plan whose lock the caller holds (prepared: its tables
+// are in the arguments of a count already), and locked a graph whose lock it holds.
+static bool give_back(PlanDevice *mine, bool prepared, const DeviceGraph *locked) {
+    Holders &h = holders();
+    std::lock_guard<std::mutex> lk(h.mu);
+    bool any = mine && !prepared && mine->drop_tables();
+    for (PlanDevice *d : h.plans) {
+        if (d == mine || !d->busy.try_lock()) continue;
+        any |= d->drop_tables();
+        d->busy.unlock();
+    }
+    for (DeviceGraph *g : h.graphs) {
+        if (g == locked || !g->mu.try_lock()) continue;
+        // a count holds its graph's bitmaps and takes them under the graph's lock
+        if (g->hubs && g->hubs.use_count() == 1) {
+            g->hubs.reset();
+            any = true;
+        }
+        if (g->core && g->core.use_count() == 1) {
+            g->core.reset();
+            any = true;
+        }
+        g->mu.unlock();
+    }
+    return any;
+}
+
+bool give_back_memory() { return give_back(nullptr, false, nullptr); }
+
+// Memory that a count cannot do without (mine, prepared, locked: see give_back).
+template <class T>
+static int need_malloc(T **p, size_t bytes, PlanDevice *mine, const DeviceGraph *locked = nullptr, bool prepared = false) {
+    int rc = GAT_OK;
+    if (try_malloc(p, bytes, &rc)) return GAT_OK;
+    if (rc) return rc;
+    if (give_back(mine, prepared, locked) && try_malloc(p, bytes, &rc)) return GAT_OK;
+    if (!rc) GAT_FAIL(GAT_ENODEV, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(hipErrorOutOfMemory));
+    return rc;
 }
 
 static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
@@ -2971,9 +3088,10 @@ static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
         return GAT_OK;
     }
     auto dg = std::make_shared<DeviceGraph>();
-    HIPCHECK(hipMalloc(&dg->off, sizeof(long long) * (size_t(g.n) + 1)));
-    HIPCHECK(hipMalloc(&dg->adj, sizeof(int) * std::max<size_t>(1, size_t(g.m))));
-    HIPCHECK(hipMalloc(&dg->split, sizeof(int) * std::max<size_t>(1, size_t(g.n))));
+    int rc = need_malloc(&dg->off, sizeof(long long) * (size_t(g.n) + 1), nullptr);
+    if (!rc) rc = need_malloc(&dg->adj, sizeof(int) * std::max<size_t>(1, size_t(g.m)), nullptr);
+    if (!rc) rc = need_malloc(&dg->split, sizeof(int) * std::max<size_t>(1, size_t(g.n)), nullptr);
+    if (rc) return rc;
     HIPCHECK(hipMemcpy(dg->off, g.off.data(), sizeof(long long) * (size_t(g.n) + 1), hipMemcpyHostToDevice));
     if (g.m) HIPCHECK(hipMemcpy(dg->adj, g.adj.data(), sizeof(int) * size_t(g.m), hipMemcpyHostToDevice));
     if (g.n) {
@@ -3000,21 +3118,6 @@ static int32_t max_out_degree(Graph &g) {
     return g.max_out;
 }
 
-// Memory that a count can do without: false, and *p null, if there is none left.
-template <class T>
-static bool try_malloc(T **p, size_t bytes, int *rc) {
-    *p = nullptr;
-    const hipError_t e = hipMalloc((void **)p, bytes);
-    if (e == hipSuccess) return true;
-    *p = nullptr;
-    (void)hipGetLastError();
-    if (e != hipErrorOutOfMemory) {
-        gat::set_error("hipMalloc failed: %s", hipGetErrorString(e));
-        *rc = GAT_ENODEV;
-    }
-    return false;
-}
-
 // Neighbourhood bitmaps, most connected vertices first, within kHubBytes: of
 // every vertex of degree >= the configured threshold, or by default of those of
 // degree >= kHubDegree and, within kHubMoreBytes, of further ones down to
@@ -3036,12 +3139,16 @@ struct HubUse {
     int n = 0, full = INT_MAX;
 };
 
-static int build_hubs(const Graph &g, DeviceGraph *dg, size_t n, int least, std::shared_ptr<HubRows> *out) {
+// optional: *out stays empty where there is no memory for the rows.
+static int build_hubs(const Graph &g, DeviceGraph *dg, size_t n, int least, bool optional, PlanDevice *mine,
+                      std::shared_ptr<HubRows> *out) {
     const long long words = ((long long)g.n + 31) / 32, n_u64 = ((long long)n * words + 1) / 2;
     auto h = std::make_shared<HubRows>();
     h->n = n;
     int rc = GAT_OK;
-    if (!try_malloc(&h->bits, 8 * (size_t)n_u64, &rc)) return rc;  // *out stays empty
+    if (optional) try_malloc(&h->bits, 8 * (size_t)n_u64, &rc);
+    else rc = need_malloc(&h->bits, 8 * (size_t)n_u64, mine, dg);
+    if (rc || !h->bits) return rc;
     hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, nullptr, (unsigned long long *)h->bits, n_u64, 0ull);
     if (!dg->ordered) {
         std::vector<int32_t> hubs, map(size_t(g.n), -1);
@@ -3050,8 +3157,9 @@ static int build_hubs(const Graph &g, DeviceGraph *dg, size_t n, int least, std:
         std::stable_sort(hubs.begin(), hubs.end(), [&](int32_t x, int32_t y) { return g.deg(x) > g.deg(y); });
         hubs.resize(n);
         for (size_t k = 0; k < n; k++) map[hubs[k]] = int32_t(k);
-        HIPCHECK(hipMalloc(&h->map, sizeof(int) * size_t(g.n)));
-        HIPCHECK(hipMalloc(&h->vertex, sizeof(int) * n));
+        rc = need_malloc(&h->map, sizeof(int) * size_t(g.n), mine, dg);
+        if (!rc) rc = need_malloc(&h->vertex, sizeof(int) * n, mine, dg);
+        if (rc) return rc;
         HIPCHECK(hipMemcpy(h->map, map.data(), sizeof(int) * size_t(g.n), hipMemcpyHostToDevice));
         HIPCHECK(hipMemcpy(h->vertex, hubs.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     }
@@ -3066,7 +3174,7 @@ static int build_hubs(const Graph &g, DeviceGraph *dg, size_t n, int least, std:
 // thr: the configured threshold, 0 for the default. The graph's rows serve if
 // there are enough of them; else they are built anew, and on a failure the
 // graph is left without any, for the next count to build.
-static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr, HubUse *out) {
+static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr, PlanDevice *mine, HubUse *out) {
     std::lock_guard<std::mutex> lk(dg->mu);
     if (dg->at_least.empty()) {
         std::vector<int> c((size_t)g.max_deg + 2, 0);
@@ -3086,19 +3194,22 @@ static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr, HubUse *out) {
     const size_t found = vertices(least), most = (size_t)(kHubBytes / row_bytes);
     const size_t always = std::min(thr ? found : vertices(std::max(least, kHubDegree)), most);  // rows that only kHubBytes limits
     size_t n = std::min({found, std::max(always, (size_t)(kHubMoreBytes / row_bytes)), most});
-    if (n > always && n >= dg->hubs_short) n = always;
-    if (n && (!dg->hubs || dg->hubs->n < n)) {
-        dg->hubs.reset();
-        std::shared_ptr<HubRows> rows;
-        int rc = build_hubs(g, dg, n, least, &rows);
-        if (!rc && !rows && n > always) {  // the rows beyond kHubDegree only where there is room
-            dg->hubs_short = n;
-            n = always;
-            rc = n ? build_hubs(g, dg, n, least, &rows) : GAT_OK;
+    auto missing = [&] { return n > (dg->hubs ? dg->hubs->n : 0); };
+    if (missing() && n > always) {  // the rows beyond kHubDegree only where there is room
+        if (dg->hubs_wait > 0) {
+            dg->hubs_wait--;
+        } else {
+            std::shared_ptr<HubRows> rows;
+            const int rc = build_hubs(g, dg, n, least, true, mine, &rows);
+            if (rc) return rc;
+            if (rows) dg->hubs = rows; else dg->hubs_wait = kRetry;
         }
+        if (missing()) n = always;
+    }
+    if (missing()) {
+        dg->hubs.reset();
+        const int rc = build_hubs(g, dg, n, least, false, mine, &dg->hubs);
         if (rc) return rc;
-        if (!rows && n) GAT_FAIL(GAT_ENODEV, "no device memory for the bitmaps of %zu vertices", n);
-        dg->hubs = rows;
     }
     out->rows = dg->hubs;
     out->n = (int)n;
@@ -3124,26 +3235,32 @@ static int core_vertices(int64_t n, long long words) {
     return lo;
 }
 
-static int ensure_core(const Graph &g, DeviceGraph *dg) {
-    std::lock_guard<std::mutex> lk(dg->mu);  // plans of one graph may be first counted on different threads
-    if (dg->core_n >= 0) return GAT_OK;
-    long long budget = std::max<long long>(1 << 21, 4ll * g.m);
-    int h = core_vertices(g.n, budget);
-    int rc = GAT_OK;
-    // fewer core vertices where memory is short
-    while (!try_malloc(&dg->core, sizeof(unsigned) * std::max<size_t>(gatk::core_row(h), 16), &rc)) {
-        if (rc) return rc;
-        if (budget <= 1 << 21) GAT_FAIL(GAT_ENODEV, "no device memory for the core bitmap (%d rows)", h);
-        budget = std::max<long long>(1 << 21, budget / 4);
-        h = core_vertices(g.n, budget);
+static int ensure_core(const Graph &g, DeviceGraph *dg, std::shared_ptr<CoreRows> *out) {
+    std::lock_guard<std::mutex> lk(dg->mu);
+    if (dg->core) {
+        *out = dg->core;
+        return GAT_OK;
     }
-    if (h > 0) {
-        hipLaunchKernelGGL(gatk::core_rows_kernel, dim3(std::min((h + 3) / 4, 4096)), dim3(256), 0, nullptr, dg->off,
-                           dg->adj, dg->split, h, dg->core);
+    auto c = std::make_shared<CoreRows>();
+    int rc = GAT_OK;
+    // fewer core vertices where memory is short, down to none
+    for (long long budget = std::max<long long>(1 << 21, 4ll * g.m);; budget = std::max<long long>(1 << 21, budget / 4)) {
+        c->n = core_vertices(g.n, budget);
+        if (try_malloc(&c->bits, sizeof(unsigned) * std::max<size_t>(gatk::core_row(c->n), 16), &rc)) break;
+        if (rc) return rc;
+        if (budget <= 1 << 21) {
+            c->n = 0;
+            break;
+        }
+    }
+    if (c->n > 0) {
+        hipLaunchKernelGGL(gatk::core_rows_kernel, dim3(std::min((c->n + 3) / 4, 4096)), dim3(256), 0, nullptr, dg->off,
+                           dg->adj, dg->split, c->n, c->bits);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipDeviceSynchronize());
     }
-    dg->core_n = h;
+    dg->core = c;
+    *out = c;
     return GAT_OK;
 }
 
@@ -3188,7 +3305,9 @@ struct Launch {
     bool edge_grain = false;  // the HBM launch takes single edges
     bool may_overflow = true; // some intersection may outgrow its LDS buffer
     bool pair = false;        // the plan has nodes swept with their leaf (GatNode::pair)
-    HubUse hubs;              // kept for as long as the count may read them
+    std::unique_lock<std::mutex> busy;  // of the plan
+    HubUse hubs;                        // kept, like the core rows, for as long as the count may read them
+    std::shared_ptr<CoreRows> core;
     bool heavy = false;   // clique: some vertex may have more than main_max neighbours below it
 };
 
@@ -3268,33 +3387,41 @@ static int clique_shape(const DeviceInfo &di, const gat_kernel_config &cfg, int 
 // Tables of kept COUNT values (GATP_KEEP_*): an int per directed edge and
 // truncation, cleared by every count, and the pools. A pool's table covers the
 // first kTabVertices vertices (of a degree-ordered graph the most visited
-// ones); there are as many tables as kPoolBytes for all pools holds. Values
-// have 24 bits and keys 32: larger graphs go without.
-constexpr long long kPoolBytes = 1ll << 29;
+// ones); there are as many tables as kPoolBytes for all pools holds, or where
+// memory is short a quarter, a sixteenth or a 64th of that. Values have 24 bits
+// and keys 32: larger graphs go without.
+constexpr long long kPoolBytes = 1ll << 29, kPoolLeast = 1ll << 23;
 constexpr int kTabVertices = 1 << 14;
 static int ensure_tables(gat_plan *p) {
     PlanDevice *d = p->dev;
     const GatPlanDev &pd = p->cp.dev;
     const Graph &g = *p->graph;
+    if (d->keep || !(pd.edge_tables || pd.n_tables)) return GAT_OK;
     if (g.m == 0 || g.max_deg >= 1 << 24 || g.m >= (1ll << 32) - 1) return GAT_OK;
-    d->keep = 0;
-    int rc = GAT_OK;
-    for (int k = 0; k < 4; k++)
-        if ((pd.edge_tables >> k & 1) && !d->edge_tab[k] &&
-            !try_malloc(&d->edge_tab[k], sizeof(gatk::KeptEdge) * (((size_t)g.m + 1) / 2 * 2), &rc))
-            return rc;
-    if (pd.n_tables == 0 || d->pool) {
-        d->keep = pd.edge_tables || pd.n_tables;
+    if (d->tables_wait > 0) {
+        d->tables_wait--;
         return GAT_OK;
     }
+    int rc = GAT_OK;
+    bool all = true;
+    for (int k = 0; k < 4 && all; k++)
+        if (pd.edge_tables >> k & 1)
+            all = try_malloc(&d->edge_tab[k], sizeof(gatk::KeptEdge) * (((size_t)g.m + 1) / 2 * 2), &rc);
     d->tab_size = std::min(g.n, kTabVertices);
-    const long long most = kPoolBytes / (8ll * pd.n_tables * d->tab_size);
-    d->pool_tables = (unsigned)std::max(1ll, std::min<long long>(most, pd.key_edges ? g.m : g.n));
-    d->pool_entries = (long long)pd.n_tables * d->pool_tables * d->tab_size;
-    if (!try_malloc(&d->pool, sizeof(gatk::KeptEntry) * d->pool_entries, &rc)) return rc;
-    d->epoch = 255;  // cleared by the first count
-    d->keep = 1;
-    return GAT_OK;
+    for (long long bytes = kPoolBytes; all && pd.n_tables && !d->pool; bytes /= 4) {
+        const long long most = bytes / (8ll * pd.n_tables * d->tab_size);
+        d->pool_tables = (unsigned)std::max(1ll, std::min<long long>(most, pd.key_edges ? g.m : g.n));
+        d->pool_entries = (long long)pd.n_tables * d->pool_tables * d->tab_size;
+        d->epoch = 255;  // cleared by the first count
+        if (!try_malloc(&d->pool, sizeof(gatk::KeptEntry) * d->pool_entries, &rc)) all = !rc && bytes > kPoolLeast;
+    }
+    if (all) {
+        d->keep = true;
+    } else {
+        d->drop_tables();
+        d->tables_wait = kRetry;
+    }
+    return rc;
 }
 
 static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
@@ -3310,20 +3437,22 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     if (cfg.block_waves > 4) GAT_FAIL(GAT_EINFEASIBLE, "block_waves %d > 4", cfg.block_waves);
     Graph &g = *p->graph;
     const GatPlanDev &pd = p->cp.dev;
-    if (!p->dev) {
-        auto *d = new PlanDevice();
-        p->dev = d;
+    if (!p->dev) {  // complete or not at all: after a failure the next count starts over
+        std::unique_ptr<PlanDevice, void (*)(PlanDevice *)> d(new PlanDevice(), destroy_plan_device);
         rc = ensure_device_graph(g, &d->dg);
         if (rc) return rc;
         HIPCHECK(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
-        HIPCHECK(hipMalloc(&d->plan, sizeof(GatPlanDev)));
+        rc = need_malloc(&d->plan, sizeof(GatPlanDev), nullptr);
+        if (!rc) rc = need_malloc(&d->ctl, sizeof(unsigned long long) * kCtlWords, nullptr);
+        if (!rc) rc = need_malloc(&d->dargs, sizeof(gatk::KArgsSet), nullptr);
+        if (rc) return rc;
         HIPCHECK(hipMemcpy(d->plan, &pd, sizeof(GatPlanDev), hipMemcpyHostToDevice));
-        HIPCHECK(hipMalloc(&d->ctl, sizeof(unsigned long long) * kCtlWords));
         HIPCHECK(hipHostMalloc((void **)&d->result, sizeof(unsigned long long) * kCtlResult, hipHostMallocDefault));
-        HIPCHECK(hipMalloc(&d->dargs, sizeof(gatk::KArgsSet)));
         for (auto &e : d->ev) HIPCHECK(hipEventCreate(&e));
+        p->dev = d.release();
     }
     PlanDevice *d = p->dev;
+    L->busy = std::unique_lock<std::mutex>(d->busy);
     const long long chunk = cfg.queue_chunk;
     const bool clique = p->cp.clique_ks != 0 && cfg.vertex_store != 1;
     if (!clique && !d->gstore) {
@@ -3335,7 +3464,8 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         while (waves > 64 && (double)waves * per_wave > 4.0 * (1 << 30)) waves /= 2;
         d->ovf_grid = waves;
         d->gstore_bytes = (size_t)waves * per_wave;
-        HIPCHECK(hipMalloc(&d->gstore, std::max<size_t>(d->gstore_bytes, 64)));
+        rc = need_malloc(&d->gstore, std::max<size_t>(d->gstore_bytes, 64), d);
+        if (rc) return rc;
     }
     if (cfg.vertex_store == 2 && !clique)
         GAT_FAIL(GAT_EINFEASIBLE, "bitmap vertex store needs a plan of cliques K3..K6 in unique or labeled mode");
@@ -3348,11 +3478,16 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     const bool split = !clique && cfg.split_us > 0;
     // subtask lists: the LDS levels (kSubCap each), then the HBM list (LDS
     // overflow of the levels plus the HBM launch's splits, 3 kSubCap)
-    if (split && !d->subs) HIPCHECK(hipMalloc(&d->subs, sizeof(gatk::SplitTask) * (kLevels + 3) * kSubCap));
+    if (split && !d->subs) {
+        rc = need_malloc(&d->subs, sizeof(gatk::SplitTask) * (kLevels + 3) * kSubCap, d);
+        if (rc) return rc;
+    }
     if (ovf_cap > d->ovf_cap) {
         if (d->ovf) HIPCHECK(hipFree(d->ovf));
         d->ovf = nullptr;
-        HIPCHECK(hipMalloc(&d->ovf, sizeof(long long) * ovf_cap));
+        d->ovf_cap = 0;
+        rc = need_malloc(&d->ovf, sizeof(long long) * ovf_cap, d);
+        if (rc) return rc;
         d->ovf_cap = ovf_cap;
     }
     // A wave's LDS: its state (with the leaf counters the plan needs) and its
@@ -3367,7 +3502,7 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     const int state_bytes = int((sizeof(gatk::WaveState) -
                                  size_t(GATP_MAX_LEAF_OPS - pd.max_leaf_ops) * sizeof(int) * 64 + 15) / 16 * 16);
     if (!clique && cfg.hub_degree >= 0) {
-        rc = ensure_hubs(g, d->dg.get(), cfg.hub_degree, &L->hubs);
+        rc = ensure_hubs(g, d->dg.get(), cfg.hub_degree, d, &L->hubs);
         if (rc) return rc;
     }
     const int staged = !clique && cfg.hub_degree >= 0 ? std::min(cfg.slot_capacity, L->hubs.full) : cfg.slot_capacity;
@@ -3455,14 +3590,14 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
     L->clique = clique;
     if (clique) {
         const int max_out = max_out_degree(g);
-        rc = ensure_core(g, d->dg.get());
+        rc = ensure_core(g, d->dg.get(), &L->core);
         if (rc) return rc;
         gatk::CArgs c{};
         c.off = a.off;
         c.adj = a.adj;
         c.split = a.split;
-        c.core = d->dg->core;
-        c.core_n = d->dg->core_n;
+        c.core = L->core->bits;
+        c.core_n = L->core->n;
         c.n = a.n;
         c.m = a.m;
         c.root_lo = 0;
@@ -3478,7 +3613,10 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         rc = clique_shape(di, cfg, max_out, L);
         if (rc) return rc;
         for (int t = 0; t < gatk::CTIERS; t++) {
-            if (L->tier_grid[t].x && !d->tier[t]) HIPCHECK(hipMalloc(&d->tier[t], sizeof(int) * ((size_t)g.n + 1)));
+            if (L->tier_grid[t].x && !d->tier[t]) {
+                rc = need_malloc(&d->tier[t], sizeof(int) * ((size_t)g.n + 1), d);
+                if (rc) return rc;
+            }
             L->ca.tier[t] = d->tier[t];
             L->ca.tier_cap[t] = d->tier[t] ? g.n + 1ll : 0;
         }
@@ -3492,8 +3630,10 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
                 if (d->goff) HIPCHECK(hipFree(d->goff));
                 d->grows = nullptr;
                 d->goff = nullptr;
-                HIPCHECK(hipMalloc(&d->grows, (size_t)groups * hcap * ws * 4));
-                HIPCHECK(hipMalloc(&d->goff, (size_t)groups * (hcap + 1) * 4));
+                d->big_cap = d->big_groups = 0;
+                rc = need_malloc(&d->grows, (size_t)groups * hcap * ws * 4, d);
+                if (!rc) rc = need_malloc(&d->goff, (size_t)groups * (hcap + 1) * 4, d);
+                if (rc) return rc;
                 d->big_cap = hcap;
                 d->big_groups = groups;
             }
@@ -3540,7 +3680,10 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
                                         : (long long)waves * (1 + (L.a.split_ticks > 0 ? kLevels : 0)) +
                                               (long long)L.ovf_grid.x * (L.a.split_ticks > 0 ? 2 : 1);
         if (need > kTlCap) GAT_FAIL(GAT_ELIMIT, "timeline needs %lld records (> %d)", need, kTlCap);
-        if (!d->tl) HIPCHECK(hipMalloc(&d->tl, sizeof(long long) * gatk::kTlFields * kTlCap));
+        if (!d->tl) {
+            const int rc = need_malloc(&d->tl, sizeof(long long) * gatk::kTlFields * kTlCap, d, nullptr, true);
+            if (rc) return rc;
+        }
         hipLaunchKernelGGL(gatk::fill_u64, dim3(64), dim3(256), 0, s, (unsigned long long *)d->tl,
                            (long long)gatk::kTlFields * kTlCap, ~0ull);
         tl = d->tl;
@@ -3974,8 +4117,12 @@ extern "C" int gat_copy_probe(uint64_t bytes, int32_t reps, double *gbps_out) {
     if (bytes < 16 || reps < 1) GAT_FAIL(GAT_EINVAL, "copy probe needs bytes >= 16 and reps >= 1");
     const long long n = (long long)(bytes / 16);
     int4 *src = nullptr, *dst = nullptr;
-    HIPCHECK(hipMalloc(&src, n * 16));
-    HIPCHECK(hipMalloc(&dst, n * 16));
+    rc = need_malloc(&src, n * 16, nullptr);
+    if (!rc) rc = need_malloc(&dst, n * 16, nullptr);
+    if (rc) {
+        if (src) (void)hipFree(src);
+        return rc;
+    }
     hipEvent_t e0, e1;
     HIPCHECK(hipEventCreate(&e0));
     HIPCHECK(hipEventCreate(&e1));

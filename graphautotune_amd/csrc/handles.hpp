@@ -9,6 +9,9 @@
 namespace gat {
 struct PlanDevice;  // device buffers of a plan (engine.hip)
 void destroy_plan_device(PlanDevice *);
+// Frees device memory that counts can do without and that none is using
+// (engine.hip); true if there was any.
+bool give_back_memory();
 }  // namespace gat
 
 struct gat_graph {

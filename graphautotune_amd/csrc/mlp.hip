@@ -19,7 +19,7 @@
 #include <type_traits>
 #include <vector>
 
-#include "common.hpp"
+#include "handles.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -294,17 +294,30 @@ using namespace gat;
         if (e_ != hipSuccess) GAT_FAIL(GAT_ENODEV, "%s failed: %s", #x, hipGetErrorString(e_));     \
     } while (0)
 
+// Device memory, if need be what counts can do without.
+template <class T>
+static hipError_t mlp_malloc(T **p, size_t bytes) {
+    for (bool again = false;; again = true) {
+        const hipError_t e = hipMalloc((void **)p, bytes);
+        if (e == hipSuccess) return e;
+        *p = nullptr;
+        (void)hipGetLastError();  // the runtime keeps an error until it is asked for
+        if (again || e != hipErrorOutOfMemory || !give_back_memory()) return e;
+    }
+}
+
 static int ensure_batch(gat_mlp *n, int B) {
     if (B <= n->cap) return GAT_OK;
     for (float **q : {&n->x, &n->t, &n->a1, &n->a2, &n->y, &n->dy, &n->d2, &n->d1})
         if (*q) (void)hipFree(*q), *q = nullptr;
+    n->cap = 0;
     const int c = ((B + 63) / 64) * 64;
-    MCHECK(hipMalloc(&n->x, sizeof(float) * (size_t)c * n->F));
-    MCHECK(hipMalloc(&n->t, sizeof(float) * c));
+    MCHECK(mlp_malloc(&n->x, sizeof(float) * (size_t)c * n->F));
+    MCHECK(mlp_malloc(&n->t, sizeof(float) * c));
     for (float **q : {&n->a1, &n->a2, &n->d2, &n->d1})
-        MCHECK(hipMalloc(q, sizeof(float) * (size_t)c * n->H));
-    MCHECK(hipMalloc(&n->y, sizeof(float) * c));
-    MCHECK(hipMalloc(&n->dy, sizeof(float) * c));
+        MCHECK(mlp_malloc(q, sizeof(float) * (size_t)c * n->H));
+    MCHECK(mlp_malloc(&n->y, sizeof(float) * c));
+    MCHECK(mlp_malloc(&n->dy, sizeof(float) * c));
     n->cap = c;
     return GAT_OK;
 }
@@ -371,8 +384,8 @@ int gat_mlp_create(int32_t in_dim, int32_t hidden, uint64_t seed, gat_mlp **out)
     fill((long long)in_dim * hidden + hidden + (long long)hidden * hidden + hidden, hidden, hidden);
     hipError_t e = hipStreamCreateWithFlags(&n->s, hipStreamNonBlocking);
     for (float **q : {&n->p, &n->g, &n->m, &n->v})
-        if (e == hipSuccess) e = hipMalloc(q, sizeof(float) * n->P);
-    if (e == hipSuccess) e = hipMalloc(&n->loss, sizeof(float));
+        if (e == hipSuccess) e = mlp_malloc(q, sizeof(float) * n->P);
+    if (e == hipSuccess) e = mlp_malloc(&n->loss, sizeof(float));
     if (e == hipSuccess) e = hipMemcpy(n->p, h.data(), sizeof(float) * n->P, hipMemcpyHostToDevice);
     std::vector<float> z(n->P, 0.f);
     if (e == hipSuccess) e = hipMemcpy(n->m, z.data(), sizeof(float) * n->P, hipMemcpyHostToDevice);

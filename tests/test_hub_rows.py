@@ -40,12 +40,13 @@ def test_failed_build_is_repeated(fake, refused):
 g = gat.Graph.erdos_renyi(100000, 4 / 100000, 1)
 p = gat.Plan(g, [HOUSE], "reference")
 p.count({"hub_degree": -1})  # everything but the bitmaps
-fake.fake_refuse(%d, 1)
+fake.fake_refuse(%d, -1)
 try:
     p.count({"hub_degree": 14})
     first = "counted"
 except GatError:
     first = "refused"
+fake.fake_refuse(1 << 60, 0)
 calls()
 p.count({"hub_degree": 14})
 result([first, len(calls(%r))])
