@@ -2974,7 +2974,8 @@ struct PlanDevice {
     bool keep = false;
     int tables_wait = 0;  // counts until tables are asked for again
     int ovf_grid = 0;
-    hipEvent_t ev[4] = {};
+    hipEvent_t ev[5] = {};  // start, after the main launch, end, after the second launches, start of the main launch
+    bool cleared = false;   // the last count cleared tables between its start and its main launch
     // clique HBM-tier rows and pair offsets
     unsigned *grows = nullptr;
     int *goff = nullptr;
@@ -3695,24 +3696,29 @@ static int enqueue(PlanDevice *d, const Launch &L, bool account, bool events, bo
     if (account) {  // W_alg is accumulated where the values are computed
         a.keep = ao.keep = 0;
     }
+    if (events) HIPCHECK(hipEventRecord(d->ev[0], s));
+    d->cleared = false;
     if (!L.clique && a.keep && a.pool) {
         // epochs 1 .. 254 for counts in turn, with the pool cleared before the
         // first; the replays of a captured count share one, so each clears it
         const bool clear = !events || d->epoch >= 254;
         if (events) d->epoch = clear ? 1 : d->epoch + 1;
         a.epoch = ao.epoch = events ? d->epoch : 255;
+        d->cleared = clear;
         if (clear)
             hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, s, (unsigned long long *)d->pool,
                                d->pool_entries, 0ull);
     }
     for (int k = 0; k < 4 && !L.clique && a.keep; k++)
-        if (a.edge_tab[k])
+        if (a.edge_tab[k]) {
+            d->cleared = true;
             hipLaunchKernelGGL(gatk::fill_u64, dim3(2048), dim3(256), 0, s, (unsigned long long *)a.edge_tab[k],
                                (a.m + 1) / 2, ~0ull);
+        }
+    if (events && d->cleared) HIPCHECK(hipEventRecord(d->ev[4], s));
     a.tl = ao.tl = tl;
     ao.bytes = a.bytes + 1;  // second launch: its own W_alg counter
     const int waves = (int)(L.grid.x * (L.block.x / 64));
-    if (events) HIPCHECK(hipEventRecord(d->ev[0], s));
     gatk::CArgs c = L.ca;
     c.account = account ? 1 : 0;
     c.tl = tl;
@@ -3831,7 +3837,7 @@ static int finish(gat_plan *p, const Launch &L, uint64_t *counts_out, gat_count_
         if (timed) {
             float ms = 0, ms_main = 0, ms_second = 0;
             HIPCHECK(hipEventElapsedTime(&ms, d->ev[0], d->ev[2]));
-            HIPCHECK(hipEventElapsedTime(&ms_main, d->ev[0], d->ev[1]));
+            HIPCHECK(hipEventElapsedTime(&ms_main, d->ev[d->cleared ? 4 : 0], d->ev[1]));
             HIPCHECK(hipEventElapsedTime(&ms_second, d->ev[1], d->ev[3]));
             st->seconds = ms / 1000.0;
             st->main_kernel_ms = ms_main;

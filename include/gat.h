@@ -169,7 +169,9 @@ typedef struct gat_kernel_config {
 
 /* Per-call statistics filled by gat_count (any pointer may be NULL). */
 typedef struct gat_count_stats {
-    double seconds;           /* device time of the count (hipEvents)        */
+    double seconds;           /* device time of the count (hipEvents), with
+                                 the clearing of the tables it keeps leaf
+                                 counts in                                    */
     double main_kernel_ms;    /* duration of the main engine launch          */
     double second_kernel_ms;  /* array store: the split and HBM overflow
                                  launches after the main one; bitmap store:
@@ -193,7 +195,9 @@ typedef struct gat_count_stats {
                                  takes the split_overflow copies)             */
 } gat_count_stats;
 
-#define GAT_FLAG_ACCOUNT 1u   /* instrumented pass: accumulate W_alg bytes  */
+#define GAT_FLAG_ACCOUNT 1u   /* instrumented pass: accumulate W_alg bytes;
+                                 every intersection is made, none is taken
+                                 from the tables of kept leaf counts         */
 #define GAT_FLAG_TIMELINE 2u  /* record per-wave / per-workgroup start and end
                                  times of every launch (gat_plan_timeline)  */
 
