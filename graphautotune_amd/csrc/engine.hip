@@ -2929,6 +2929,7 @@ struct DeviceGraph {
     long long *off = nullptr;
     int *adj = nullptr;
     int *split = nullptr;
+    double neighbour_degree = 0;  // mean degree of a neighbour: sum of d^2 over sum of d
     std::mutex mu;  // guards what follows; held while the bitmaps are built
     std::shared_ptr<CoreRows> core;
     std::shared_ptr<HubRows> hubs;
@@ -2953,7 +2954,8 @@ struct DeviceGraph {
 struct PlanDevice {
     std::mutex busy;  // held by a count from its preparation to its end
     hipStream_t stream = nullptr;
-    GatPlanDev *plan = nullptr;
+    GatPlanDev pd;                          // the plan as it runs on its graph (choose_kept)
+    GatPlanDev *plan = nullptr;             // a copy on the device
     unsigned long long *ctl = nullptr;      // control words (kCtl*)
     unsigned long long *result = nullptr;   // the first kCtlResult of them in pinned host memory
     long long *ovf = nullptr;
@@ -3099,6 +3101,9 @@ static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
         hipLaunchKernelGGL(gatk::split_kernel, dim3(1024), dim3(256), 0, nullptr, dg->off, dg->adj, g.n, dg->split);
         HIPCHECK(hipGetLastError());
     }
+    double squares = 0;
+    for (int32_t v = 0; v < g.n; v++) squares += (double)g.deg(v) * g.deg(v);
+    dg->neighbour_degree = g.m ? squares / (double)g.m : 0;
     HIPCHECK(hipDeviceSynchronize());
     g.dev = dg;
     *out = dg;
@@ -3395,7 +3400,7 @@ constexpr long long kPoolBytes = 1ll << 29, kPoolLeast = 1ll << 23;
 constexpr int kTabVertices = 1 << 14;
 static int ensure_tables(gat_plan *p) {
     PlanDevice *d = p->dev;
-    const GatPlanDev &pd = p->cp.dev;
+    const GatPlanDev &pd = d->pd;
     const Graph &g = *p->graph;
     if (d->keep || !(pd.edge_tables || pd.n_tables)) return GAT_OK;
     if (g.m == 0 || g.max_deg >= 1 << 24 || g.m >= (1ll << 32) - 1) return GAT_OK;
@@ -3447,7 +3452,8 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         if (!rc) rc = need_malloc(&d->ctl, sizeof(unsigned long long) * kCtlWords, nullptr);
         if (!rc) rc = need_malloc(&d->dargs, sizeof(gatk::KArgsSet), nullptr);
         if (rc) return rc;
-        HIPCHECK(hipMemcpy(d->plan, &pd, sizeof(GatPlanDev), hipMemcpyHostToDevice));
+        choose_kept(p->cp.dev, d->dg->neighbour_degree, (double)g.m, &d->pd);
+        HIPCHECK(hipMemcpy(d->plan, &d->pd, sizeof(GatPlanDev), hipMemcpyHostToDevice));
         HIPCHECK(hipHostMalloc((void **)&d->result, sizeof(unsigned long long) * kCtlResult, hipHostMallocDefault));
         for (auto &e : d->ev) HIPCHECK(hipEventCreate(&e));
         p->dev = d.release();

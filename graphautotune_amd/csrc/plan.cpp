@@ -1,6 +1,7 @@
 #include "plan.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <numeric>
@@ -706,23 +707,68 @@ int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOption
     return GAT_OK;
 }
 
+// A kept value costs a look into the table, tests for the excluded vertices and
+// a store, about as much as the sweep of two lists of some 20 entries. It pays
+// where the lists are longer or the value is wanted again. Plain over kept time
+// (above 1 the tables gain), 14 patterns in unique and reference mode on 12 random,
+// Chung-Lu and R-MAT graphs:
+//   KEEP_EDGE, whole lists, by r: 9: 0.83-0.85, 14: 1.05-1.17, 25: 1.0-1.48, 34:
+//     1.3-1.55, 41 and more: 1.5-6; truncated at c: 9: 0.79-0.85, 14: 0.89-0.99,
+//     25: 0.89-1.15, 41 and more: 1.1-3.
+//   KEEP_SUM, by r: 25: 0.90, 31: 0.79-0.90, 41: 0.93-0.95, 61: 0.93-0.95, 65 and
+//     more: 0.98-1.04, and up to 3 on single edges between hubs.
+//   KEEP_POOL: an r-regular graph has r^h walks of h steps from the key to c, so
+//     lambda = r^(h + 1) / m of them end in one c. h = 2, one vertex: lambda up to
+//     0.3: 0.73-0.91, 0.5: 0.9-1.0, 1.3: 1.1-1.4; the root edge: 1.3: 0.7-0.8, 2:
+//     0.9-1.0, 19: 1.3; h = 3: up to 1.4: 0.65-0.88, 5: 0.8, 15: 1.0, 78: 2.1.
+// The pair sweep pays for itself (C5, unique: 2.0 at lambda 0.008).
+void choose_kept(const GatPlanDev &plan, double r, double m, GatPlanDev *out) {
+    *out = plan;
+    GatPlanDev &d = *out;
+    d.n_tables = d.edge_tables = d.key_edges = 0;
+    for (int i = 1; i < d.n_nodes; i++) {
+        GatNode &g = d.nodes[i];
+        if (!g.leaf) continue;
+        const bool pair = d.nodes[g.parent].pair != 0;
+        for (int k = g.op_begin; k < g.op_begin + g.op_count; k++) {
+            GatOp &o = d.ops[k];
+            if (o.kind != GATP_COUNT || o.father < 0) continue;
+            if (o.keep == GATP_KEEP_EDGE && r < (o.table ? 32 : 20)) o.keep = GATP_KEEP_NONE;
+            if (o.keep == GATP_KEEP_SUM && r < 64) o.keep = GATP_KEEP_NONE;
+            if (o.keep == GATP_KEEP_POOL && !pair) {
+                const int h = o.key == 1 ? g.depth : g.depth - 1;
+                const double lambda = std::pow(r, h + 1) / m;
+                if (lambda < (h <= 2 ? 1 : 16) * (o.key == 3 ? 4 : 1)) o.keep = GATP_KEEP_NONE;
+            }
+            if (o.keep == GATP_KEEP_NONE) g.kept = 0;
+            if (o.keep == GATP_KEEP_EDGE || o.keep == GATP_KEEP_SUM) d.edge_tables |= 1 << o.table;
+            if (o.keep == GATP_KEEP_POOL) {
+                d.n_tables = std::max(d.n_tables, o.table + 1);
+                if (o.key == 3) d.key_edges = 1;
+            }
+        }
+    }
+}
+
 std::string describe_plan(const GatPlanDev &d) {
     std::ostringstream os;
-    static const char *kinds[] = {"ALIAS", "LIST", "COUNT"};
+    static const char *kinds[] = {"ALIAS", "LIST", "COUNT"}, *keeps[] = {"", " keep edge ", " keep pool ", " keep sum "};
     os << "nodes " << d.n_nodes << " slots " << d.n_slots << " ops " << d.n_ops << " terms " << d.n_terms
        << " store " << d.n_store << " max_leaf_ops " << d.max_leaf_ops << "\n";
     for (int i = 0; i < d.n_nodes; i++) {
         const GatNode &g = d.nodes[i];
         os << "node " << i << " depth " << int(g.depth) << " parent " << g.parent << " loop " << g.loop_slot
            << " bound 0x" << std::hex << int(g.bound) << " excl 0x" << int(g.excl) << " ap 0x" << int(g.ap_levels)
-           << std::dec << (g.leaf ? " leaf" : "") << " children " << g.child_begin << "+" << g.child_count
+           << std::dec << (g.leaf ? " leaf" : "") << (g.pair ? " pair" : "") << " children " << g.child_begin << "+" << g.child_count
            << " sib " << g.next_sibling << "\n";
         for (int k = 0; k < g.op_count; k++) {
             const GatOp &o = d.ops[g.op_begin + k];
             os << "   op slot " << o.slot << " " << kinds[o.kind] << " father " << o.father << " groups[";
             for (int j = 0; j < o.ngroups; j++) os << std::hex << "0x" << int(o.groups[j]) << std::dec << " ";
             os << "] excl 0x" << std::hex << int(o.excl) << std::dec << " store " << int(o.store) << " leaf_idx "
-               << int(o.leaf_idx) << "\n";
+               << int(o.leaf_idx) << keeps[int(o.keep)];
+            if (o.keep) os << int(o.table) << " key 0x" << std::hex << int(o.key) << std::dec;
+            os << "\n";
         }
         for (int t = 0; t < g.term_count; t++) {
             const GatTerm &tm = d.terms[g.term_begin + t];

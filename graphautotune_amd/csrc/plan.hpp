@@ -52,6 +52,11 @@ struct PlanOptions {
 // mode: GAT_MODE_UNIQUE / GAT_MODE_REFERENCE / GAT_MODE_LABELED
 int compile_plan(const std::vector<std::string> &adj, int mode, const PlanOptions &opt, CompiledPlan *out);
 
+// The plan as it runs on a graph with m directed edges and a mean neighbour
+// degree r (sum of d^2 over sum of d): COUNTs whose kept value would hardly be
+// asked for again there are not kept.
+void choose_kept(const GatPlanDev &plan, double r, double m, GatPlanDev *out);
+
 std::string describe_plan(const GatPlanDev &d);
 
 }  // namespace gat

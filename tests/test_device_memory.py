@@ -124,10 +124,10 @@ result([small, none, any(quiet), count(p)])
 def test_edge_tables_are_not_held_for_nothing(fake):
     """The pool is refused: what the edge tables took is free again."""
     got = fakehip.run(fake, """
-g = gat.Graph.erdos_renyi(20000, 6 / 20000, 1)
+g = gat.Graph.erdos_renyi(3000, 60 / 3000, 1)
 gat.Plan(g, [TRIANGLE], "unique").count({"vertex_store": 1, "split_us": -1})  # the graph is on the device
 p = gat.Plan(g, [HOUSE], "unique")
-fake.fake_refuse(8 << 20, -1)
+fake.fake_refuse(8000000, -1)  # pools have 8.4 MB and more, set buffers 4.7
 calls()
 p.count({"split_us": -1})
 l = calls()
