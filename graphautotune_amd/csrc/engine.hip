@@ -1923,27 +1923,16 @@ struct CArgs {
     int cap;                     // slot_capacity as the clique store takes it
     int main_max;                // largest d of the main launch: min(CMAIN, cap)
     int chunk;                   // vertices per main-queue grab
-    int lin_thr;
     long long *tl;               // timeline records (GAT_FLAG_TIMELINE), or null
     int tl_base;                 // first record of this launch
 };
 
-// hit[u] |= y[u] in N+(x[u]) for the lanes with act[u]: U searches of lists
+// hit[u] |= y[u] in the n[u] entries from a.adj[base[u]] on: U searches of lists
 // side by side, so that a round of them waits for one memory latency.
 template <int U>
-__device__ __forceinline__ void search_below(const CArgs &a, const int (&x)[U], const int (&y)[U], const bool (&act)[U],
+__device__ __forceinline__ void search_below(const CArgs &a, long long (&base)[U], int (&n)[U], const int (&y)[U],
                                              bool (&hit)[U]) {
-    long long base[U];
-    int n[U], longest = 0;
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        base[u] = 0;
-        n[u] = 0;
-        if (act[u]) {
-            base[u] = a.off[x[u]];
-            n[u] = a.split[x[u]];
-        }
-    }
+    int longest = 0;
 #pragma unroll
     for (int u = 0; u < U; u++) longest = max(longest, n[u]);
     // halve every list until one entry is left (the last entry <= y, if any)
@@ -2013,21 +2002,30 @@ __device__ __forceinline__ unsigned long long vtx_rows(const CArgs &a, LP L, int
                         if (j <= last) put(p0 + j * stride, b + u, ballot(v[u][j] & 1u));
             }
         } else {
-            for (int j = 0; j <= last; j++) {
-                const int p = p0 + j * stride, xj = uni(L[p]);
-                const int *xa = a.adj + a.off[xj];
-                const int xl = a.split[xj];
-                const bool core = xj < a.core_n;
-                const unsigned *cr = a.core + core_row(core ? xj : 0);
-                for (int b = 0; b < nb; b++) {
-                    const int q = b * W + ln;
-                    bool hit = false;
-                    if (q < p) {
-                        const int y = L[q];
-                        hit = core ? (cr[y >> 5] >> (y & 31)) & 1u : has(xa, xl, y, a.lin_thr);
-                    }
-                    put(p, b, ballot(hit));
+            long long xb[R];
+            int xn[R];
+#pragma unroll
+            for (int j = 0; j < R; j++) {
+                xb[j] = a.off[x[j]];
+                xn[j] = a.split[x[j]];
+            }
+            for (int b = 0; b < nb; b++) {
+                const int q = b * W + ln;
+                int y[R], n[R];
+                long long base[R];
+                bool hit[R];
+#pragma unroll
+                for (int j = 0; j < R; j++) {
+                    const bool in = j <= last && q < p0 + j * stride, core = x[j] < a.core_n;
+                    y[j] = in ? L[q] : 0;
+                    hit[j] = in && core && (a.core[core_row(x[j]) + (y[j] >> 5)] >> (y[j] & 31) & 1u);
+                    base[j] = xb[j];
+                    n[j] = in && !core ? xn[j] : 0;
                 }
+                search_below<R>(a, base, n, y, hit);
+#pragma unroll
+                for (int j = 0; j < R; j++)
+                    if (j <= last) put(p0 + j * stride, b, ballot(hit[j]));
             }
         }
         const int done = x[R - 1] < a.core_n ? 2 * ((nb + 1) / 2 * 2) : 2 * nb;  // words written
@@ -2462,13 +2460,20 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
                         word[u] = 0;
                         if (in[u] && x[u] < a.core_n) word[u] = a.core[core_row(x[u]) + (y[u] >> 5)] >> (y[u] & 31);
                     }
-                    bool hit[U], far[U];
+                    bool hit[U];
+                    long long base[U];
+                    int n[U];
 #pragma unroll
                     for (int u = 0; u < U; u++) {
                         hit[u] = word[u] & 1u;
-                        far[u] = in[u] && x[u] >= a.core_n;
+                        base[u] = 0;
+                        n[u] = 0;
+                        if (in[u] && x[u] >= a.core_n) {
+                            base[u] = a.off[x[u]];
+                            n[u] = a.split[x[u]];
+                        }
                     }
-                    search_below<U>(a, x, y, far, hit);
+                    search_below<U>(a, base, n, y, hit);
 #pragma unroll
                     for (int u = 0; u < U; u++) {
                         const unsigned long long m = ballot(hit[u]);
@@ -2526,6 +2531,10 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
                 C.L[ln] = y;
                 // core vertices come first in the sorted list
                 const int pc = __popcll(ballot(ln < d && y < a.core_n));
+                // the others' lists, for the searches below
+                const bool far = pc < d && ln < d && y >= a.core_n;
+                const long long far_base = far ? a.off[y] : 0;
+                const int far_n = far ? a.split[y] : 0;
                 unsigned long long row_l = 0;  // row ln
                 constexpr int U = 8;           // row reads in flight
                 for (int p = 1; p < pc; p += U) {
@@ -2550,19 +2559,21 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
                 const int p0 = max(pc, 1), k0 = p0 * (p0 - 1) / 2, k1 = d * (d - 1) / 2;
                 constexpr int F = 4;  // searches in flight
                 for (int kb = k0; kb < k1; kb += F * W) {
-                    int p[F], q[F], x[F], z[F];
-                    bool in[F], hit[F];
+                    int p[F], q[F], n[F], z[F];
+                    long long base[F];
+                    bool hit[F];
 #pragma unroll
                     for (int u = 0; u < F; u++) {
                         const int k = kb + u * W + ln;
-                        in[u] = k < k1;
                         hit[u] = false;
                         p[u] = q[u] = 0;
-                        if (in[u]) tri_pair(k, &p[u], &q[u]);
-                        x[u] = C.L[p[u]];
+                        if (k < k1) tri_pair(k, &p[u], &q[u]);
+                        base[u] = bperm64(far_base, p[u]);
+                        const int len = bperm(far_n, p[u]);  // by every lane
+                        n[u] = k < k1 ? len : 0;
                         z[u] = C.L[q[u]];
                     }
-                    search_below<F>(a, x, z, in, hit);
+                    search_below<F>(a, base, n, z, hit);
 #pragma unroll
                     for (int u = 0; u < F; u++) {
                         const unsigned long long m = ballot(hit[u]);
@@ -2611,12 +2622,20 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
     }
 }
 
-// Next item of a tier's queue: the vertex, or -1 when the queue is drained.
-__device__ __forceinline__ int tier_item(const CArgs &a, int tier, int *part, int *parts) {
+// Next item of a tier's queue: the vertex, or -1 when the queue is drained. A
+// workgroup takes several at a time where there are many (an atomic on one
+// address takes 17 ns, 1.7 ms for 100,000 vertices). next, last: its items.
+__device__ __forceinline__ int tier_item(const CArgs &a, int tier, unsigned long long *next, unsigned long long *last,
+                                         int *part, int *parts) {
     const unsigned long long made = a.ovf_n[tier], cap = (unsigned long long)a.tier_cap[tier];
     const unsigned long long vertices = made < cap ? made : cap;
     const int np = clique_parts(a.kmax, vertices, (int)gridDim.x);
-    const unsigned long long r = atomicAdd(&a.queue[1 + tier], 1ull);
+    if (*next == *last) {
+        const unsigned long long share = vertices * np / (16ull * gridDim.x), grab = share < 1 ? 1 : share < 16 ? share : 16;
+        *next = atomicAdd(&a.queue[1 + tier], grab);
+        *last = *next + grab;
+    }
+    const unsigned long long r = (*next)++;
     *part = (int)(r % np);
     *parts = np;
     return r / np < vertices ? a.tier[tier][r / np] : -1;
@@ -2636,13 +2655,19 @@ __global__ void __launch_bounds__(64 * NW, clique_occupancy(TIER)) clique_block_
     int *L = reinterpret_cast<int *>(rows + tier_row_words(MW));
     unsigned *buf = reinterpret_cast<unsigned *>(L) + wid * 2 * CCOLS;
     __shared__ int vsh, psh, nsh;
+    unsigned long long next = 0, last = 0;  // thread 0: items taken from the queue
     unsigned long long acc[7] = {0, 0, 0, 0, 0, 0, 0}, bytes = 0;
     constexpr bool ACC = MODE & 1, tl = (MODE & 2) != 0;
     const long long tl_t0 = tl ? wall_clock64() : 0;
     long long tl_build = 0, tl_count = 0, tl_items = 0, tl_pairs = 0, c0 = 0, c1 = 0;
     for (;;) {
         if (tl) c0 = clock64();
-        if (threadIdx.x == 0) vsh = tier_item(a, TIER, &psh, &nsh);
+        if (threadIdx.x == 0) {
+            int part, parts;
+            vsh = tier_item(a, TIER, &next, &last, &part, &parts);
+            psh = part;
+            nsh = parts;
+        }
         __syncthreads();
         const int v0 = vsh, part = psh, parts = nsh;
         if (v0 < 0) break;
@@ -2654,6 +2679,7 @@ __global__ void __launch_bounds__(64 * NW, clique_occupancy(TIER)) clique_block_
         if (fits)
             for (int k = threadIdx.x; k < d; k += 64 * NW) L[k] = a.adj[rb + k];
         __syncthreads();
+        bool any = false;
         if (fits) {
             unsigned long long bb = 0;  // every part builds the rows; W_alg and #K3 charge one build
             const unsigned long long pr = vtx_rows<ACC>(a, (const int *)L, d, rows, w, wid, NW, ln, bb);
@@ -2662,10 +2688,11 @@ __global__ void __launch_bounds__(64 * NW, clique_occupancy(TIER)) clique_block_
                 if (ACC) bytes += bb + (threadIdx.x == 0 ? 4ull * d + 16ull : 0ull);
                 tl_pairs += (long long)pr;
             }
+            any = pr != 0;
         }
-        __syncthreads();  // the rows are complete, and L is free for the column lists
+        any = __syncthreads_or(any);  // the rows are complete, and L is free for the column lists
         if (tl) c1 = clock64();
-        if (fits && a.kmax >= 4) {
+        if (any && a.kmax >= 4) {
             const int first = part * NW + wid, stride = NW * parts;
             unsigned long long none = 0;
             if (a.kmax == 4)
@@ -2696,6 +2723,7 @@ __global__ void __launch_bounds__(64 * CNW3) clique_hbm_kernel(CArgs a) {
     constexpr int TIER = 3, NW = CNW3;
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
     __shared__ int vsh, psh, nsh;
+    unsigned long long next = 0, last = 0;  // thread 0: items taken from the queue
     __shared__ int wtot[NW];
     unsigned *rows = a.grows + (long long)blockIdx.x * a.hcap * row_words(a.hcap);
     int *off = a.goff + (long long)blockIdx.x * (a.hcap + 1);
@@ -2705,7 +2733,12 @@ __global__ void __launch_bounds__(64 * CNW3) clique_hbm_kernel(CArgs a) {
     long long tl_build = 0, tl_count = 0, tl_items = 0, tl_pairs = 0, c0 = 0, c1 = 0;
     for (;;) {
         if (tl) c0 = clock64();
-        if (threadIdx.x == 0) vsh = tier_item(a, TIER, &psh, &nsh);
+        if (threadIdx.x == 0) {
+            int part, parts;
+            vsh = tier_item(a, TIER, &next, &last, &part, &parts);
+            psh = part;
+            nsh = parts;
+        }
         __syncthreads();
         const int v0 = vsh, part = psh, parts = nsh;
         if (v0 < 0) break;
@@ -3317,13 +3350,19 @@ struct Launch {
     bool heavy = false;   // clique: some vertex may have more than main_max neighbours below it
 };
 
-// Vertices per chunk of the clique main launch: as configured, but no more
-// than one and no fewer than a quarter of a wave's share. (Chunks mix heavy
-// and light vertices, so that few of them balance; a chunk per grab costs an
-// atomic, and a wave without a chunk is idle.)
+// Vertices per chunk of the clique main launch: a wave's whole share, or half to
+// a quarter of it, and no fewer than configured, where shares are long for the
+// number of waves. Chunks mix heavy and light vertices, so that whole shares
+// balance well; every further chunk is a grab, an atomic on one address (17 ns
+// each, one after another), and should cost a few per cent of the vertices it
+// hands out. us with chunks of a quarter share / of this rule: K3 on Chung-Lu
+// 130,000 of degree 12 364 / 102, K4 on random graphs of degree 40 (50,000
+// vertices) 357 / 271, 24 (200,000) 649 / 437 and 8 (1 M) 460 / 207, K3-K5 on
+// Chung-Lu 262,144 of degree 24 845 / 772.
 static int clique_chunk(int configured, long long vertices, long long waves) {
     const long long share = std::max(1ll, (vertices + waves - 1) / waves);
-    return (int)std::min(share, std::max<long long>(configured, (share + 3) / 4));
+    const long long chunks = std::max(1ll, std::min({4ll, share / std::max(1, configured), 1 + 6 * share / waves}));
+    return (int)((share + chunks - 1) / chunks);
 }
 
 // Restrict a prepared count to the root vertices [lo, hi): the array store
@@ -3365,7 +3404,6 @@ static int clique_shape(const DeviceInfo &di, const gat_kernel_config &cfg, int 
     gatk::CArgs &c = L->ca;
     c.cap = std::max(32, std::min(gatk::CMAXD, cfg.slot_capacity / 32 * 32));
     L->chunk = cfg.queue_chunk;
-    c.lin_thr = cfg.search_linear_threshold;
     L->block = dim3(64 * cfg.block_waves);
     L->grid = dim3(std::max(1, std::max(1, cfg.waves_per_cu * di.cus) / cfg.block_waves));
     L->clique_lds = sizeof(gatk::CWave) * cfg.block_waves;
@@ -3963,7 +4001,7 @@ extern "C" int gat_count_shard_edges(gat_plan *p, const gat_kernel_config *cfg, 
 // from word 64 on), then
 // kNaBody int32 entries laid out for the graph's size: the split[] array (n),
 // the lists of workgroup tiers 0 (n), 1 (kNaTierCap) and 2 (kNaTierCap / 2),
-// and the core bitmap in the rest (28 to 58 MiB, so 21,000 to 31,000 core
+// and the core bitmap within the rest (28 to 58 MiB, so up to 31,000 core
 // vertices). 64 MiB and 17 KiB in all.
 constexpr int kNaMaxV = 1 << 22;
 constexpr long long kNaTierCap = 1 << 20;
@@ -4033,7 +4071,9 @@ extern "C" int gat_count_cliques_noalloc(const int64_t *d_offsets, const int32_t
     unsigned *core = reinterpret_cast<unsigned *>(c.tier[2] + c.tier_cap[2]);
     const long long used = reinterpret_cast<int *>(core) - split;
     c.core = core;
-    c.core_n = core_vertices(v_cnt, kNaBody - used);
+    // built in every call: as large as for a graph of degree 32 (58 MB of rows
+    // for 50,000 vertices of degree 40 took 80 of 430 us)
+    c.core_n = core_vertices(v_cnt, std::min(kNaBody - used, std::max<long long>(1 << 21, 128ll * v_cnt)));
     c.n = v_cnt;
     c.m = 0;
     c.root_lo = 0;

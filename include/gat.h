@@ -120,7 +120,9 @@ typedef struct gat_kernel_config {
     int32_t block_waves;      /* waves per workgroup (threads_per_block/64)   */
     int32_t waves_per_cu;     /* persistent grid = waves_per_cu * CUs (0: 16
                                  for the array store, 8 for the clique store) */
-    int32_t queue_chunk;      /* directed edges taken per work-queue grab      */
+    int32_t queue_chunk;      /* directed edges taken per work-queue grab;
+                                 clique store: least vertices per grab where a
+                                 wave's share is long enough for several      */
     int32_t slot_capacity;    /* int32 entries per LDS prefix-set slot; clique
                                  store: vertices with more neighbours below
                                  them (at most 256 counts) always leave the
