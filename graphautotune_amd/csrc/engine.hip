@@ -1850,6 +1850,7 @@ __global__ void __launch_bounds__(256) engine_plain_sub_kernel(const KArgs *__re
 // waves of a workgroup with rows in LDS (d <= 256, 512, 1024) or in HBM.
 constexpr int CMAXD = 256;  // largest slot_capacity the clique store honours
 constexpr int CMAIN = 64;   // main launch: d <= min(CMAIN, slot_capacity)
+constexpr int CDEFER = 32;  // #K6: it hands on denser vertices with d > CDEFER
 constexpr int CT0W = 8;     // workgroup tier 0: rows of 8 words, d <= 256
 constexpr int CT1W = 16;    // workgroup tier 1: d <= 512
 constexpr int CT2W = 32;    // workgroup tier 2: d <= 1024
@@ -2306,6 +2307,7 @@ constexpr int CTINY = 11;
 // words) and the pair list.
 struct alignas(16) CWave {
     int L[CMAIN];
+    int deferred[W];
     unsigned long long rows[CMAIN];
     unsigned short pairs[W * (CTINY * (CTINY - 1) / 2)];
 };
@@ -2393,6 +2395,11 @@ static_assert(CTIERS == 4, "ovf_n[4] and [5] count vertices with d > cap");
 // own number and takes further ones from the queue: a grab is an atomic on
 // one address, 17 ns each however many waves there are (chunks of 4 vertices
 // from a counter alone held R-MAT s20's launch at 4.6 ms).
+// #K6: the walk of one wave grows with the cube of d where the rows are dense
+// (R-MAT s14: 1.75 ms with vertices up to 64 here, 0.60 up to 32), so a vertex
+// with d > CDEFER and a quarter of the pairs adjacent goes to tier 0, its rows
+// built in vain. By size alone sparse ones went too (a random graph of 200,000
+// vertices and degree 60: 2.26 ms, now 1.46).
 // Of a block of up to 64 vertices of a chunk, the tiny ones (d <= CTINY) are
 // taken together, one position pair per lane, and keep all their rows in one
 // word (row p at bit p (p - 1) / 2); the others follow one by one, with the
@@ -2400,8 +2407,10 @@ static_assert(CTIERS == 4, "ovf_n[4] and [5] count vertices with d > cap");
 // MODE bit 0: accumulate W_alg; bit 1: timeline records (separate
 // instantiations, so that a timed count carries none of their work or
 // registers).
+// 128 registers (16 waves per CU where the config asks for as many; with 134, K4 on
+// a random graph of 50,000 vertices and degree 40 took 262 us instead of 178).
 template <int MODE>
-__global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
+__global__ void __launch_bounds__(256, 4) clique_kernel(CArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int wid = threadIdx.x / W, ln = threadIdx.x % W;
     CWave &C = reinterpret_cast<CWave *>(smem)[wid];
@@ -2506,26 +2515,24 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
                 }
             }
             unsigned long long todo = ballot(d_l > CTINY && d_l <= lim);
-            int d = 0, y = 0;
+            int d = 0, y = 0, vertex = 0, n_deferred = 0;
             if (todo) {
                 const int l = __ffsll((long long)todo) - 1;
                 d = LanePull{l}(d_l);
+                vertex = LanePull{l}((int)v);
                 const long long rb = LanePull{l}(b_l);
                 if (ln < d) y = a.adj[rb + ln];
             }
             while (todo) {
                 const long long c0 = tl ? clock64() : 0;
                 todo &= todo - 1;
-                int dn = 0, yn = 0;  // the next vertex's list
+                int dn = 0, yn = 0, vn = 0;  // the next vertex's list
                 if (todo) {
                     const int l = __ffsll((long long)todo) - 1;
                     dn = LanePull{l}(d_l);
+                    vn = LanePull{l}((int)v);
                     const long long rb = LanePull{l}(b_l);
                     if (ln < dn) yn = a.adj[rb + ln];
-                }
-                if (ACC) {
-                    if (ln == 0) bytes += 4ull * d + 16ull;
-                    if (ln < d) bytes += 4ull * (a.split[y] + ln) + 16ull + 4ull * ((ln >> 5) + 1);
                 }
                 int run = 0;
                 C.L[ln] = y;
@@ -2555,10 +2562,12 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
                 }
                 C.rows[ln] = row_l;
                 wsync();
-                // the other vertices' rows: one pair (p, q) per lane
+                // the other vertices' rows: one pair (p, q) per lane, eight searches of
+                // a lane in flight where that many are left (of four at a time, K3 on a
+                // random graph of 200,000 vertices and degree 60 took 1.54 ms, now 1.43)
                 const int p0 = max(pc, 1), k0 = p0 * (p0 - 1) / 2, k1 = d * (d - 1) / 2;
-                constexpr int F = 4;  // searches in flight
-                for (int kb = k0; kb < k1; kb += F * W) {
+                auto search = [&](auto flight, int kb) {  // so many searches side by side
+                    constexpr int F = decltype(flight)::value;
                     int p[F], q[F], n[F], z[F];
                     long long base[F];
                     bool hit[F];
@@ -2583,11 +2592,24 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
                         }
                         run += __popcll(m);
                     }
-                }
-                if (ln == 0) acc[3] += (unsigned long long)run;
+                };
+                int kb = k0;
+                for (; kb + 4 * W < k1; kb += 8 * W) search(std::integral_constant<int, 8>{}, kb);
+                if (kb < k1) search(std::integral_constant<int, 4>{}, kb);
                 wsync();
                 const long long c1 = tl ? clock64() : 0;
-                if (a.kmax >= 4) {
+                const bool defer = a.kmax >= 6 && d > CDEFER && 8 * run > d * (d - 1);
+                if (defer) {
+                    if (ln == 0) C.deferred[n_deferred] = vertex;
+                    n_deferred++;
+                } else {
+                    if (ln == 0) acc[3] += (unsigned long long)run;
+                    if (ACC) {
+                        if (ln == 0) bytes += 4ull * d + 16ull;
+                        if (ln < d) bytes += 4ull * (a.split[y] + ln) + 16ull + 4ull * ((ln >> 5) + 1);
+                    }
+                }
+                if (a.kmax >= 4 && !defer) {
                     auto row = [&](int p) { return C.rows[p]; };
                     for (int k = ln; k < run; k += W) {
                         const int pq = C.pairs[k];
@@ -2603,6 +2625,18 @@ __global__ void __launch_bounds__(256) clique_kernel(CArgs a) {
                 }
                 d = dn;
                 y = yn;
+                vertex = vn;
+            }
+            if (n_deferred) {
+                wsync();
+                unsigned long long r = 0;
+                if (ln == 0) r = atomicAdd(&a.ovf_n[0], (unsigned long long)n_deferred);
+                const long long at = uni64((long long)__shfl(r, 0)) + ln;
+                if (ln < n_deferred) {
+                    if (at < a.tier_cap[0]) a.tier[0][at] = C.deferred[ln];
+                    else atomicOr(a.err, 4u);
+                }
+                wsync();
             }
         }
         // the queue counts the chunks after the waves' own; it is read before
@@ -3413,11 +3447,10 @@ static int clique_shape(const DeviceInfo &di, const gat_kernel_config &cfg, int 
     // 64 B: the kernels' own static LDS
     c.lds_dmax = lds[2] + 64 <= di.lds_per_block ? 32 * gatk::CT2W : 32 * gatk::CT1W;
     const int waves[3] = {gatk::CNW0, gatk::CNW1, gatk::CNW2};
-    // #K6 leaves the main launch earlier: its walk on one wave grows with d^3
-    // (R-MAT s14: 1.75 ms with vertices up to 64 there, 0.60 ms up to 32; s16
-    // the same either way; #K3 to #K5 lose up to 10 % below 64)
-    c.main_max = std::min(c.kmax >= 6 ? gatk::CMAIN / 2 : gatk::CMAIN, c.cap);
-    const int above[4] = {c.main_max, 32 * gatk::CT0W, 32 * gatk::CT1W, c.lds_dmax};
+    // (#K3 to #K5 lose up to 10 % below 64)
+    c.main_max = std::min(gatk::CMAIN, c.cap);
+    const int above[4] = {c.kmax >= 6 ? std::min(gatk::CDEFER, c.main_max) : c.main_max, 32 * gatk::CT0W, 32 * gatk::CT1W,
+                          c.lds_dmax};
     for (int t = 0; t < 3; t++) {
         L->tier_lds[t] = lds[t];
         const int per_cu = std::max(1, std::min((int)(di.lds_per_cu / (lds[t] + 64)), 4 * gatk::clique_occupancy(t) / waves[t]));
