@@ -109,8 +109,8 @@ struct KArgs {
     // tab_size on; key x uses table x % pool_tables, whose entry c holds the tag
     // x + 1, the value and the epoch for the key that wrote it last. Every count has its
     // own epoch, so nothing of an earlier one is taken. One pool for all waves:
-    // with a table per wave the subtasks of one root each filled their own
-    // (C5 108 ms, now 56; house on Chung-Lu 65,536 46 ms, now 36).
+    // with a table per wave the subtasks of one root each filled their own (before
+    // the pair sweep C5 108 ms instead of 56, house on Chung-Lu 65,536 46 instead of 36).
     KeptEdge *edge_tab[4];
     KeptEntry *pool;
     unsigned pool_tables;
@@ -297,7 +297,8 @@ __device__ __forceinline__ bool has(P a, int len, int x, int lin_thr) {
 // 20 ns each on this chip, so one head would feed a launch at most 50 tasks per
 // microsecond and hold back every wave that asks meanwhile (C4 + P4 on a random
 // graph of 1.6M directed edges: 8.8 ms with 16 edges per task and 19 ms with 4;
-// 3.8 and 4.3 ms with 64 heads; a launch without work: 50 and 6 us). A queue has kHeads heads on cache lines of their own; head q hands out the items
+// 3.8 and 4.3 ms with 64 heads; a launch without work: 50 and 6 us). A queue has
+// kHeads heads on cache lines of their own; head q hands out the items
 // (r / kRun kHeads + q) kRun + r % kRun, r = 0, 1, ..: runs of kRun neighbouring
 // items, which share a root and the tables kept for it, go to the waves of one
 // head, and waves 8 apart sit on one XCD. A wave whose head is empty moves on to
@@ -737,9 +738,9 @@ __device__ __forceinline__ bool want_split(const KArgs &a, const WaveState *S) {
 // A loop whose first `done` candidates took `ticks`: will the other `left` take
 // more than 1 / kTailShare of the split budget? In the tail such a rest does not
 // wait for the budget: idle waves are there to take it, and one subtask costs 10
-// to 20 us. (Counts of a few roots are tails from their start: C5 of one light
-// root of Chung-Lu 1M, 1.7 to 5.3 ms in the mean of eight, 4.8 when every level
-// of subtasks waited for the budget.)
+// to 20 us. (Counts of a few roots are tails from their start: C5 of one root of
+// Chung-Lu 1M took 4.7 ms in the mean of eight while every level of subtasks
+// waited for the budget, and takes 1.3.)
 constexpr int kTailShare = 8;
 __device__ __forceinline__ bool rest_is_long(const KArgs &a, long long ticks, int done, int left) {
     return done > 0 && ticks * left * kTailShare > a.split_ticks * done;
@@ -811,7 +812,9 @@ __device__ __noinline__ bool split_shallowest(const Ctx C, int d) {
     for (int k = uni(S->base_depth); k <= d; k++) {
         const int cur = uni(S->f_cur[k]), fh = uni(S->f_hi[k]);
         if (fh - cur < 2) continue;
-        if (!donate(C, k, uni(S->f_node[k]), cur, fh, C.P.nodes[uni(S->f_node[k])].leaf ? W : C.P.nodes[uni(S->f_node[k])].pair ? kPairChunk : 1, !GS)) return false;
+        const int node = uni(S->f_node[k]);
+        const int least = C.P.nodes[node].leaf ? W : C.P.nodes[node].pair ? kPairChunk : 1;
+        if (!donate(C, k, node, cur, fh, least, !GS)) return false;
         if (C.ln == 0) S->f_hi[k] = cur;
         wsync();
         return true;
@@ -1870,10 +1873,12 @@ __device__ __forceinline__ int clique_parts(int kmax, unsigned long long vertice
     return (int)(p < mx ? p : mx);
 }
 // Waves per workgroup: enough to share one vertex's work, few enough that
-// the workgroups of a CU (bounded by LDS, 11, 39 and 160 KB each, and by registers) overlap
-// one's row build with another's counting.
+// the workgroups of a CU (bounded by LDS, 11, 37 and 139 KB each, and by
+// registers) overlap one's row build with another's counting.
 constexpr int CNW0 = 4, CNW1 = 4, CNW2 = 8, CNW3 = 16;
-// Waves per SIMD the tiers' registers leave room for.
+// Waves per SIMD that the tiers' registers are held to. Tiers 0 and 1 spill for it
+// (93 and 11 registers): without spills, with three and two waves, K4 + K5 on
+// R-MAT s20 takes 14.3 ms instead of 12.1 (K4 on R-MAT s14 149 us instead of 167).
 constexpr int clique_occupancy(int tier) { return tier == 0 ? 4 : tier == 1 ? 3 : 2; }
 // Words per bit row of a list of d vertices: enough for d bits, rounded up
 // to an odd number so that lanes reading the same word of different rows
@@ -2074,7 +2079,8 @@ __device__ __forceinline__ v4i operand_rows(unsigned x) {  // bits 0..3 of each 
 __device__ __forceinline__ v4i operand_cols(unsigned x) {  // ... as 0.5, 1.0, 2.0, 2.0
     return v4i{(int)(x & 0x11111111u), (int)(x & 0x22222222u), (int)(x & 0x44444444u), (int)((x >> 1) & 0x44444444u)};
 }
-__device__ __forceinline__ v4f mfma_bits(v4i rows, v4i cols, v4f c) {  // 4-bit operands take four registers; scale arguments 0 select the unscaled form
+// 4-bit operands take four registers; scale arguments 0 select the unscaled form.
+__device__ __forceinline__ v4f mfma_bits(v4i rows, v4i cols, v4f c) {
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
         __builtin_shufflevector(rows, rows, 0, 1, 2, 3, -1, -1, -1, -1),
         __builtin_shufflevector(cols, cols, 0, 1, 2, 3, -1, -1, -1, -1), c, kFp4, kFp4, 0, 0, 0, 0);
@@ -3087,7 +3093,8 @@ void destroy_plan_device(PlanDevice *d) {
     if (d->graph) (void)hipGraphDestroy(d->graph);
     for (auto &e : d->ev)
         if (e) (void)hipEventDestroy(e);
-    for (void *p : {(void *)d->plan, (void *)d->dargs, (void *)d->tl, (void *)d->ctl, (void *)d->ovf, (void *)d->subs, (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2], (void *)d->tier[3],
+    for (void *p : {(void *)d->plan, (void *)d->dargs, (void *)d->tl, (void *)d->ctl, (void *)d->ovf, (void *)d->subs,
+                    (void *)d->tier[0], (void *)d->tier[1], (void *)d->tier[2], (void *)d->tier[3],
                     (void *)d->gstore, (void *)d->grows, (void *)d->goff})
         if (p) (void)hipFree(p);
     if (d->result) (void)hipHostFree(d->result);
@@ -3196,10 +3203,10 @@ static int32_t max_out_degree(Graph &g) {
 // degree >= kHubDegree and, within kHubMoreBytes, of further ones down to
 // hub_default(n). One word of a bitmap replaces a search of about log2(degree)
 // dependent reads, but in many sparse rows every word is a cache line of its
-// own. ms with a threshold of 256 / 64 / 16: house on Chung-Lu 65,536 22.0 /
-// 19.1 / 19.1, C5 on R-MAT s13 24.3 / 22.0 / 21.8, 21 patterns on R-MAT s10
-// 11.1 / 8.8 / 7.3, C4 + P4 on a random graph of 100,000 vertices and mean
-// degree 16 3.8 / 3.8 / 5.6. Built outside the timed count, like the graph
+// own. ms with a threshold of 256 / 64 / 16: house on Chung-Lu 65,536 18.6 /
+// 16.7 / 16.8, C5 on R-MAT s13 18.1 / 15.2 / 15.0, 21 patterns on R-MAT s10
+// 10.3 / 8.3 / 6.9, C4 + P4 on a random graph of 100,000 vertices and mean
+// degree 16 3.9 / 3.9 / 5.7. Built outside the timed count, like the graph
 // upload itself, when a graph's first count needs them or a later one needs more.
 constexpr double kHubBytes = 8.0 * (1ull << 30), kHubMoreBytes = 1.0 * (1ull << 30);
 constexpr int kHubDegree = 256;
@@ -3265,7 +3272,8 @@ static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr, PlanDevice *min
     const int least = thr ? thr : hub_default(g.n);
     const double row_bytes = 4.0 * (double)std::max(1ll, ((long long)g.n + 31) / 32);
     const size_t found = vertices(least), most = (size_t)(kHubBytes / row_bytes);
-    const size_t always = std::min(thr ? found : vertices(std::max(least, kHubDegree)), most);  // rows that only kHubBytes limits
+    // rows that only kHubBytes limits
+    const size_t always = std::min(thr ? found : vertices(std::max(least, kHubDegree)), most);
     size_t n = std::min({found, std::max(always, (size_t)(kHubMoreBytes / row_bytes)), most});
     auto missing = [&] { return n > (dg->hubs ? dg->hubs->n : 0); };
     if (missing() && n > always) {  // the rows beyond kHubDegree only where there is room
@@ -4148,7 +4156,8 @@ extern "C" int gat_count_cliques_noalloc(const int64_t *d_offsets, const int32_t
     if (err & 16u)
         GAT_FAIL(GAT_ELIMIT, "a vertex has more than %d neighbours below it; the allocation-free count has no HBM tier",
                  c.lds_dmax);
-    if ((err & 4u) || heavy > (unsigned long long)kNaTierCap) GAT_FAIL(GAT_ELIMIT, "more than %lld heavy vertices for one workgroup tier", kNaTierCap);
+    if ((err & 4u) || heavy > (unsigned long long)kNaTierCap)
+        GAT_FAIL(GAT_ELIMIT, "more than %lld heavy vertices for one workgroup tier", kNaTierCap);
     if (err) GAT_FAIL(GAT_EINTERNAL, "engine reported an internal inconsistency (flags 0x%x)", err);
     for (int i = 0; i < gatk::kCountCopies; i++)
         for (int k = 0; k < 8; k++) raw[k] += copies[i * GATP_MAX_TERMS + k];
