@@ -3002,12 +3002,12 @@ struct DeviceGraph {
     long long *off = nullptr;
     int *adj = nullptr;
     int *split = nullptr;
-    double neighbour_degree = 0;  // mean degree of a neighbour: sum of d^2 over sum of d
     std::mutex mu;  // guards what follows; held while the bitmaps are built
     std::shared_ptr<CoreRows> core;
     std::shared_ptr<HubRows> hubs;
-    std::vector<int> at_least;  // at_least[d]: vertices of degree >= d, d <= max_deg + 1
+    std::vector<int> at_least;  // degree_stats: at_least[d]: vertices of degree >= d, d <= max_deg + 1
     bool ordered = false;       // ids by descending degree
+    double neighbour_degree = 0;  // mean degree of a neighbour: sum of d^2 over sum of d
     int hubs_wait = 0;          // counts until the optional rows are asked for again
     DeviceGraph() {
         std::lock_guard<std::mutex> lk(holders().mu);
@@ -3175,9 +3175,6 @@ static int ensure_device_graph(Graph &g, std::shared_ptr<DeviceGraph> *out) {
         hipLaunchKernelGGL(gatk::split_kernel, dim3(1024), dim3(256), 0, nullptr, dg->off, dg->adj, g.n, dg->split);
         HIPCHECK(hipGetLastError());
     }
-    double squares = 0;
-    for (int32_t v = 0; v < g.n; v++) squares += (double)g.deg(v) * g.deg(v);
-    dg->neighbour_degree = g.m ? squares / (double)g.m : 0;
     HIPCHECK(hipDeviceSynchronize());
     g.dev = dg;
     *out = dg;
@@ -3211,6 +3208,23 @@ static int32_t max_out_degree(Graph &g) {
 constexpr double kHubBytes = 8.0 * (1ull << 30), kHubMoreBytes = 1.0 * (1ull << 30);
 constexpr int kHubDegree = 256;
 static int hub_default(int64_t n) { return n <= 16384 ? 16 : 64; }
+
+// Counts of the array store need the graph's degrees; dg->mu is held.
+static void degree_stats(const Graph &g, DeviceGraph *dg) {
+    if (!dg->at_least.empty()) return;
+    std::vector<int> c((size_t)g.max_deg + 2, 0);
+    bool ordered = true;
+    for (int32_t v = 0; v < g.n; v++) {
+        c[g.deg(v)]++;
+        ordered = ordered && (v == 0 || g.deg(v) <= g.deg(v - 1));
+    }
+    double squares = 0;
+    for (size_t d = 0; d < c.size(); d++) squares += (double)c[d] * d * d;
+    for (size_t d = c.size() - 1; d-- > 0;) c[d] += c[d + 1];
+    dg->ordered = ordered;
+    dg->neighbour_degree = g.m ? squares / (double)g.m : 0;
+    dg->at_least = std::move(c);
+}
 
 // What a count uses of them: the first n rows. full: every vertex from this
 // degree on has one.
@@ -3256,17 +3270,7 @@ static int build_hubs(const Graph &g, DeviceGraph *dg, size_t n, int least, bool
 // graph is left without any, for the next count to build.
 static int ensure_hubs(const Graph &g, DeviceGraph *dg, int thr, PlanDevice *mine, HubUse *out) {
     std::lock_guard<std::mutex> lk(dg->mu);
-    if (dg->at_least.empty()) {
-        std::vector<int> c((size_t)g.max_deg + 2, 0);
-        bool ordered = true;
-        for (int32_t v = 0; v < g.n; v++) {
-            c[g.deg(v)]++;
-            ordered = ordered && (v == 0 || g.deg(v) <= g.deg(v - 1));
-        }
-        for (size_t d = c.size() - 1; d-- > 0;) c[d] += c[d + 1];
-        dg->ordered = ordered;
-        dg->at_least = std::move(c);
-    }
+    degree_stats(g, dg);
     const std::vector<int> &at_least = dg->at_least;
     auto vertices = [&](int degree) -> size_t { return degree < (int)at_least.size() ? at_least[degree] : 0; };
     const int least = thr ? thr : hub_default(g.n);
@@ -3531,7 +3535,11 @@ static int prepare(gat_plan *p, const gat_kernel_config *cfg_in, Launch *L) {
         if (!rc) rc = need_malloc(&d->ctl, sizeof(unsigned long long) * kCtlWords, nullptr);
         if (!rc) rc = need_malloc(&d->dargs, sizeof(gatk::KArgsSet), nullptr);
         if (rc) return rc;
-        choose_kept(p->cp.dev, d->dg->neighbour_degree, (double)g.m, &d->pd);
+        if (pd.edge_tables || pd.n_tables) {
+            std::lock_guard<std::mutex> lk(d->dg->mu);
+            degree_stats(g, d->dg.get());
+        }
+        choose_kept(pd, d->dg->neighbour_degree, (double)g.m, &d->pd);
         HIPCHECK(hipMemcpy(d->plan, &d->pd, sizeof(GatPlanDev), hipMemcpyHostToDevice));
         HIPCHECK(hipHostMalloc((void **)&d->result, sizeof(unsigned long long) * kCtlResult, hipHostMallocDefault));
         for (auto &e : d->ev) HIPCHECK(hipEventCreate(&e));
